@@ -47,6 +47,7 @@
 namespace hd {
 
 constexpr u32 kStack = 23;  // STACK_SIZE, fraction bits of float (trace.frag:52-54)
+using u8 = unsigned char;
 constexpr u32 kThreads = 256; // workgroup of the beam and traversal kernels
 // The frame kernel's pixel tile (workgroup) is kT x kT, kT in {8, 16}, picked by the tuning.
 constexpr u32 kMaxIter = 1u << 16;
@@ -55,12 +56,13 @@ __device__ inline float fmx(float a, float b) { return a < b ? b : a; } // std::
 __device__ inline float fmn(float a, float b) { return b < a ? b : a; }
 __device__ inline u32 f2u(float f) { return __float_as_uint(f); }
 __device__ inline float u2f(u32 u) { return __uint_as_float(u); }
-// Bit i of the result = (byte i of x != 0), i < 4: bit 7 of each byte is set by the byte's top bit
-// or by a carry out of its low 7 bits (no carry crosses bytes); the multiply by 2^0+2^7+2^14+2^21
-// moves bits 7, 15, 23, 31 to 28..31 without overlapping partial products.
-__device__ inline u32 nonzero_bytes4(u32 x) {
-	const u32 t = (((x & 0x7F7F7F7Fu) + 0x7F7F7F7Fu) | x) & 0x80808080u;
-	return (t * 0x00204081u) >> 28u;
+// DAG_GetLeafFirstChildBits (trace.frag:56-67): bit i of the result = (byte i of w0, w1 is not 0),
+// i < 8. Bit 7 of each byte is set by the byte's top bit or by a carry out of its low 7 bits (no
+// carry crosses bytes); two byte dot products with the weights 2^i add the eight flags, times 128.
+__device__ inline u32 nonzero_bytes8(u32 w0, u32 w1) {
+	const u32 t0 = (((w0 & 0x7F7F7F7Fu) + 0x7F7F7F7Fu) | w0) & 0x80808080u;
+	const u32 t1 = (((w1 & 0x7F7F7F7Fu) + 0x7F7F7F7Fu) | w1) & 0x80808080u;
+	return __builtin_amdgcn_udot4(t1, 0x80402010u, __builtin_amdgcn_udot4(t0, 0x08040201u, 0u, false), false) >> 7u;
 }
 
 struct MarchOut {
@@ -72,12 +74,32 @@ struct MarchOut {
 	float pick[3];
 };
 
-// DAG_RayMarch (trace.frag:69-270). stack: LDS base for this thread, stride = blockDim.
-// kCount: also count the pool words the march reads (reads += ...), for the algorithmic-bytes pass.
+// A node as the march enters it at a scale: the pointer and the 8 child bits. Below the leaf scale
+// the pointer is the leaf's byte, which is its child bits too. Inner nodes and leaves take one load
+// path (word 1 exists for both: a leaf's second mask word, an inner node's first child).
 template <bool kCount>
+__device__ inline uint2 march_node(const u32 *__restrict__ W, u32 ptr, bool at_leaf, u32 &reads) {
+	const u32 w0 = W[(u64)ptr], w1 = W[(u64)ptr + 1u];
+	if (kCount)
+		reads += at_leaf ? 2 : 1;
+	return make_uint2(ptr, at_leaf ? nonzero_bytes8(w0, w1) : w0);
+}
+
+// DAG_RayMarch (trace.frag:69-270). stack: LDS base for this thread, stride = blockDim.
+// kLod: the LOD cut-off is on (a finite proj_factor; without it scale_exp2 * inf is never below t).
+// kCount: also count the pool words the march reads (reads += ...), for the algorithmic-bytes pass.
+//
+// The position is kept as the bits of its three floats: they stay multiples of the current cube size
+// in [1, 2), so adding a cube is adding its bit, the child's index is that bit of each coordinate, and
+// the bits that a step back changes say whether it leaves the parent (a bit above the cube's changed)
+// and up to which scale (the highest one). A step out of the root borrows from the exponent: bit 23.
+// A stack entry holds the node's child bits beside its pointer, so a pop reads no pool word: the
+// chain of a ray that goes from empty cube to empty cube is LDS and registers.
+// 1M incoherent rays on a 4096^3 terrain: @RAYS@.
+template <bool kCount, bool kLod>
 __device__ inline MarchOut march(const u32 *__restrict__ W, u32 root, u32 leaf_level, float proj_factor,
                                  float proj_bias, float ox, float oy, float oz, float dx, float dy, float dz,
-                                 u32 *stack, u32 stride, u32 &reads) {
+                                 u32 *stack, u8 *bits, u32 stride, u32 &reads) {
 	MarchOut out;
 	out.hit = false;
 	out.iter = 0;
@@ -88,13 +110,12 @@ __device__ inline MarchOut march(const u32 *__restrict__ W, u32 root, u32 leaf_l
 		out.vox[i] = 0, out.hit_pos[i] = 0.0f, out.norm[i] = 0.0f, out.pick[i] = 0.0f;
 	if (root == kNull)
 		return out;
-	u32 iter = 0;
 	ox += 1.0f, oy += 1.0f, oz += 1.0f;
 	const float eps = u2f((127u - kStack) << 23u);
 	dx = fabsf(dx) > eps ? dx : (dx >= 0 ? eps : -eps);
 	dy = fabsf(dy) > eps ? dy : (dy >= 0 ? eps : -eps);
 	dz = fabsf(dz) > eps ? dz : (dz >= 0 ? eps : -eps);
-	float tcx = 1.0f / -fabsf(dx), tcy = 1.0f / -fabsf(dy), tcz = 1.0f / -fabsf(dz);
+	const float tcx = 1.0f / -fabsf(dx), tcy = 1.0f / -fabsf(dy), tcz = 1.0f / -fabsf(dz);
 	float tbx = tcx * ox, tby = tcy * oy, tbz = tcz * oz;
 	u32 oct = 0;
 	if (dx > 0.0f)
@@ -103,105 +124,84 @@ __device__ inline MarchOut march(const u32 *__restrict__ W, u32 root, u32 leaf_l
 		oct ^= 2u, tby = 3.0f * tcy - tby;
 	if (dz > 0.0f)
 		oct ^= 4u, tbz = 3.0f * tcz - tbz;
+	// A NaN on the x axis makes t_min NaN: such a ray enters no node and ends without a result. A NaN
+	// on another axis never wins a comparison below, and fminf passes over it as the comparisons do.
+	if (tbx != tbx)
+		return out;
 	float t_min = fmx(fmx(2.0f * tcx - tbx, 2.0f * tcy - tby), 2.0f * tcz - tbz);
 	float t_max = fmn(fmn(tcx - tbx, tcy - tby), tcz - tbz);
 	float h = t_max;
 	t_min = fmx(t_min, 0.0f);
 	t_max = fmn(t_max, 1.0f);
-	u32 parent = root, child_bits = 0;
-	float px = 1.0f, py = 1.0f, pz = 1.0f;
-	u32 idx = 0;
+	constexpr u32 kOne = 127u << 23u; // 1.0f
+	u32 scale = kStack - 1, cube = 1u << (kStack - 1);
+	u32 px = kOne, py = kOne, pz = kOne;
 	if (1.5f * tcx - tbx > t_min)
-		idx ^= 1u, px = 1.5f;
+		px |= cube;
 	if (1.5f * tcy - tby > t_min)
-		idx ^= 2u, py = 1.5f;
+		py |= cube;
 	if (1.5f * tcz - tbz > t_min)
-		idx ^= 4u, pz = 1.5f;
-	u32 scale = kStack - 1;
+		pz |= cube;
 	float scale_exp2 = 0.5f;
 	const u32 leaf_scale = kStack - leaf_level;
-	for (;;) {
-		// A valid ray takes at most a few thousand steps; the cap only guards the device against a
-		// malformed pool (it is never reached by the parity cases).
-		if (++iter > kMaxIter)
+	uint2 node = march_node<kCount>(W, root, scale == leaf_scale, reads);
+	u32 iter = 1;
+	// A valid ray takes at most a few thousand steps; the cap only guards the device against a
+	// malformed pool (it is never reached by the parity cases).
+	for (;; ++iter) {
+		if (iter > kMaxIter)
 			return out;
-		if (child_bits == 0u) {
-			if (scale >= leaf_scale) { // one load path for inner nodes and leaves (lanes diverge less)
-				const bool at_leaf = scale == leaf_scale;
-				// word 1 exists for both (a leaf's second mask word, an inner node's first child)
-				const u32 w0 = W[parent], w1 = W[parent + 1u];
-				child_bits = w0;
-				if (kCount)
-					reads += at_leaf ? 2 : 1;
-				if (at_leaf) // DAG_GetLeafFirstChildBits (trace.frag:56-67): bit i = byte i != 0
-					child_bits = nonzero_bytes4(w0) | (nonzero_bytes4(w1) << 4u);
-			} else
-				child_bits = parent;
-		}
-		float tx = px * tcx - tbx, ty = py * tcy - tby, tz = pz * tcz - tbz;
-		float tc_max = fmn(fmn(tx, ty), tz);
-		u32 child_shift = idx ^ oct, child_mask = 1u << child_shift;
-		if ((child_bits & child_mask) != 0 && t_min <= t_max) {
-			float half = scale_exp2 * 0.5f;
-			float cx = half * tcx + tx, cy = half * tcy + ty, cz = half * tcz + tz;
-			if (scale < leaf_scale || scale_exp2 * proj_factor < tc_max + proj_bias)
+		const float tx = u2f(px) * tcx - tbx, ty = u2f(py) * tcy - tby, tz = u2f(pz) * tcz - tbz;
+		const float tc_max = fminf(fminf(tx, ty), tz);
+		const u32 child = (((px >> scale) & 1u) | (((py >> scale) & 1u) << 1u) | (((pz >> scale) & 1u) << 2u)) ^ oct;
+		if (((node.y >> child) & 1u) != 0u && t_min <= t_max) {
+			if (scale < leaf_scale || (kLod && scale_exp2 * proj_factor < tc_max + proj_bias))
 				break;
-			if (tc_max < h)
-				stack[(scale - leaf_scale) * stride] = parent;
+			if (tc_max < h) {
+				stack[(scale - leaf_scale) * stride] = node.x;
+				bits[(scale - leaf_scale) * stride] = (u8)node.y;
+			}
 			h = tc_max;
 			if (kCount)
 				reads += 1;
 			// one load for both node kinds: an inner node's child pointer, or the leaf word holding the
 			// child's byte
 			const bool inner = scale > leaf_scale;
-			const u32 w = W[inner ? parent + 1u + (u32)__builtin_popcount(child_bits & (child_mask - 1u))
-			                      : parent + (child_shift >> 2u)];
-			parent = inner ? w : (w >> ((child_shift & 3u) << 3u)) & 0xFFu;
-			idx = 0u;
+			const u32 below = (u32)__builtin_popcount(node.y & ((1u << child) - 1u));
+			const u32 w = W[(u64)node.x + (inner ? below + 1u : child >> 2u)];
 			--scale;
-			scale_exp2 = half;
-			if (cx > t_min)
-				idx ^= 1u, px += scale_exp2;
-			if (cy > t_min)
-				idx ^= 2u, py += scale_exp2;
-			if (cz > t_min)
-				idx ^= 4u, pz += scale_exp2;
-			child_bits = 0;
-			continue;
-		}
-		u32 step = 0;
-		if (tx <= tc_max)
-			step ^= 1u, px -= scale_exp2;
-		if (ty <= tc_max)
-			step ^= 2u, py -= scale_exp2;
-		if (tz <= tc_max)
-			step ^= 4u, pz -= scale_exp2;
-		t_min = tc_max;
-		idx ^= step;
-		if ((idx & step) != 0) {
-			u32 diff = 0;
-			if (step & 1u)
-				diff |= f2u(px) ^ f2u(px + scale_exp2);
-			if (step & 2u)
-				diff |= f2u(py) ^ f2u(py + scale_exp2);
-			if (step & 4u)
-				diff |= f2u(pz) ^ f2u(pz + scale_exp2);
-			scale = diff ? 31u - (u32)__builtin_clz(diff) : 0xFFFFFFFFu; // findMSB(0) = -1
-			if (scale >= kStack)
-				break;
-			scale_exp2 = u2f((scale - kStack + 127u) << 23u);
-			parent = stack[(scale - leaf_scale) * stride];
-			u32 shx = f2u(px) >> scale, shy = f2u(py) >> scale, shz = f2u(pz) >> scale;
-			px = u2f(shx << scale);
-			py = u2f(shy << scale);
-			pz = u2f(shz << scale);
-			idx = (shx & 1u) | ((shy & 1u) << 1u) | ((shz & 1u) << 2u);
-			h = 0.0f;
-			child_bits = 0;
+			cube >>= 1u;
+			scale_exp2 *= 0.5f;
+			const float cx = scale_exp2 * tcx + tx, cy = scale_exp2 * tcy + ty, cz = scale_exp2 * tcz + tz;
+			px |= cx > t_min ? cube : 0u;
+			py |= cy > t_min ? cube : 0u;
+			pz |= cz > t_min ? cube : 0u;
+			if (inner)
+				node = march_node<kCount>(W, w, scale == leaf_scale, reads);
+			else
+				node.x = node.y = (w >> ((child & 3u) << 3u)) & 0xFFu;
+		} else {
+			const u32 qx = px - (tx <= tc_max ? cube : 0u), qy = py - (ty <= tc_max ? cube : 0u),
+			          qz = pz - (tz <= tc_max ? cube : 0u);
+			const u32 diff = (px ^ qx) | (py ^ qy) | (pz ^ qz);
+			px = qx, py = qy, pz = qz;
+			t_min = tc_max;
+			if (diff >= 2u * cube) {
+				scale = 31u - (u32)__builtin_clz(diff);
+				if (scale >= kStack)
+					break;
+				cube = 1u << scale;
+				scale_exp2 = u2f((scale - kStack + 127u) << 23u);
+				node.x = stack[(scale - leaf_scale) * stride];
+				node.y = bits[(scale - leaf_scale) * stride];
+				px &= 0u - cube, py &= 0u - cube, pz &= 0u - cube;
+				h = 0.0f;
+			}
 		}
 	}
+	const float fx = u2f(px), fy = u2f(py), fz = u2f(pz);
 	// normal / voxel / hit position (trace.frag:223-258)
-	float ex = tcx * (px + scale_exp2) - tbx, ey = tcy * (py + scale_exp2) - tby, ez = tcz * (pz + scale_exp2) - tbz;
+	float ex = tcx * (fx + scale_exp2) - tbx, ey = tcy * (fy + scale_exp2) - tby, ez = tcz * (fz + scale_exp2) - tbz;
 	float n[3];
 	if (ex > ey && ex > ez)
 		n[0] = -1, n[1] = 0, n[2] = 0;
@@ -227,7 +227,7 @@ __device__ inline MarchOut march(const u32 *__restrict__ W, u32 root, u32 leaf_l
 		return out;
 	}
 	u32 vs = 1u << (scale - voxel_scale);
-	float pp[3] = {px, py, pz}, oo[3] = {ox, oy, oz}, dd[3] = {dx, dy, dz};
+	float pp[3] = {fx, fy, fz}, oo[3] = {ox, oy, oz}, dd[3] = {dx, dy, dz};
 	for (int i = 0; i < 3; ++i) {
 		u32 v = (f2u(pp[i]) & 0x7FFFFFu) >> voxel_scale;
 		if (oct & (1u << i))
@@ -361,7 +361,7 @@ __device__ inline u32 q8(float x) { return (u32)(fmn(fmx(x, 0.0f), 1.0f) * 255.0
 
 template <bool kCount, u32 kT> __global__ void __launch_bounds__(kT *kT) k_trace(TraceArgs A) {
 	constexpr u32 kTT = kT * kT;
-	extern __shared__ u32 stack_lds[]; // node levels x kTT words (trace_lds_bytes)
+	extern __shared__ u32 stack_lds[]; // node levels x kTT words, then as many bytes (trace_lds_bytes)
 	// view of this tile (binary search over the tile prefix); a fixed grid may run past the last tile
 	u32 tile = blockIdx.x, lo = 0, hi = A.n_views;
 	if (tile >= A.tile_start[A.n_views])
@@ -384,6 +384,7 @@ template <bool kCount, u32 kT> __global__ void __launch_bounds__(kT *kT) k_trace
 	if (px >= V.width || py >= V.height)
 		return;
 	u32 *stack = stack_lds + threadIdx.x;
+	u8 *bits = (u8 *)(stack_lds + A.leaf_level * kTT) + threadIdx.x;
 	// Camera_GenRay (trace.frag:366-370), gl_FragCoord at pixel centres, origin top-left
 	const float u = (float(px) + 0.5f) / float(V.width), w = (float(py) + 0.5f) / float(V.height);
 	const float cx = u * 2.0f - 1.0f, cy = w * 2.0f - 1.0f;
@@ -401,19 +402,19 @@ template <bool kCount, u32 kT> __global__ void __launch_bounds__(kT *kT) k_trace
 			for (int i = 0; i < 3; ++i)
 				h.vox[i] = 0, h.hit_pos[i] = 0.0f, h.norm[i] = 0.0f, h.pick[i] = 0.0f;
 		} else
-			h = march<kCount>(A.words, root, A.leaf_level, V.proj_factor, t0, V.pos[0] + t0 * dx, V.pos[1] + t0 * dy,
-			                  V.pos[2] + t0 * dz, dx, dy, dz, stack, kTT, reads);
+			h = march<kCount, true>(A.words, root, A.leaf_level, V.proj_factor, t0, V.pos[0] + t0 * dx, V.pos[1] + t0 * dy,
+			                  V.pos[2] + t0 * dz, dx, dy, dz, stack, bits, kTT, reads);
 	} else
-		h = march<kCount>(A.words, root, A.leaf_level, V.proj_factor, 0.0f, V.pos[0], V.pos[1], V.pos[2], dx, dy,
-		                  dz, stack, kTT, reads);
+		h = march<kCount, true>(A.words, root, A.leaf_level, V.proj_factor, 0.0f, V.pos[0], V.pos[1], V.pos[2], dx, dy,
+		                  dz, stack, bits, kTT, reads);
 	u32 iters = h.iter;
 	float lx = 4.0f, ly = 5.0f, lz = 3.0f;
 	float ll = sqrtf(lx * lx + ly * ly + lz * lz);
 	lx = lx / ll, ly = ly / ll, lz = lz / ll;
 	bool shadow = false;
 	if (h.hit && (V.flags & HD_TRACE_SHADOW)) {
-		MarchOut s = march<kCount>(A.words, root, A.leaf_level, __builtin_inff(), 0.0f, h.hit_pos[0], h.hit_pos[1],
-		                           h.hit_pos[2], lx, ly, lz, stack, kTT, reads);
+		MarchOut s = march<kCount, false>(A.words, root, A.leaf_level, __builtin_inff(), 0.0f, h.hit_pos[0], h.hit_pos[1],
+		                           h.hit_pos[2], lx, ly, lz, stack, bits, kTT, reads);
 		shadow = s.hit;
 		iters += s.iter;
 	}
@@ -470,8 +471,10 @@ __global__ void __launch_bounds__(kThreads) k_beam(TraceArgs A, float *__restric
 	float len = sqrtf(dx * dx + dy * dy + dz * dz);
 	dx = dx / len, dy = dy / len, dz = dz / len;
 	u32 reads = 0;
-	MarchOut h = march<false>(A.words, root, A.leaf_level, V.proj_factor * (1.0f / float(kBeamBlock)), 0.0f, V.pos[0],
-	                          V.pos[1], V.pos[2], dx, dy, dz, stack_lds + threadIdx.x, kThreads, reads);
+	u32 *stack = stack_lds + threadIdx.x;
+	u8 *bits = (u8 *)(stack_lds + A.leaf_level * kThreads) + threadIdx.x;
+	MarchOut h = march<false, true>(A.words, root, A.leaf_level, V.proj_factor * (1.0f / float(kBeamBlock)), 0.0f, V.pos[0],
+	                          V.pos[1], V.pos[2], dx, dy, dz, stack, bits, kThreads, reads);
 	beam[i] = h.hit ? fmaxf(h.t - h.scale, 0.0f) : __builtin_inff();
 }
 
@@ -483,8 +486,10 @@ __global__ void __launch_bounds__(kThreads) k_traversal(const u32 *__restrict__ 
 	if (i >= n)
 		return;
 	u32 reads = 0;
-	MarchOut h = march<false>(W, root, leaf_level, __builtin_inff(), 0.0f, o[3 * i], o[3 * i + 1], o[3 * i + 2],
-	                          d[3 * i], d[3 * i + 1], d[3 * i + 2], stack_lds + threadIdx.x, kThreads, reads);
+	u32 *stack = stack_lds + threadIdx.x;
+	u8 *bits = (u8 *)(stack_lds + leaf_level * kThreads) + threadIdx.x;
+	MarchOut h = march<false, false>(W, root, leaf_level, __builtin_inff(), 0.0f, o[3 * i], o[3 * i + 1], o[3 * i + 2],
+	                          d[3 * i], d[3 * i + 1], d[3 * i + 2], stack, bits, kThreads, reads);
 	out[4 * i] = h.hit ? h.pick[0] : 0.0f;
 	out[4 * i + 1] = h.hit ? h.pick[1] : 0.0f;
 	out[4 * i + 2] = h.hit ? h.pick[2] : 0.0f;
@@ -495,7 +500,7 @@ __global__ void __launch_bounds__(kThreads) k_traversal(const u32 *__restrict__ 
 // The march keeps one stack word per node level and thread in LDS (pushes and pops stay at scales
 // >= the leaf scale, so the slots are scale - leaf_scale in [0, levels)); sizing the stack to the
 // pool's levels rather than the 23 float scales leaves room for more resident waves.
-static u32 trace_lds_bytes(u32 levels, u32 threads) { return levels * threads * 4u; }
+static u32 trace_lds_bytes(u32 levels, u32 threads) { return levels * threads * 5u; }
 static void launch_trace(bool count, u32 n_tiles, hipStream_t s, const TraceArgs &A) {
 	if (g_tuning.trace_tile == 8) {
 		const u32 lds = trace_lds_bytes(A.leaf_level, 64);
