@@ -105,3 +105,22 @@ def test_gc_twice_leaves_the_pool_unchanged():
     assert np.array_equal(dev.full_words(), w1)
     assert_same_pool(dev, ora, "second gc")
 
+
+
+@pytest.mark.parametrize("bits,wbpp,pbpb", [(12, 4, 0), (11, 4, 1), (9, 6, 0), (3, 5, 5), (1, 6, 6), (1, 9, 3)])
+def test_gc_bucket_shapes(bits, wbpp, pbpb):
+    """Buckets smaller than a bitmap word and of one, of a lane's four words and of more nodes than a
+    wavefront has lanes (places across page tails), some of them empty: bit-exact, twice in a row."""
+    capi = _capi()
+    cfg = small_cfg(64, bits, wbpp, pbpb, 3)
+    e = random_edits(16, 64, 11 + bits, True)
+    dev, ora = capi.DevicePool(cfg), O.OraclePool(cfg)
+    for part in (e[:10], e[10:]):
+        dev.edit(part)
+        ora.edit(part)
+        keep_d, keep_o = dev.root, ora.root
+        dev.gc(extra_roots=(keep_d,))
+        ora.gc(extra_roots=(keep_o,))
+        assert ora.overflows() == 0
+        assert_same_pool(dev, ora, f"gc, {1 << bits} buckets of {cfg.words_per_bucket} words")
+        assert np.array_equal(dev.filled(), ora.filled())

@@ -85,18 +85,17 @@ constexpr u64 kWordsPad = 16;
 
 struct Pool;
 // Device buffers of a node-pool GC (hd_gc.hip), sized by the pool's configuration: per level a
-// bitmap of live node starts over the level's words and its popcount prefix (node ranks); new
-// pointers by rank for two adjacent levels; one level's staged words, new-bucket keys, bucket
-// lists, counts and offsets.
+// bitmap of live node starts over the level's words; new pointers at half the old offset for two
+// adjacent levels; one level's remapped nodes, the new buckets' node lists (cap entries each) and
+// counts.
 struct GcPlan {
 	struct Level {
-		u32 *bits = nullptr, *rank = nullptr;
-		u64 words = 0, base = 0, nw = 0, buckets = 0;
+		u32 *bits = nullptr;
+		u64 words = 0, base = 0, buckets = 0;
 	};
 	std::vector<Level> lv;
 	u32 *newp[2] = {nullptr, nullptr};
-	u32 *stage = nullptr, *key = nullptr, *list = nullptr, *cnt = nullptr, *bstart = nullptr, *fill = nullptr,
-	    *bsum = nullptr;
+	u32 *stage = nullptr, *list = nullptr, *cnt = nullptr, cap = 0;
 	int prepare(Pool &p, const char *prefix);
 };
 
@@ -139,7 +138,7 @@ struct Tuning {
 extern Tuning g_tuning; // hd_pool.hip
 
 int make_filled(Pool &p);               // hd_pool.hip
-void launch_make_filled(Pool &p, hipStream_t s); // hd_pool.hip: the chain's lookup into d_filled, queued only
+void launch_refill(Pool &p, hipStream_t s); // hd_pool.hip: the chain found again when d_filled misses a node, queued only
 // A whole GC queued on stream s over device roots (remapped in place); the filled chain is a root
 // when has_filled and is found again into d_filled. No host synchronisation (hd_gc.hip).
 int gc_queue(Pool &p, const GcPlan &G, hipStream_t s, u32 *d_roots, u32 n_roots, bool has_filled);

@@ -21,8 +21,12 @@ void set_error(const char *fmt, ...) {
 }
 
 // NodePool::make_filled_node_pointers (NodePool.hpp:240-262), one thread: the all-solid leaf,
-// then the all-solid inner node of every level, each found or appended in its bucket.
-__global__ void k_make_filled(u32 *words, u32 *bucket_words, DevConfig c, u32 *out, u32 *meta) {
+// then the all-solid inner node of every level, each found or appended in its bucket. missing: only
+// when some node of the chain in out is null (its levels are found one after another: 20 us at 11 levels).
+__global__ void k_make_filled(u32 *words, u32 *bucket_words, DevConfig c, u32 *out, u32 *meta, bool missing) {
+	const bool null = threadIdx.x < c.L && out[threadIdx.x] == kNull;
+	if (missing && !__ballot(null))
+		return;
 	if (threadIdx.x | blockIdx.x)
 		return;
 	u32 node[9];
@@ -52,14 +56,14 @@ __global__ void k_make_filled(u32 *words, u32 *bucket_words, DevConfig c, u32 *o
 	}
 }
 
-void launch_make_filled(Pool &p, hipStream_t s) {
-	k_make_filled<<<1, 64, 0, s>>>(p.words, p.bucket_words, p.dc, p.d_filled, p.meta);
+void launch_refill(Pool &p, hipStream_t s) {
+	k_make_filled<<<1, 64, 0, s>>>(p.words, p.bucket_words, p.dc, p.d_filled, p.meta, true);
 }
 
 int make_filled(Pool &p) {
 	if (!p.filled.empty())
 		return HD_OK;
-	k_make_filled<<<1, 64, 0, p.stream>>>(p.words, p.bucket_words, p.dc, p.d_filled, p.meta);
+	k_make_filled<<<1, 64, 0, p.stream>>>(p.words, p.bucket_words, p.dc, p.d_filled, p.meta, false);
 	HD_TRY(hipGetLastError());
 	p.filled.resize(p.dc.L);
 	HD_TRY(hipMemcpyAsync(p.filled.data(), p.d_filled, p.dc.L * 4, hipMemcpyDeviceToHost, p.stream));

