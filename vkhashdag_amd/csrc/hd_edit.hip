@@ -19,6 +19,7 @@
 
 #include <rocprim/rocprim.hpp>
 
+#include <algorithm>
 #include <chrono>
 #include <cmath>
 #include <cstdlib>
@@ -812,6 +813,10 @@ constexpr u32 kWalkShort = 16; // at most this many: one thread walks the bucket
 struct Pair {
 	u32 a, b;
 };
+// A pair's flags (PairOut::flag) as its slot's bits of the node's pmask word.
+__device__ inline u32 pair_bits(u32 f, u32 k) {
+	return ((f & 1u) << k) | (((f >> 1) & 1u) << (8 + k)) | (((f >> 2) & 1u) << (16 + k)) | ((f >> 3) << (24 + k));
+}
 // Block-wide exclusive scan of kAT pairs: shuffle scans inside each wavefront, one LDS exchange
 // of the wavefront totals (two barriers). sh needs kAT / 64 entries.
 __device__ inline Pair block_excl_scan2(Pair x, Pair *sh, Pair &total) {
@@ -841,7 +846,22 @@ __device__ inline Pair block_excl_scan2(Pair x, Pair *sh, Pair &total) {
 }
 
 // per-pass device counters: pm[kPmHdr + l] entries of level l, pm[kPmHdr + L + l] list words
-enum PassMeta : u32 { kPmOverflow = 0, kPmEvents = 1, kPmLeafTotal = 2, kPmGen = 3, kPmRest = 4, kPmHdr = 5 };
+// (chained passes: kPmCut the first edit that must not share the pass, as ~index, 0 if none; kPmFull
+// whether a bucket or the color pool was full; kPmRoot, kPmCroot, kPmNodes the roots and the color node count
+// that the pass leaves)
+enum PassMeta : u32 {
+	kPmOverflow = 0,
+	kPmEvents = 1,
+	kPmLeafTotal = 2,
+	kPmGen = 3,
+	kPmRest = 4,
+	kPmCut = 5,
+	kPmFull = 6,
+	kPmRoot = 7,
+	kPmCroot = 8,
+	kPmNodes = 9,
+	kPmHdr = 10
+};
 // counters accumulated over the passes of one hd_edit call
 enum AccMeta : u32 { kAccEntries = 0, kAccUpserts = 1, kAccJobs = 2, kAccOverflow = 3, kAccCount = 4 };
 
@@ -857,6 +877,7 @@ struct ALevel {
 	u32 *ores, *ccnt, *cbase, *own; // color results, SetNode passes
 	uint4 *pev; // 8 per entry (levels color leaf .. L - 2, color leaves rebuilt in LDS): a pushed
 	            // child's {voxel offset in its job, colors, wb, 0}, valid where pmask bit 16 + slot is set
+	u32 *prev; // chained passes: the entry of the latest earlier edit at the same node, or kNull
 	u32 cap, list_cap;
 };
 
@@ -1073,8 +1094,10 @@ __device__ inline PairOut expand_pair_e(const EditParams &P, u32 l, const ALevel
 	bool proceed = c.t == kProceed;
 	// bit 0: proceeds, bit 1: the child's pointer changed (a terminal result, or the state a folded
 	// list leaves a proceeding child in: the join compares proceeding results with kids, so it must
-	// know the slot changed even when the result equals that state), bit 2: pushed a color
-	u32 flag = (proceed ? 1u : 0u) | (kid != old ? 2u : 0u) | (c.push ? 4u : 0u);
+	// know the slot changed even when the result equals that state), bit 2: pushed a color, bit 3: the
+	// edit gave the child its color state (else the child keeps the one it had)
+	u32 flag = (proceed ? 1u : 0u) | (kid != old ? 2u : 0u) | (c.push ? 4u : 0u) |
+	           ((c.sf & kSfFinal) && !(sf_in & kSfFinal) ? 8u : 0u);
 	return PairOut{flag, proceed && cnt > 1 ? cnt : 0u, make_uint4(c.octree, c.sf, single, cnt), kid};
 }
 __device__ inline PairOut expand_pair(const EditParams &P, u32 l, const ALevel &A, u64 t, PushEvent *__restrict__ ev,
@@ -1083,8 +1106,9 @@ __device__ inline PairOut expand_pair(const EditParams &P, u32 l, const ALevel &
 }
 
 // Writes the child entry of a proceeding pair (k_emit). m8: proceed flags of the pair's node in
-// bits 0-7, its changed children in bits 8-15 and its pushed children in bits 16-23 (valid
-// on slot 0), idx / lo: the child's entry index and list offset at level l + 1.
+// bits 0-7, its changed children in bits 8-15, its pushed children in bits 16-23 and those the edit
+// gave a color state in bits 24-31 (valid on slot 0), idx / lo: the child's entry index and list offset
+// at level l + 1.
 // bits: expand_pair_e's record of the list edits that touch the child, or null to test them again.
 // by_wave: the list is written by coop_emit (only the bound is checked here).
 __device__ inline Entry emit_pair_e(const EditParams &P, u32 l, const ALevel &A, const ALevel &N,
@@ -1346,7 +1370,7 @@ __device__ inline Pair expand_emit_range(const EditParams &P, u32 l, const ALeve
 			if ((t & 7u) == 0)
 				for (u32 k = 0; k < 8; ++k) {
 					u32 f = sflag[threadIdx.x + k];
-					m8 |= ((f & 1u) << k) | (((f >> 1) & 1u) << (8 + k)) | (((f >> 2) & 1u) << (16 + k));
+					m8 |= pair_bits(f, k);
 				}
 			emit_pair(P, l, A, N, pm, t, m8, o, base.a + off.a, base.b + off.b, by_wave);
 		}
@@ -1465,15 +1489,83 @@ __device__ inline void root_entry(const EditParams &P, const ALevel &A0, u32 *__
 	}
 }
 
+// ---- chained passes (plain mode, several edits in one level-synchronous pass)
+// A chained pass applies edits one after another, as so many passes would, word for word, when no two
+// of them reach the same leaf (nor, with colors, the same color leaf): each edit has its own root
+// entry and its own entries below, so a level's entries are in the order (edit, DFS), the order in which
+// sequential edits append to a bucket. All edits read the nodes as they were before the pass. Where
+// several pass through one node (the levels near the root), each leaves a version of it: an entry's
+// untouched slots hold what the latest earlier version left there (ALevel::prev links the versions), and
+// a node that an edit leaves unchanged is its version before the edit.
+//
+// A colored edit's decisions depend on whether a node is null and whether its color state is the edit's
+// color, which earlier edits of the pass may have changed. So nothing is final before the end: the joins
+// compare each colored edit's start state with the one it decided by (chain_join, chain_decide), appends
+// count only past the saved bucket counters, and color chunks are written last. The first edit that does
+// not hold ends the pass (kPmCut): the counters are restored, the edits before it run again as one pass and
+// the others as a next one. A full bucket (the reference keeps the old pointer there, and what follows
+// depends on it) or color pool sends the edits through single passes.
+//
+// f(edit, entry at level l) for the earlier edits that pass through entry E's node, latest first, until it
+// returns false. From level l - 1 only (E's parent's versions that proceed into E's slot), so the entries
+// of E's own level need not be complete.
+template <typename F>
+__device__ inline void chain_versions(const ALevel *__restrict__ lv, u32 l, const Entry &E, F f) {
+	if (l == 0) { // every edit's root entry has its edit's index
+		for (u32 k = E.loff; k-- > 0;)
+			if (!f(k, k))
+				return;
+		return;
+	}
+	const ALevel &A = lv[l - 1u];
+	const u32 slot = E.sf & 7u;
+	for (u32 q = ldg(A.prev, E.parent); q != kNull; q = ldg(A.prev, q)) {
+		const u32 m = ldg(A.pmask, q);
+		if ((m >> slot) & 1u)
+			if (!f(ldg(&A.ent[q].loff, 0), ldg(A.first_child, q) + (u32)__builtin_popcount(m & ((1u << slot) - 1u))))
+				return;
+	}
+}
+__device__ inline void chain_cut(u32 *__restrict__ pm, u32 edit) { atomicMax(&pm[kPmCut], ~edit); }
+// prev of entry e.
+__device__ inline void chain_link(const ALevel *__restrict__ lv, u32 l, const Entry &E, u32 e) {
+	u32 p = kNull;
+	chain_versions(lv, l, E, [&](u32, u32 q) {
+		p = q < lv[l].cap ? q : kNull; // (past it only when a level outgrew its bound, which is reported)
+		return false;
+	});
+	stg(lv[l].prev, e, p);
+}
+// The root entries of a chained pass, a thread per edit (the whole block calls this).
+__device__ inline void chain_roots(const EditParams &P, const ALevel &A0, const u32 *__restrict__ roots,
+                                   u32 *__restrict__ pm) {
+	const u32 root = roots[0], croot = roots[1];
+	for (u32 k = threadIdx.x; k < P.n_edits; k += kAT) {
+		const DevEditor ed = P.editor(k);
+		const Classified c = classify_single(P, ed, 0, 0, 0, 0, root, croot, 0u);
+		const Entry E{0, 0, 0, root, kNull, c.sf & ~kSfNewJob, c.octree, kNull, k, 1u};
+		if (c.t != kProceed)
+			chain_cut(pm, k);
+		stg(A0.ent, k, E);
+		stg(A0.prev, k, k ? k - 1u : kNull);
+	}
+	if (threadIdx.x == 0) {
+		pm[kPmHdr] = P.n_edits;
+		pm[kPmHdr + P.c.L] = 0u;
+	}
+}
+
 // Single workgroup: clears the pass counters, classifies the root and expands levels [0, l_end)
 // (every one small enough for one block), with the current level's entries and count in LDS.
 constexpr u32 kTopEnt = kTopPairs / 8;
 constexpr u32 kTopEdits = 1024; // a pass with at most this many edits reads them from LDS in a_top
-// kLists: the pass has more than one edit (nodes may carry edit lists).
-template <bool kLists>
+// kMode: one edit; several (nodes may carry edit lists); several chained (an entry has one edit each).
+enum : u32 { kTopOne = 0, kTopLists = 1, kTopChain = 2 };
+template <u32 kMode>
 __global__ void __launch_bounds__(kAT) a_top(EditParams P0, const ALevel *__restrict__ lv, u32 *__restrict__ roots,
                                              u32 *__restrict__ pm, u32 pm_words, u32 l_end, PushEvent *ev, u32 ev_cap,
                                              u32 *__restrict__ gen_ctr) {
+	constexpr bool kLists = kMode == kTopLists, kChain = kMode == kTopChain;
 	__shared__ Pair sh[kAT];
 	__shared__ u32 sflag[kAT];
 	__shared__ Entry sent[2][kTopEnt];
@@ -1496,13 +1588,24 @@ __global__ void __launch_bounds__(kAT) a_top(EditParams P0, const ALevel *__rest
 		sfilled[threadIdx.x] = P.filled[threadIdx.x];
 	P.filled = sfilled;
 	__syncthreads();
+	if (kChain) {
+		chain_roots(P, lv[0], roots, pm);
+		__syncthreads();
+		for (u32 k = threadIdx.x; k < P.n_edits; k += kAT)
+			sent[0][k] = lv[0].ent[k];
+		if (threadIdx.x == 0)
+			scount = P.n_edits;
+	}
 	if (threadIdx.x < 64) {
-		root_entry(P, lv[0], roots, pm, threadIdx.x);
+		if (!kChain)
+			root_entry(P, lv[0], roots, pm, threadIdx.x);
 		if (threadIdx.x == 0) {
 			pm[kPmGen] = atomicAdd(gen_ctr, P.c.L) + 1u; // this pass's dedup generations: pm[kPmGen] + level
-			scount = pm[kPmHdr];
-			if (scount)
-				sent[0][0] = lv[0].ent[0];
+			if (!kChain) {
+				scount = pm[kPmHdr];
+				if (scount)
+					sent[0][0] = lv[0].ent[0];
+			}
 		}
 	}
 	__syncthreads();
@@ -1512,7 +1615,7 @@ __global__ void __launch_bounds__(kAT) a_top(EditParams P0, const ALevel *__rest
 	if (threadIdx.x < 64) {
 		const u32 lane = threadIdx.x;
 		u32 l = 0, n = scount;
-		for (; l < l_end && n <= 8u; ++l) {
+		for (; !kChain && l < l_end && n <= 8u; ++l) {
 			const ALevel A = lv[l], N = lv[l + 1];
 			const Entry *cur = sent[l & 1];
 			Entry *nxt = sent[(l + 1) & 1];
@@ -1536,6 +1639,7 @@ __global__ void __launch_bounds__(kAT) a_top(EditParams P0, const ALevel *__rest
 				                  by_wave ? &hits2 : nullptr);
 			}
 			const u64 bp = __ballot(o.flag & 1u), bt = __ballot((o.flag >> 1) & 1u), bu = __ballot((o.flag >> 2) & 1u);
+			// (the color-state bits are read in chained passes only)
 			const u64 below = (1ull << lane) - 1ull;
 			u32 lc = o.lcnt; // inclusive wave scan of the list lengths (a single-edit pass has none)
 			if (kLists)
@@ -1612,6 +1716,8 @@ __global__ void __launch_bounds__(kAT) a_top(EditParams P0, const ALevel *__rest
 				bits = kLists && !by_wave && E.llen <= kTopEdits ? sbits[threadIdx.x] : nullptr;
 				o = expand_pair_e(P, l, A, t, E, ev, pm, ev_cap, bits, by_wave ? &hits : nullptr,
 				                  by_wave ? &hits2 : nullptr);
+				if (kChain && (t & 7u) == 0 && l)
+					chain_link(lv, l, E, (u32)(t >> 3));
 			}
 			sflag[threadIdx.x] = o.flag;
 			Pair tile;
@@ -1621,7 +1727,7 @@ __global__ void __launch_bounds__(kAT) a_top(EditParams P0, const ALevel *__rest
 				if ((t & 7u) == 0)
 					for (u32 k = 0; k < 8; ++k) {
 						u32 f = sflag[threadIdx.x + k];
-						m8 |= ((f & 1u) << k) | (((f >> 1) & 1u) << (8 + k)) | (((f >> 2) & 1u) << (16 + k));
+						m8 |= pair_bits(f, k);
 					}
 				const u32 idx = base.a + off.a;
 				Entry ne = emit_pair_e(P, l, A, N, pm, t, E, o.kid, m8, o, idx, base.b + off.b, bits, by_wave);
@@ -1657,6 +1763,7 @@ __global__ void __launch_bounds__(kAT) a_top(EditParams P0, const ALevel *__rest
 }
 
 // Large levels: a_count (classify, block totals) then a_emit (block prefix, stable emit).
+template <bool kChain>
 __global__ void __launch_bounds__(kAT) a_count(EditParams P, u32 l, const ALevel *__restrict__ lv, u32 *__restrict__ pm,
                                                u32 *__restrict__ flag, u32 *__restrict__ lcnt,
                                                uint4 *__restrict__ cstate, PushEvent *ev, u32 ev_cap,
@@ -1683,6 +1790,8 @@ __global__ void __launch_bounds__(kAT) a_count(EditParams P, u32 l, const ALevel
 			continue;
 		PairOut o = expand_pair_e(P, l, A, t, A.ent[(u32)(t >> 3)], ev, pm, ev_cap, nullptr, by_wave ? &hits : nullptr,
 		                          by_wave ? &hits2 : nullptr);
+		if (kChain && (t & 7u) == 0)
+			chain_link(lv, l, A.ent[(u32)(t >> 3)], (u32)(t >> 3));
 		flag[t] = o.flag;
 		lcnt[t] = o.lcnt;
 		cstate[t] = o.cs;
@@ -2416,6 +2525,220 @@ __global__ void __launch_bounds__(kAT) a_build(EditParams P, u32 l, const ALevel
 		} while (__syncthreads_or(todo));
 	}
 }
+// child_result_fresh of a chained pass: x the result, y bit 0 a fresh append, bit 1 unchanged (the
+// node's version before the edit, whatever x says: also when its bucket was full).
+__device__ inline uint2 chain_child(const ALevel &C, const GroupTable &G, u32 c) {
+	const u32 cc = min(c, C.cap - 1u);
+	const u32 pend = ldg(C.pend, cc), st = ldg(C.status, cc), r = ldg(C.res, cc), s = ldg(C.slot, cc);
+	const u32 pt = ldg(&C.ent[cc].ptr, 0);
+	const u32 si = s & G.mask;
+	const u32 gf = ldg(G.gfail, si), gr = ldg(G.gres, si);
+	const bool same = pend ? r == kNull && gf : st == pt, fresh = pend && r == kNull && !gf;
+	return make_uint2(!pend ? st : (r != kNull ? r : gr), (fresh ? 1u : 0u) | (same || c >= C.cap ? 2u : 0u));
+}
+// The join of a chained pass (build_node with versions): a slot that the edit changed takes its result,
+// the others what the latest earlier version left there, or the node as it was before the pass. link(q):
+// {prev, pmask, first_child} of entry q.
+template <typename Link>
+__device__ inline Built chain_join(const EditParams &P, u32 l, const ALevel &A, const ALevel &C, const GroupTable &G,
+                                   u32 e, u32 *__restrict__ pm, Link link) {
+	const JoinIn q = load_join(A, e);
+	const u32 pmk = q.pmw & 0xFFu, cnt = (u32)__builtin_popcount(pmk);
+	const u32 kv[8] = {q.k0.x, q.k0.y, q.k0.z, q.k0.w, q.k1.x, q.k1.y, q.k1.z, q.k1.w};
+	uint2 cr[8];
+#pragma unroll
+	for (u32 j = 0; j < 8; ++j)
+		cr[j] = cnt ? chain_child(C, G, q.fc + min(j, cnt - 1u)) : make_uint2(kNull, 2u);
+	u32 nk[8], st[8], own = 0; // the slots after and before the edit, those that it changed
+	bool fresh = false;
+#pragma unroll
+	for (u32 i = 0; i < 8; ++i) {
+		const u32 rank = (u32)__builtin_popcount(pmk & ((1u << i) - 1u));
+		uint2 c = cr[0];
+#pragma unroll
+		for (u32 j = 1; j <= i; ++j)
+			c = rank == j ? cr[j] : c;
+		const bool pr = (pmk >> i) & 1u, set = pr ? !(c.y & 2u) : ((q.pmw >> (8u + i)) & 1u) != 0u;
+		nk[i] = pr ? c.x : kv[i];
+		st[i] = kv[i];
+		own |= (set ? 1u : 0u) << i;
+		fresh |= set && (c.y & 1u) && pr;
+	}
+	Built o{};
+	o.k = 0;
+	const bool colored = (ldg(&A.ent[e].sf, 0) & kSfActive) != 0u;
+	// the earlier versions, latest first (a colored edit looks at every slot, to compare; an uncolored one
+	// at those that it inherits)
+	u32 need = colored ? 0xFFu : own ? 0xFFu & ~own : 0u;
+	for (u32 v = need ? link(e).x : kNull; v != kNull && need;) {
+		const uint4 t = link(v);
+		const u32 set = ((t.y & 0xFFu) | (t.y >> 8)) & need & 0xFFu;
+		for (u32 m = set; m; m &= m - 1u) {
+			const u32 i = (u32)__builtin_ctz(m);
+			uint2 c;
+			if ((t.y >> i) & 1u)
+				c = chain_child(C, G, t.z + (u32)__builtin_popcount(t.y & ((1u << i) - 1u)));
+			else
+				c = make_uint2(ldg(A.kids, 8ull * v + i), 0u);
+			if (c.y & 2u)
+				continue;
+			fresh |= !((own >> i) & 1u) && (c.y & 1u);
+			need &= ~(1u << i);
+#pragma unroll
+			for (u32 k = 0; k < 8; ++k)
+				st[k] = k == i ? c.x : st[k];
+		}
+		v = t.x;
+	}
+	if (colored) { // (a slot that the edit covers whole does not depend on what was there)
+		bool bad = false;
+#pragma unroll
+		for (u32 i = 0; i < 8; ++i)
+			bad |= !((q.pmw >> (8u + i)) & 1u) && (st[i] == kNull) != (kv[i] == kNull);
+		if (bad)
+			chain_cut(pm, ldg(&A.ent[e].loff, 0));
+	}
+	if (!own) { // unchanged
+		stg(A.pend, e, 0u);
+		stg(A.status, e, q.ptr);
+		return o;
+	}
+#pragma unroll
+	for (u32 i = 0; i < 8; ++i)
+		nk[i] = (own >> i) & 1u ? nk[i] : st[i];
+	u32 nm = 0;
+#pragma unroll
+	for (u32 i = 0; i < 8; ++i)
+		nm |= (nk[i] != kNull ? 1u : 0u) << i;
+	if (!nm) {
+		stg(A.pend, e, 0u);
+		stg(A.status, e, kNull);
+		return o;
+	}
+	pack_inner(nm, nk, o.c);
+	o.k = (u32)__builtin_popcount(nm) + 1u;
+	o.h = murmur_regs(o.c, o.k);
+	o.b = P.c.level_base[l] + (o.h & ((1u << P.c.bucket_bits[l]) - 1u));
+	o.need = fresh;
+	return o;
+}
+// a_build of a chained pass. The links of a level near the root (at most kLinkEntries entries, long
+// version chains) are staged in LDS; below, a node has a version or two.
+constexpr u32 kLinkEntries = 512;
+template <u32 kCap>
+__global__ void __launch_bounds__(kAT) a_build_chain(EditParams P, u32 l, const ALevel *__restrict__ lv,
+                                                     u32 *__restrict__ pm, GroupTable G) {
+	__shared__ __align__(16) u32 stage[kCap];
+	__shared__ uint4 links[kLinkEntries];
+	__shared__ u32 top;
+	const ALevel A = lv[l], C = lv[l + 1];
+	const u32 n = pm[kPmHdr + l];
+	auto load = [&](u32 q) { return make_uint4(ldg(A.prev, q), ldg(A.pmask, q), ldg(A.first_child, q), 0u); };
+	if (n <= kLinkEntries)
+		for (u32 i = threadIdx.x; i < n; i += kAT)
+			links[i] = load(i);
+	__syncthreads();
+	for (u32 e0 = blockIdx.x * blockDim.x; e0 < n; e0 += gridDim.x * blockDim.x) { // uniform trip count
+		const u32 e = e0 + threadIdx.x;
+		Built o{};
+		o.k = 0;
+		if (e < n)
+			o = chain_join(P, l, A, C, G, e, pm, [&](u32 q) { return n <= kLinkEntries ? links[q] : load(q); });
+		bool todo = o.k != 0;
+		do { // an entry whose bucket found the stage full looks again after the reset
+			if (threadIdx.x == 0)
+				top = 0;
+			__syncthreads();
+			if (todo)
+				todo = !find_entry(P, l, A, e, o, stage, &top, kCap);
+		} while (__syncthreads_or(todo));
+	}
+}
+// Before a chained pass's first append: the bucket counters, the pool's full-bucket flag (cleared, so that
+// the pass sees its own) and the append count are saved.
+__global__ void a_chain_begin(const u32 *__restrict__ bucket_words, u32 *__restrict__ saved, u64 n,
+                              u32 *__restrict__ meta, const u32 *__restrict__ acc) {
+	const u64 t0 = (u64)blockIdx.x * blockDim.x + threadIdx.x;
+	for (u64 i = t0; i < n; i += (u64)gridDim.x * blockDim.x)
+		saved[i] = bucket_words[i];
+	if (t0 == 0) {
+		saved[n] = atomicAnd(&meta[kMetaOverflow], ~1u) & 1u;
+		saved[n + 1u] = acc[kAccUpserts];
+	}
+}
+// A chained pass that did not hold: its appends are past the saved counters.
+__global__ void a_chain_restore(u32 *__restrict__ bucket_words, const u32 *__restrict__ saved, u64 n) {
+	for (u64 i = (u64)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (u64)gridDim.x * blockDim.x)
+		bucket_words[i] = saved[i];
+}
+constexpr u32 kChainEdits = 128; // edits of a chained pass
+// After the node levels (one workgroup): the pass's root is the last version that changed it; a colored
+// edit must have found the root null or not as before the pass; whether a bucket was full.
+__global__ void __launch_bounds__(kChainEdits) a_chain_end(EditParams P, const ALevel *__restrict__ lv,
+                                                           u32 *__restrict__ pm, GroupTable G,
+                                                           const u32 *__restrict__ roots,
+                                                           const u32 *__restrict__ saved, u64 n_saved) {
+	__shared__ uint2 ver[kChainEdits];
+	const u32 k = threadIdx.x, n = pm[kPmHdr], root = roots[0];
+	if (k < n)
+		ver[k] = chain_child(lv[0], G, k);
+	__syncthreads();
+	if (k < n) {
+		u32 at = root; // the root that edit k finds
+		for (u32 j = k; j-- > 0;)
+			if (!(ver[j].y & 2u)) {
+				at = ver[j].x;
+				break;
+			}
+		if ((at == kNull) != (root == kNull) && (ldg(&lv[0].ent[k].sf, 0) & kSfActive))
+			chain_cut(pm, k);
+		if (k == n - 1u) {
+			pm[kPmRoot] = ver[k].y & 2u ? at : ver[k].x;
+			pm[kPmCroot] = roots[1];
+			pm[kPmNodes] = P.meta[kMetaColorNodes];
+			if (P.meta[kMetaOverflow] & 1u) {
+				atomicAnd(&P.meta[kMetaOverflow], ~1u);
+				pm[kPmFull] = 1u;
+				chain_cut(pm, 0u);
+			}
+			atomicOr(&P.meta[kMetaOverflow], saved[n_saved]);
+		}
+	}
+}
+// The last kernel of a chained pass (one workgroup): the roots, color counters and statistics, if it held.
+__global__ void __launch_bounds__(kAT) a_chain_commit(EditParams P, const ALevel *__restrict__ lv,
+                                                      const u32 *__restrict__ pm, u32 *__restrict__ roots,
+                                                      u32 *__restrict__ acc, const u32 *__restrict__ saved, u64 n_saved) {
+	if (pm[kPmCut]) {
+		if (threadIdx.x == 0) {
+			acc[kAccOverflow] |= pm[kPmOverflow];
+			acc[kAccUpserts] = saved[n_saved + 1u];
+		}
+		return;
+	}
+	u32 jobs = 0; // the color leaves that colored edits enter
+	if (P.stateful)
+		for (u32 e = threadIdx.x; e < pm[kPmHdr + P.c.color_leaf]; e += kAT)
+			jobs += ldg(&lv[P.c.color_leaf].ent[e].sf, 0) & kSfActive ? 1u : 0u;
+#pragma unroll
+	for (u32 d = 32; d > 0; d >>= 1)
+		jobs += (u32)__shfl_xor((int)jobs, (int)d);
+	if ((threadIdx.x & 63u) == 0 && jobs)
+		atomicAdd(&acc[kAccJobs], jobs);
+	if (threadIdx.x)
+		return;
+	roots[0] = pm[kPmRoot];
+	roots[1] = pm[kPmCroot];
+	if (P.stateful) {
+		P.meta[kMetaColorNodes] = pm[kPmNodes];
+		P.meta[kMetaColorLeaves] += pm[kPmLeafTotal];
+	}
+	u32 tot = 0;
+	for (u32 l = 0; l < P.c.L; ++l)
+		tot += pm[kPmHdr + l];
+	acc[kAccEntries] += tot;
+	acc[kAccOverflow] |= pm[kPmOverflow];
+}
 __global__ void __launch_bounds__(kAT) a_dedup(EditParams P, u32 l, const ALevel *__restrict__ lv,
                                                const u32 *__restrict__ pm, GroupTable G, u32 *__restrict__ bcnt,
                                                u32 *__restrict__ head, u32 *__restrict__ blist) {
@@ -3023,7 +3346,7 @@ __global__ void __launch_bounds__(kEncThreads, 3) a_job_rest(EditParams P, const
 	const u32 leafL = P.c.color_leaf;
 	u32 *ores = lv[leafL].ores;
 	const u32 leaf_base = P.meta[kMetaColorLeaves];
-	const u32 nrest = pm[kPmRest];
+	const u32 nrest = pm[kPmCut] ? 0u : pm[kPmRest]; // (a chained pass that did not hold writes nothing)
 	for (u32 i = blockIdx.x; i < nrest; i += gridDim.x) {
 		const u32 e = rest[i];
 		__syncthreads(); // the previous job's readers are done with S
@@ -3153,7 +3476,7 @@ __global__ void __launch_bounds__(kEncThreads) a_encode_write(EditParams P, cons
 	const u32 leafL = P.c.color_leaf;
 	const Entry *ent = lv[leafL].ent;
 	u32 *ores = lv[leafL].ores;
-	const u32 n = pm[kPmHdr + leafL];
+	const u32 n = pm[kPmCut] ? 0u : pm[kPmHdr + leafL]; // (a chained pass that did not hold writes nothing)
 	const u32 leaf_base = P.meta[kMetaColorLeaves];
 	__shared__ u64 s_wm;
 	for (u32 c0 = blockIdx.x; c0 < n; c0 += gridDim.x * kJobChunk)
@@ -4134,6 +4457,206 @@ __global__ void __launch_bounds__(kSetNodeThreads) a_setnode(EditParams P, const
 	}
 }
 
+// ---- SetNode of a chained pass, level by level over all edits, eight lanes per entry (a slot each)
+// An entry's slots after its edit are what the edit gave them (a child's decision, or a color state), else
+// what the latest earlier colored version gave them, else the children of the node's state before the
+// pass. Decisions: kColorKeep (the state before the edit), kColorNewNode, or a state. A new node's index
+// is not known before every edit's decisions are counted, so a slot refers to it by its entry (node tag, the
+// node capacity + entry: no real node has that index).
+constexpr u32 kColorKeep = 0x3FFFFFFEu; // (color-node capacities are below 2^30 - 1, chained passes' far below)
+struct ChainColor {
+	const ALevel *lv;
+	const u32 *info, *appo; // the color leaf jobs' sizes and append offsets
+	u32 leaf_base, node_cap;
+};
+// The state a color leaf job leaves its node in (a_encode_write's and a_job_rest's result).
+__device__ inline u32 chain_job_state(const EditParams &P, const ChainColor &K, u32 c) {
+	const ALevel &J = K.lv[P.c.color_leaf];
+	const u32 own = ldg(&J.ent[c].octree, 0);
+	if (!(ldg(&J.ent[c].sf, 0) & kSfWriter) || (ldg(K.info, 4ull * c + 2u) & 1u))
+		return own;
+	return cmake(kTagLeaf, K.leaf_base + ldg(K.appo, c));
+}
+// What entry q's edit made of slot i; false if it left the slot as it was.
+__device__ inline bool chain_slot(const EditParams &P, const ChainColor &K, u32 l, u32 q, u32 i, u32 sf, u32 &val) {
+	const ALevel &A = K.lv[l];
+	if (sf & kSfFinal) { // the whole node has the edit's color
+		val = ldg(&A.ent[q].octree, 0);
+		return true;
+	}
+	const u32 m = ldg(A.pmask, q);
+	if (!((m >> i) & 1u)) {
+		val = ldg(A.okids, 8ull * q + i);
+		return ((m >> (24u + i)) & 1u) != 0u;
+	}
+	const u32 c = ldg(A.first_child, q) + (u32)__builtin_popcount(m & 0xFFu & ((1u << i) - 1u));
+	if (l + 1u == P.c.color_leaf) {
+		val = chain_job_state(P, K, c);
+		return true;
+	}
+	const u32 r = ldg(K.lv[l + 1u].ores, c);
+	val = r == kColorNewNode ? cmake(kTagNode, K.node_cap + c) : r;
+	return r != kColorKeep;
+}
+// Slot i of entry e before its edit.
+__device__ inline u32 chain_before(const EditParams &P, const ChainColor &K, u32 l, u32 e, u32 i, u32 own) {
+	const ALevel &A = K.lv[l];
+	for (u32 q = ldg(A.prev, e); q != kNull; q = ldg(A.prev, q)) {
+		const u32 sf = ldg(&A.ent[q].sf, 0);
+		u32 val;
+		if ((sf & kSfActive) && chain_slot(P, K, l, q, i, sf, val))
+			return val;
+	}
+	return color_child(P.cnodes, own, i);
+}
+__device__ inline u32 byte_of(u64 ballot, u32 lane) { return (u32)(ballot >> (lane & 56u)) & 0xFFu; }
+// The color state that edit k's decisions compare with (HD_COLOR_NULL: none is equal to its color).
+__device__ inline u32 chain_color(const EditParams &P, u32 k) {
+	const hd_color c = P.edits[k].color;
+	return c.colors >> 24 || c.weight ? kColorNull : cmake(kTagColor, c.colors);
+}
+// Decision of entry e (lane i: slot i) and its appended nodes; cuts the pass at an edit that took another
+// color state for its own color, or the other way round, than it finds.
+__device__ inline void chain_decide(const EditParams &P, const ChainColor &K, u32 l, u32 e, u32 i, u32 *__restrict__ pm) {
+	const ALevel &A = K.lv[l];
+	const u32 lane = threadIdx.x & 63u, sf = ldg(&A.ent[e].sf, 0), own = ldg(&A.ent[e].octree, 0);
+	u32 r = kColorKeep, c = 0;
+	if ((sf & kSfActive) && (sf & kSfFinal))
+		r = own;
+	else if (sf & kSfActive) {
+		const u32 m = ldg(A.pmask, e), kid = ldg(A.kids, 8ull * e + i), k = ldg(&A.ent[e].loff, 0);
+		const u32 was = chain_before(P, K, l, e, i, own);
+		u32 ch = was;
+		if (!chain_slot(P, K, l, e, i, sf, ch))
+			ch = was;
+		if (((m >> i) & 1u) && l + 1u < P.c.color_leaf)
+			c = ldg(K.lv[l + 1u].ccnt, ldg(A.first_child, e) + (u32)__builtin_popcount(m & 0xFFu & ((1u << i) - 1u)));
+		const u32 mine = chain_color(P, k);
+		if (kid != kNull && !((m >> (8u + i)) & 1u) && (was == mine) != (color_child(P.cnodes, own, i) == mine) &&
+		    mine != kColorNull)
+			chain_cut(pm, k);
+#pragma unroll
+		for (u32 d = 1; d < 8; d <<= 1)
+			c += (u32)__shfl_xor((int)c, (int)d);
+		const u32 ch0 = (u32)__shfl((int)ch, (int)(lane & 56u));
+		const bool null = byte_of(__ballot(ctag(ch) == kTagNull), lane) == 0xFFu;
+		const bool one = byte_of(__ballot(ch == ch0), lane) == 0xFFu && ctag(ch0) == kTagColor;
+		const bool kept = byte_of(__ballot(ch == was), lane) == 0xFFu;
+		r = null ? kColorNull : one ? ch0 : kept ? kColorKeep : kColorNewNode;
+		c += r == kColorNewNode ? 1u : 0u;
+	}
+	if (i == 0) {
+		A.ores[e] = r;
+		A.ccnt[e] = c;
+	}
+}
+// The first post-order indices of entry e's proceeding children.
+__device__ inline void chain_base(const EditParams &P, const ChainColor &K, u32 l, u32 e, u32 i) {
+	const ALevel &A = K.lv[l], &C = K.lv[l + 1u];
+	const u32 m = ldg(A.pmask, e), base = ldg(A.cbase, e);
+	const bool pr = ((m >> i) & 1u) && (ldg(&A.ent[e].sf, 0) & kSfActive);
+	const u32 ci = ldg(A.first_child, e) + (u32)__builtin_popcount(m & 0xFFu & ((1u << i) - 1u));
+	const u32 c = pr ? ldg(C.ccnt, ci) : 0u;
+	u32 x = c;
+#pragma unroll
+	for (u32 d = 1; d < 8; d <<= 1) {
+		const u32 y = (u32)__shfl_up((int)x, (int)d);
+		if (i >= d)
+			x += y;
+	}
+	if (pr)
+		C.cbase[ci] = base + x - c;
+}
+__global__ void __launch_bounds__(kAT) a_chain_up(EditParams P, ChainColor K, u32 l, u32 *__restrict__ pm) {
+	K.leaf_base = P.meta[kMetaColorLeaves];
+	const u32 n = pm[kPmHdr + l], t0 = blockIdx.x * blockDim.x + threadIdx.x;
+	for (u32 e = t0 >> 3; e < n; e += gridDim.x * blockDim.x >> 3)
+		chain_decide(P, K, l, e, t0 & 7u, pm);
+}
+__global__ void __launch_bounds__(kAT) a_chain_down(EditParams P, ChainColor K, u32 l, const u32 *__restrict__ pm) {
+	const u32 n = pm[kPmHdr + l], t0 = blockIdx.x * blockDim.x + threadIdx.x;
+	for (u32 e = t0 >> 3; e < n; e += gridDim.x * blockDim.x >> 3)
+		chain_base(P, K, l, e, t0 & 7u);
+}
+// One workgroup: the decisions of the levels [0, lb), the root's versions, each edit's first node index
+// (an edit's nodes follow those of the edits before it), and the indices of the levels up to lb.
+__global__ void __launch_bounds__(kSetNodeThreads) a_chain_top(EditParams P, ChainColor K, u32 lb, u32 *__restrict__ pm,
+                                                               const u32 *__restrict__ roots, u64 leaf_cap) {
+	__shared__ u32 dec[kChainEdits], cnt[kChainEdits], act[kChainEdits], out[2];
+	K.leaf_base = P.meta[kMetaColorLeaves];
+	const u32 n = pm[kPmHdr], i = threadIdx.x & 7u;
+	for (u32 l = lb; l-- > 0;) {
+		for (u32 e = threadIdx.x >> 3; e < pm[kPmHdr + l]; e += kSetNodeThreads >> 3)
+			chain_decide(P, K, l, e, i, pm);
+		__syncthreads();
+	}
+	const ALevel &A = K.lv[0];
+	for (u32 k = threadIdx.x; k < n; k += kSetNodeThreads) {
+		dec[k] = A.ores[k];
+		cnt[k] = A.ccnt[k];
+		act[k] = ldg(&A.ent[k].sf, 0) & kSfActive;
+	}
+	__syncthreads();
+	for (u32 k = threadIdx.x; k < n; k += kSetNodeThreads) {
+		const u32 base0 = pm[kPmNodes], croot = roots[1];
+		u32 base = base0, at = croot; // the color root that edit k finds
+		for (u32 j = 0; j < k; ++j)
+			if (act[j]) {
+				base += cnt[j];
+				if (dec[j] != kColorKeep)
+					at = dec[j] == kColorNewNode ? cmake(kTagNode, base - 1u) : dec[j];
+			}
+		A.cbase[k] = base;
+		const u32 mine = chain_color(P, k);
+		if (act[k] && roots[0] != kNull && mine != kColorNull && (at == mine) != (croot == mine))
+			chain_cut(pm, k);
+		if (k == n - 1u) {
+			if (act[k]) {
+				base += cnt[k];
+				if (dec[k] != kColorKeep)
+					at = dec[k] == kColorNewNode ? cmake(kTagNode, base - 1u) : dec[k];
+			}
+			out[0] = base;
+			out[1] = at;
+			if (base > K.node_cap || (u64)K.leaf_base + pm[kPmLeafTotal] > leaf_cap) {
+				pm[kPmFull] = 1u;
+				chain_cut(pm, 0u);
+			}
+		}
+	}
+	__syncthreads();
+	if (threadIdx.x == 0 && n) {
+		pm[kPmNodes] = out[0];
+		pm[kPmCroot] = out[1];
+	}
+	for (u32 l = 0; l < lb && l + 1u < P.c.color_leaf; ++l) {
+		for (u32 e = threadIdx.x >> 3; e < pm[kPmHdr + l]; e += kSetNodeThreads >> 3)
+			chain_base(P, K, l, e, i);
+		__syncthreads();
+	}
+}
+// Every new node, at its index (blockIdx.y: the level).
+__global__ void __launch_bounds__(kAT) a_chain_nodes(EditParams P, ChainColor K, const u32 *__restrict__ pm) {
+	if (pm[kPmCut])
+		return;
+	K.leaf_base = P.meta[kMetaColorLeaves];
+	const u32 l = blockIdx.y, n = pm[kPmHdr + l], t0 = blockIdx.x * blockDim.x + threadIdx.x, i = t0 & 7u;
+	const ALevel &A = K.lv[l];
+	for (u32 e = t0 >> 3; e < n; e += gridDim.x * blockDim.x >> 3) {
+		const u32 sf = ldg(&A.ent[e].sf, 0);
+		if (!(sf & kSfActive) || ldg(A.ores, e) != kColorNewNode)
+			continue;
+		u32 ch = 0;
+		if (!chain_slot(P, K, l, e, i, sf, ch))
+			ch = chain_before(P, K, l, e, i, ldg(&A.ent[e].octree, 0));
+		if (ctag(ch) == kTagNode && ch >= K.node_cap) { // a node of this pass: its index
+			const u32 c = ch - K.node_cap;
+			ch = cmake(kTagNode, ldg(K.lv[l + 1u].cbase, c) + ldg(K.lv[l + 1u].ccnt, c) - 1u);
+		}
+		P.cnodes[8ull * (ldg(A.cbase, e) + ldg(A.ccnt, e) - 1u) + i] = ch;
+	}
+}
+
 __global__ void a_set_roots(u32 *roots, u32 root, u32 croot, u32 *acc) {
 	if (threadIdx.x | blockIdx.x)
 		return;
@@ -4579,6 +5102,7 @@ struct PassPlan {
 	u32 first = 0, count = 0;
 	bool stateful = false, async = false;
 	bool folded = false; // the edits may overlap (folded lists)
+	bool chained = false; // the edits one after another in one pass (versions of shared nodes)
 	std::vector<u64> cap, list_cap;
 	u64 ev_cap = 0, bytes = 0;
 };
@@ -4645,8 +5169,8 @@ static void plan_pass(const Pool &p, const hd_edit_desc *edits, PassPlan &pp) {
 			S[l] += edit_level_bound(edits[pp.first + k], vl, l);
 	pp.cap.assign(L, 0);
 	pp.list_cap.assign(L, 0);
-	pp.cap[0] = 1;
-	pp.list_cap[0] = pp.count > 1 ? pp.count : 0;
+	pp.cap[0] = pp.chained ? pp.count : 1;
+	pp.list_cap[0] = pp.count > 1 && !pp.chained ? pp.count : 0;
 	const u64 lim = 1ull << 31;
 	// A folded pass: a node's list holds the edits from the first that crosses it on (the last one
 	// that fills or clears it whole, and the whole-node edits after that, are folded into its
@@ -4677,7 +5201,7 @@ static void plan_pass(const Pool &p, const hd_edit_desc *edits, PassPlan &pp) {
 		if (pp.folded)
 			pp.list_cap[l] = std::min(S[l] + std::min(inner[l], (u64)pp.count * pp.cap[l]), lim);
 		else
-			pp.list_cap[l] = pp.count > 1 ? std::min(2 * S[l], lim) : 0;
+			pp.list_cap[l] = pp.count > 1 && !pp.chained ? std::min(2 * S[l], lim) : 0;
 	}
 	pp.ev_cap = 0;
 	u64 pev_bytes = 0;
@@ -4719,7 +5243,8 @@ struct AsyncBufs {
 	ALevel *d_lv = nullptr;
 	u32 *pm = nullptr, *roots = nullptr, *acc = nullptr, *bcnt = nullptr, *head = nullptr, *blist = nullptr;
 	u32 *flag = nullptr, *lcnt = nullptr, *info = nullptr, *app = nullptr, *appo = nullptr, *etmp = nullptr, *rest = nullptr;
-	u32 *tsum = nullptr; // per-tile totals of the jobs' append scan
+	u32 *tsum = nullptr;  // per-tile totals of the jobs' append scan
+	u32 *saved = nullptr; // chained passes: the bucket counters before the pass, its flag and append count
 	uint4 *cstate = nullptr, *jrange = nullptr;
 	u32 etmp_cap = 0; // staging words of LDS jobs (bump-allocated)
 	Pair *bsum = nullptr;
@@ -4744,10 +5269,11 @@ static int async_setup(Pool &p, const std::vector<PassPlan> &plans, const std::v
 	const u32 L = p.dc.L, leafL = p.dc.color_leaf;
 	std::vector<u64> cap(L, 0), lcap(L, 0);
 	u64 ev = 0, maxpairs = 8;
-	bool stateful = false;
+	bool stateful = false, chained = false;
 	for (auto &pp : plans) {
 		if (!pp.async)
 			continue;
+		chained |= pp.chained;
 		for (u32 l = 0; l < L; ++l) {
 			cap[l] = std::max(cap[l], pp.cap[l]);
 			lcap[l] = std::max(lcap[l], pp.list_cap[l]);
@@ -4769,6 +5295,8 @@ static int async_setup(Pool &p, const std::vector<PassPlan> &plans, const std::v
 			HD_RET(buf(p, (pre + "kids").c_str(), l, 8 * c, &A.kids));
 			HD_RET(buf(p, (pre + "fchild").c_str(), l, c, &A.first_child));
 			HD_RET(buf(p, (pre + "pmask").c_str(), l, c, &A.pmask));
+			if (chained)
+				HD_RET(buf(p, (pre + "prev").c_str(), l, c, &A.prev));
 			if (stateful && l < leafL)
 				HD_RET(buf(p, (pre + "okids").c_str(), l, 8 * c, &A.okids));
 		}
@@ -4790,6 +5318,8 @@ static int async_setup(Pool &p, const std::vector<PassPlan> &plans, const std::v
 			HD_RET(buf(p, (pre + "own").c_str(), l, c, &A.own));
 		}
 	}
+	if (chained)
+		HD_RET(p.scratch.get<u32>(pre + "saved", p.total_buckets + 2, &B.saved));
 	HD_RET(p.scratch.get<ALevel>(pre + "levels", L, &B.d_lv));
 	HD_TRY(hipMemcpyAsync(B.d_lv, B.lv.data(), L * sizeof(ALevel), hipMemcpyHostToDevice, p.stream));
 	HD_RET(p.scratch.get<u32>(pre + "pm", kPmHdr + 2 * L, &B.pm));
@@ -4920,6 +5450,26 @@ static void queue_setnode(const Pool &p, const PassPlan &pp, const EditParams &P
 		a_setnode_down<<<grid_for(pp.cap[l], 256, 4096), 256, 0, s>>>(P, B.d_lv, B.pm, l, p.cnode_cap);
 }
 
+// SetNode of a chained pass: grid launches for the levels of more entries than one workgroup takes in a
+// few rounds, one workgroup for those above them (256 sphere edits on the 4096^3 terrain: @SETNODE@).
+constexpr u64 kChainWide = 1024;
+static void queue_chain_setnode(const Pool &p, const PassPlan &pp, const EditParams &P, const AsyncBufs &B, hipStream_t s) {
+	const u32 leafL = p.dc.color_leaf;
+	const ChainColor K{B.d_lv, B.info, B.appo, 0u, (u32)p.cnode_cap};
+	u32 lb = leafL;
+	u64 widest = 1;
+	for (u32 l = 0; l < leafL; ++l)
+		widest = std::max(widest, pp.cap[l]);
+	while (lb > 1 && pp.cap[lb - 1] > kChainWide)
+		--lb;
+	for (u32 l = leafL; l-- > lb;)
+		a_chain_up<<<grid_for(8 * pp.cap[l], kAT, 2048), kAT, 0, s>>>(P, K, l, B.pm);
+	a_chain_top<<<1, kSetNodeThreads, 0, s>>>(P, K, lb, B.pm, B.roots, p.cleaf_cap);
+	for (u32 l = lb; l + 1 < leafL; ++l)
+		a_chain_down<<<grid_for(8 * pp.cap[l], kAT, 2048), kAT, 0, s>>>(P, K, l, B.pm);
+	a_chain_nodes<<<dim3(grid_for(8 * widest, kAT, 1024), leafL), kAT, 0, s>>>(P, K, B.pm);
+}
+
 // Queues one sync-free pass (no host synchronization).
 static int queue_pass(Pool &p, const PassPlan &pp, AsyncBufs &B, bool reserve = true) {
 	const u32 L = p.dc.L, leafL = p.dc.color_leaf;
@@ -4931,28 +5481,32 @@ static int queue_pass(Pool &p, const PassPlan &pp, AsyncBufs &B, bool reserve = 
 	// most the pass's edits, and shrink with depth), so list-heavy levels go to the wide kernels
 	// (a pass of thousands of edits leaves only the root to the one workgroup: the wide kernels take
 	// the level below's nodes in parallel, 4096 mixed edits 0.8 ms faster)
-	const u64 lf = (std::min<u32>(pp.count, 4096) + 7) / 8;
+	const u64 lf = pp.chained ? 1 : (std::min<u32>(pp.count, 4096) + 7) / 8; // (chained: no lists)
 	u32 top_end = 0;
 	const u64 top_pairs = std::min<u64>(g_tuning.top_pairs, kTopPairs);
 	while (top_end + 1 < L && 8 * pp.cap[top_end] * lf <= top_pairs)
 		++top_end;
 	if (reserve)
 		HD_RET(gen_reserve(p, B, 1));
-	const auto top = pp.count > 1 ? a_top<true> : a_top<false>;
+	const auto top = pp.chained ? a_top<kTopChain> : pp.count > 1 ? a_top<kTopLists> : a_top<kTopOne>;
 	top<<<1, kAT, 0, p.stream>>>(P, B.d_lv, B.roots, B.pm, kPmHdr + 2 * L, top_end, B.ev, (u32)pp.ev_cap, B.gen_ctr);
 	// one 256-pair tile per block up to the block cap: a block's tiles are a chain of dependent round
 	// trips (entry, node words, color child), so a mid-size level spread over few blocks waits on
 	// them in turn (256 sphere edits on the 4096^3 terrain: 44.1 -> 41.0 ms per step vs 2048 pairs)
 	for (u32 l = top_end; l + 1 < L; ++l) {
 		u32 G = grid_for(8 * pp.cap[l] * lf, kAT, kMaxEmitBlocks);
-		a_count<<<G, kAT, 0, p.stream>>>(P, l, B.d_lv, B.pm, B.flag, B.lcnt, B.cstate, B.ev, (u32)pp.ev_cap, B.bsum);
+		(pp.chained ? a_count<true> : a_count<false>)<<<G, kAT, 0, p.stream>>>(P, l, B.d_lv, B.pm, B.flag, B.lcnt, B.cstate,
+		                                                                       B.ev, (u32)pp.ev_cap, B.bsum);
 		a_emit<<<G, kAT, 0, p.stream>>>(P, l, B.d_lv, B.pm, B.flag, B.lcnt, B.cstate, B.bsum);
 	}
+	if (pp.chained)
+		a_chain_begin<<<grid_for(p.total_buckets, kAT, 1024), kAT, 0, p.stream>>>(p.bucket_words, B.saved, p.total_buckets,
+		                                                                         p.meta, B.acc);
 	const bool colors = pp.stateful && pp.cap[leafL] > 0;
 	// A colored pass that proceeds only above the color leaves (its fills and clears land at or above
 	// them) has no color leaf job, yet the octree above the leaves may change (a fill color at a
 	// proceeding node, cleared children): SetNode alone, once the top-down has classified them.
-	if (pp.stateful && !colors && leafL > 0)
+	if (pp.stateful && !colors && leafL > 0 && !pp.chained)
 		queue_setnode(p, pp, P, B, p.stream);
 	const bool ljobs = lds_jobs(p.dc);
 	if (colors && !ljobs) { // the jobs' dense colors on the color stream, beside the leaves
@@ -4979,8 +5533,17 @@ static int queue_pass(Pool &p, const PassPlan &pp, AsyncBufs &B, bool reserve = 
 		a_leaf<kLeafNodes><<<leaf_grid, kAT, 0, p.stream>>>(P, B.d_lv, B.pm, B.lcol, B.lmask, B.lidx);
 	int l_from = -1; // levels [0, l_from] are small enough for a_bottom
 	const u64 small_level = std::min<u32>(g_tuning.small_level, kSmallLevel);
-	while (l_from + 1 < (int)L && pp.cap[l_from + 1] <= small_level)
+	while (!pp.chained && l_from + 1 < (int)L && pp.cap[l_from + 1] <= small_level)
 		++l_from;
+	auto write_colors = [&](hipStream_t s) { // the encoded chunks to their places
+		const u32 G = grid_for(pp.cap[leafL], 1, 8192);
+		a_encode_write<<<G, kEncThreads, 0, s>>>(P, B.d_lv, B.pm, B.dense, V, B.info, B.appo, p.cleaf_cap, B.etmp);
+		if (ljobs) {
+			const auto rest = V == kJobV ? a_job_rest<true> : a_job_rest<false>;
+			rest<<<std::min(G, 1024u), kEncThreads, 0, s>>>(P, B.d_lv, B.pm, B.jrange, B.lidx, B.ecol, V, B.info, B.appo,
+			                                               p.cleaf_cap, B.rest);
+		}
+	};
 	// the color leaves (job rebuild and encode) and SetNode on the color stream, beside the node
 	// levels; they start once the node levels have passed level color_after (L: right after the
 	// leaves)
@@ -5007,13 +5570,12 @@ static int queue_pass(Pool &p, const PassPlan &pp, AsyncBufs &B, bool reserve = 
 		a_scan_app<<<grid_for(pp.cap[leafL], kScanTile, 1024), kScanThreads, 0, p.cstream>>>(leafL, B.pm, B.app,
 		                                                                                    B.appo, B.tsum);
 		a_scan_fix<<<grid_for(pp.cap[leafL], 256 * 8, 1024), 256, 0, p.cstream>>>(leafL, B.pm, B.appo, B.tsum);
-		a_encode_write<<<G, kEncThreads, 0, p.cstream>>>(P, B.d_lv, B.pm, B.dense, V, B.info, B.appo, p.cleaf_cap,
-		                                                 B.etmp);
-		if (ljobs) {
-			const auto rest = V == kJobV ? a_job_rest<true> : a_job_rest<false>;
-			rest<<<std::min(G, 1024u), kEncThreads, 0, p.cstream>>>(P, B.d_lv, B.pm, B.jrange, B.lidx, B.ecol, V, B.info,
-			                                                        B.appo, p.cleaf_cap, B.rest);
-		} else
+		if (pp.chained) { // written once the pass is known to hold
+			HD_TRY(hipEventRecord(p.ev_color, p.cstream));
+			return HD_OK;
+		}
+		write_colors(p.cstream);
+		if (!ljobs)
 			a_encode_rest<<<std::min(G, 1024u), kEncThreads, 0, p.cstream>>>(P, B.d_lv, B.pm, B.dense, V, B.info,
 			                                                                 B.appo, p.cleaf_cap, B.rest);
 		queue_setnode(p, pp, P, B, p.cstream);
@@ -5026,7 +5588,9 @@ static int queue_pass(Pool &p, const PassPlan &pp, AsyncBufs &B, bool reserve = 
 		HD_RET(queue_colors());
 	for (int l = (int)L - 1; l > l_from; --l) {
 		u32 G = grid_for(pp.cap[l], kAT, 4096);
-		if (l + 1 < (int)L)
+		if (l + 1 < (int)L && pp.chained)
+			a_build_chain<16384><<<G, kAT, 0, p.stream>>>(P, (u32)l, B.d_lv, B.pm, B.G);
+		else if (l + 1 < (int)L)
 			// a single-edit pass has few color jobs beside it: twice the stage (256 sphere edits on
 			// the 4096^3 terrain: 41.1 -> 40.3 ms per step; the 4096-edit batch 1 % slower with it)
 			(pp.count == 1 ? a_build<20480> : a_build<10240>)<<<G, kAT, 0, p.stream>>>(P, (u32)l, B.d_lv, B.pm, B.G);
@@ -5037,11 +5601,40 @@ static int queue_pass(Pool &p, const PassPlan &pp, AsyncBufs &B, bool reserve = 
 	}
 	if (!colors_queued)
 		HD_RET(queue_colors());
-	a_bottom<<<1, kAT, 0, p.stream>>>(P, B.d_lv, B.pm, l_from, B.G, B.roots, B.acc, p.cnode_cap);
+	if (pp.chained) {
+		a_chain_end<<<1, kChainEdits, 0, p.stream>>>(P, B.d_lv, B.pm, B.G, B.roots, B.saved, p.total_buckets);
+		if (colors)
+			HD_TRY(hipStreamWaitEvent(p.stream, p.ev_color, 0));
+		if (pp.stateful)
+			queue_chain_setnode(p, pp, P, B, p.stream);
+		if (colors)
+			write_colors(p.stream);
+		a_chain_commit<<<1, kAT, 0, p.stream>>>(P, B.d_lv, B.pm, B.roots, B.acc, B.saved, p.total_buckets);
+		HD_TRY(hipGetLastError());
+		return HD_OK;
+	} else
+		a_bottom<<<1, kAT, 0, p.stream>>>(P, B.d_lv, B.pm, l_from, B.G, B.roots, B.acc, p.cnode_cap);
 	if (colors) // the next pass (and any host read) follows both streams
 		HD_TRY(hipStreamWaitEvent(p.stream, p.ev_color, 0));
 	HD_TRY(hipGetLastError());
 	return HD_OK;
+}
+
+// count edits from first on as one chained pass, or one by one when that is as fast (a chained pass
+// takes about as long as two single ones).
+constexpr u32 kChainMin = 3;
+constexpr u64 kChainBudget = 4ull << 30; // pass buffers a chained pass may take
+static void chain_split(u32 first, u32 count, std::vector<PassPlan> &plans) {
+	PassPlan pp;
+	pp.first = first, pp.count = count;
+	if (count >= kChainMin) {
+		pp.chained = true;
+		plans.push_back(pp);
+		return;
+	}
+	pp.count = 1;
+	for (u32 k = 0; k < count; ++k, ++pp.first)
+		plans.push_back(pp);
 }
 
 static bool force_sync_path() {
@@ -5057,12 +5650,25 @@ static int edit_sequence(Pool &p, u32 root, u32 croot, const std::vector<hd_edit
 	HD_RET(make_filled(p));
 	const bool sync_only = force_sync_path();
 	bool any_async = false;
-	for (auto &pp : plans) {
-		plan_pass(p, flat.data(), pp);
-		if (sync_only)
-			pp.async = false;
-		any_async |= pp.async;
+	std::vector<PassPlan> planned;
+	for (const PassPlan &q : plans) {
+		std::vector<PassPlan> part{q};
+		plan_pass(p, flat.data(), part[0]);
+		if (q.chained && !part[0].async) { // the synchronized pipeline has no chained passes
+			part.clear();
+			for (u32 k = 0; k < q.count; ++k)
+				chain_split(q.first + k, 1, part);
+			for (PassPlan &pp : part)
+				plan_pass(p, flat.data(), pp);
+		}
+		for (PassPlan &pp : part) {
+			if (sync_only)
+				pp.async = false;
+			any_async |= pp.async;
+			planned.push_back(pp);
+		}
 	}
+	plans.swap(planned);
 	if (!any_async) {
 		for (auto &pp : plans)
 			HD_RET(edit_pass(p, root, croot, flat.data() + pp.first, pp.count, &root, &croot));
@@ -5074,12 +5680,37 @@ static int edit_sequence(Pool &p, u32 root, u32 croot, const std::vector<hd_edit
 	HD_RET(async_setup(p, plans, flat, B));
 	a_set_roots<<<1, 64, 0, p.stream>>>(B.roots, root, croot, B.acc);
 	bool on_device = true;
-	for (auto &pp : plans) {
+	std::vector<PassPlan> todo(plans.rbegin(), plans.rend()); // a stack, first pass on top
+	while (!todo.empty()) {
+		const PassPlan pp = todo.back();
+		todo.pop_back();
 		if (pp.async) {
 			if (!on_device)
 				a_set_roots_keep<<<1, 64, 0, p.stream>>>(B.roots, root, croot);
 			on_device = true;
 			HD_RET(queue_pass(p, pp, B));
+			if (!pp.chained)
+				continue;
+			HD_TRY(hipMemcpyAsync(p.h_pass, B.pm, 4 * kPmHdr, hipMemcpyDeviceToHost, p.stream));
+			HD_TRY(hipStreamSynchronize(p.stream));
+			if (!p.h_pass[kPmCut])
+				continue;
+			// it did not hold: the edits before the cut in one pass, then the others; or one by one
+			a_chain_restore<<<grid_for(p.total_buckets, kAT, 1024), kAT, 0, p.stream>>>(p.bucket_words, B.saved,
+			                                                                           p.total_buckets);
+			std::vector<PassPlan> part;
+			if (p.h_pass[kPmFull])
+				for (u32 k = 0; k < pp.count; ++k)
+					chain_split(pp.first + k, 1, part);
+			else {
+				const u32 head = std::max(~p.h_pass[kPmCut], 1u);
+				chain_split(pp.first, head, part);
+				chain_split(pp.first + head, pp.count - head, part);
+			}
+			for (auto it = part.rbegin(); it != part.rend(); ++it) {
+				plan_pass(p, flat.data(), *it);
+				todo.push_back(*it);
+			}
 		} else {
 			if (on_device) {
 				u32 rr[2];
@@ -5125,12 +5756,70 @@ static void batched_plans(const Pool &p, const hd_edit_desc *edits, u32 n, std::
 			plans.push_back(pp);
 		}
 }
-static void plain_plans(const hd_edit_desc *edits, u32 n, std::vector<hd_edit_desc> &flat,
+// Whether an edit may share a chained pass at all: no column fill, colors (if any) plain RGB8.
+static bool chains(const Pool &p, const hd_edit_desc &d) {
+	if (d.kind == HD_EDIT_COLUMN_FILL)
+		return false;
+	return !is_stateful(d) || (d.color.has_value && !d.color.bits_per_weight && lds_jobs(p.dc) && p.dc.color_leaf > 0);
+}
+// Whether two edits may reach the same node of size S or below: its cube would meet both shapes, so
+// their S-aligned bounds meet and their distance is at most the cube's diagonal.
+static bool may_share_nodes(const hd_edit_desc &a, const hd_edit_desc &b, i64 S) {
+	auto ball = [](const hd_edit_desc &d) { return d.kind <= HD_EDIT_SPHERE_PAINT; };
+	auto radius = [](const hd_edit_desc &d) { return std::sqrt((double)d.r2) + 1.0; };
+	double d2 = 0;
+	for (int i = 0; i < 3; ++i) {
+		double lo[2], hi[2]; // the shapes' closed bounds, spheres as their centre
+		i64 c0[2], c1[2];    // the nodes whose closed cubes meet them
+		for (int k = 0; k < 2; ++k) {
+			const hd_edit_desc &d = k ? b : a;
+			lo[k] = (double)d.p0[i];
+			hi[k] = ball(d) ? lo[k] : std::max(lo[k], (double)d.p1[i]);
+			const double r = ball(d) ? radius(d) : 0.0;
+			c0[k] = (i64)std::floor((lo[k] - r) / (double)S) - 1;
+			c1[k] = (i64)std::floor((hi[k] + r) / (double)S);
+		}
+		if (c1[0] < c0[1] || c1[1] < c0[0])
+			return false;
+		const double g = std::max(0.0, std::max(lo[0] - hi[1], lo[1] - hi[0]));
+		d2 += g * g;
+	}
+	const double reach = (ball(a) ? radius(a) : 0.0) + (ball(b) ? radius(b) : 0.0) + (double)S * std::sqrt(3.0) + 1.0;
+	return d2 <= reach * reach;
+}
+// The passes of a plain call: runs of consecutive edits of which no two may reach the same leaf (with
+// colors: the same color leaf), each run one chained pass; the others one by one.
+static void plain_plans(const Pool &p, const hd_edit_desc *edits, u32 n, std::vector<hd_edit_desc> &flat,
                         std::vector<PassPlan> &plans) {
 	flat.assign(edits, edits + n);
-	plans.assign(n, PassPlan{});
-	for (u32 i = 0; i < n; ++i)
-		plans[i].first = i, plans[i].count = 1;
+	for (u32 i = 0; i < n;) {
+		u32 j = i + 1u;
+		if (chains(p, edits[i]) && !force_sync_path())
+			for (; j < n && j - i < kChainEdits && chains(p, edits[j]); ++j) {
+				bool apart = true;
+				for (u32 k = i; k < j && apart; ++k) {
+					const bool col = is_stateful(edits[j]) || is_stateful(edits[k]);
+					const u32 bits = col ? std::max(2u, p.dc.voxel_level - p.dc.color_leaf) : 2u;
+					apart = !may_share_nodes(edits[k], edits[j], (i64)1 << bits);
+				}
+				if (!apart)
+					break;
+			}
+		// a run whose buffers together exceed the budget is halved
+		for (u32 m = j - i;; m = (m + 1u) / 2u) {
+			std::vector<PassPlan> part;
+			chain_split(i, m, part);
+			if (part[0].chained) {
+				plan_pass(p, flat.data(), part[0]);
+				const u64 symbols = part[0].stateful ? p.cnode_cap + *std::max_element(part[0].cap.begin(), part[0].cap.end()) : 0;
+				if (!part[0].async || part[0].bytes > kChainBudget || symbols >= kColorKeep)
+					continue;
+			}
+			plans.insert(plans.end(), part.begin(), part.end());
+			i += m;
+			break;
+		}
+	}
 }
 
 // Folded passes: runs of consecutive edits, each run one pass whose node edit lists keep submission
@@ -5225,7 +5914,7 @@ int edit_batched(Pool &p, u32 root, u32 croot, const hd_edit_desc *edits, u32 n,
 int edit_plain(Pool &p, u32 root, u32 croot, const hd_edit_desc *edits, u32 n, u32 *root_out, u32 *croot_out) {
 	std::vector<hd_edit_desc> flat;
 	std::vector<PassPlan> plans;
-	plain_plans(edits, n, flat, plans);
+	plain_plans(p, edits, n, flat, plans);
 	p.last_groups = n;
 	return edit_sequence(p, root, croot, flat, plans, root_out, croot_out);
 }
@@ -5237,7 +5926,7 @@ static int edit_reserve(Pool &p, const hd_edit_desc *edits, u32 n, u32 mode) {
 	if (mode == HD_MODE_BATCHED && n > 1)
 		batch_plans(p, edits, n, flat, plans);
 	else
-		plain_plans(edits, n, flat, plans);
+		plain_plans(p, edits, n, flat, plans);
 	bool any_async = false;
 	for (auto &pp : plans) {
 		plan_pass(p, flat.data(), pp);

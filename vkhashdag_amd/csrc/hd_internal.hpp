@@ -124,6 +124,7 @@ struct Pool {
 	u32 last_groups = 0;
 	double last_ms = 0;
 	u32 edit_gen = 0; // generation of the sync-free pass's group table (hd_edit.hip)
+	u32 *h_pass = nullptr; // pinned: a chained pass's counters, read back after its top-down
 	GcPlan gc_plan;   // hd_gc's buffers
 };
 

@@ -192,6 +192,8 @@ int hd_pool_create(const hd_config *cfg, hd_pool **out) {
 		return fail(e);
 	if ((e = hipEventCreateWithFlags(&p.ev_color, hipEventDisableTiming)) != hipSuccess)
 		return fail(e);
+	if ((e = hipHostMalloc((void **)&p.h_pass, 64, hipHostMallocDefault)) != hipSuccess)
+		return fail(e);
 	if ((e = hipMalloc(&p.words, (words + kWordsPad) * 4)) != hipSuccess)
 		return fail(e);
 	if ((e = hipMalloc(&p.bucket_words, buckets * 4)) != hipSuccess)
@@ -233,6 +235,8 @@ int hd_pool_destroy(hd_pool *h) {
 	                  (void *)p.cleaves, (void *)p.hm_mn, (void *)p.hm_mx, (void *)p.d_hm})
 		if (ptr)
 			(void)hipFree(ptr);
+	if (p.h_pass)
+		(void)hipHostFree(p.h_pass);
 	if (p.stream)
 		(void)hipStreamDestroy(p.stream);
 	if (p.cstream)
