@@ -24,6 +24,7 @@
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
+#include <functional>
 #include <string>
 
 namespace hd {
@@ -817,9 +818,9 @@ struct Pair {
 __device__ inline u32 pair_bits(u32 f, u32 k) {
 	return ((f & 1u) << k) | (((f >> 1) & 1u) << (8 + k)) | (((f >> 2) & 1u) << (16 + k)) | ((f >> 3) << (24 + k));
 }
-// Block-wide exclusive scan of kAT pairs: shuffle scans inside each wavefront, one LDS exchange
-// of the wavefront totals (two barriers). sh needs kAT / 64 entries.
-__device__ inline Pair block_excl_scan2(Pair x, Pair *sh, Pair &total) {
+// Block-wide exclusive scan of kT pairs: shuffle scans inside each wavefront, one LDS exchange
+// of the wavefront totals (two barriers). sh needs kT / 64 entries.
+template <u32 kT = kAT> __device__ inline Pair block_excl_scan2(Pair x, Pair *sh, Pair &total) {
 	const u32 lane = threadIdx.x & 63u, w = threadIdx.x >> 6;
 	Pair v = x;
 #pragma unroll
@@ -833,7 +834,7 @@ __device__ inline Pair block_excl_scan2(Pair x, Pair *sh, Pair &total) {
 	__syncthreads();
 	Pair pre{0, 0}, tot{0, 0};
 #pragma unroll
-	for (u32 k = 0; k < kAT / 64; ++k) {
+	for (u32 k = 0; k < kT / 64; ++k) {
 		Pair s = sh[k];
 		if (k < w)
 			pre.a += s.a, pre.b += s.b;
@@ -1540,7 +1541,7 @@ __device__ inline void chain_link(const ALevel *__restrict__ lv, u32 l, const En
 __device__ inline void chain_roots(const EditParams &P, const ALevel &A0, const u32 *__restrict__ roots,
                                    u32 *__restrict__ pm) {
 	const u32 root = roots[0], croot = roots[1];
-	for (u32 k = threadIdx.x; k < P.n_edits; k += kAT) {
+	for (u32 k = threadIdx.x; k < P.n_edits; k += blockDim.x) {
 		const DevEditor ed = P.editor(k);
 		const Classified c = classify_single(P, ed, 0, 0, 0, 0, root, croot, 0u);
 		const Entry E{0, 0, 0, root, kNull, c.sf & ~kSfNewJob, c.octree, kNull, k, 1u};
@@ -1560,27 +1561,31 @@ __device__ inline void chain_roots(const EditParams &P, const ALevel &A0, const 
 constexpr u32 kTopEnt = kTopPairs / 8;
 constexpr u32 kTopEdits = 1024; // a pass with at most this many edits reads them from LDS in a_top
 // kMode: one edit; several (nodes may carry edit lists); several chained (an entry has one edit each).
+// A chained pass's levels hold an entry per edit and more: its workgroup takes a level of up to 128 entries
+// at once (256 sphere edits on the 4096^3 terrain, 27 per pass: @TOP@ us a pass).
 enum : u32 { kTopOne = 0, kTopLists = 1, kTopChain = 2 };
+template <u32 kMode> constexpr u32 kTopThreads = kMode == kTopChain ? 1024 : kAT;
 template <u32 kMode>
-__global__ void __launch_bounds__(kAT) a_top(EditParams P0, const ALevel *__restrict__ lv, u32 *__restrict__ roots,
+__global__ void __launch_bounds__(kTopThreads<kMode>) a_top(EditParams P0, const ALevel *__restrict__ lv, u32 *__restrict__ roots,
                                              u32 *__restrict__ pm, u32 pm_words, u32 l_end, PushEvent *ev, u32 ev_cap,
                                              u32 *__restrict__ gen_ctr) {
+	constexpr u32 kT = kTopThreads<kMode>;
 	constexpr bool kLists = kMode == kTopLists, kChain = kMode == kTopChain;
-	__shared__ Pair sh[kAT];
-	__shared__ u32 sflag[kAT];
+	__shared__ Pair sh[kT];
+	__shared__ u32 sflag[kT];
 	__shared__ Entry sent[2][kTopEnt];
 	__shared__ u32 scount;
 	__shared__ hd_edit_desc sedit[kTopEdits];
 	__shared__ u32 sfilled[HD_MAX_LEVELS];
-	__shared__ u32 sbits[kLists ? kAT : 1][kTopEdits / 32]; // per thread: the list edits touching its child
-	for (u32 i = threadIdx.x; i < pm_words; i += kAT)
+	__shared__ u32 sbits[kLists ? kT : 1][kTopEdits / 32]; // per thread: the list edits touching its child
+	for (u32 i = threadIdx.x; i < pm_words; i += kT)
 		pm[i] = 0;
 	// the pass's edits and the filled chain are read by every classification: keep them in LDS
 	EditParams P = P0;
 	if (P.n_edits <= kTopEdits) {
 		const u32 *src = reinterpret_cast<const u32 *>(P.edits);
 		u32 *dst = reinterpret_cast<u32 *>(sedit);
-		for (u32 i = threadIdx.x; i < P.n_edits * (u32)(sizeof(hd_edit_desc) / 4); i += kAT)
+		for (u32 i = threadIdx.x; i < P.n_edits * (u32)(sizeof(hd_edit_desc) / 4); i += kT)
 			dst[i] = src[i];
 		P.edits = sedit;
 	}
@@ -1591,7 +1596,7 @@ __global__ void __launch_bounds__(kAT) a_top(EditParams P0, const ALevel *__rest
 	if (kChain) {
 		chain_roots(P, lv[0], roots, pm);
 		__syncthreads();
-		for (u32 k = threadIdx.x; k < P.n_edits; k += kAT)
+		for (u32 k = threadIdx.x; k < P.n_edits; k += kT)
 			sent[0][k] = lv[0].ent[k];
 		if (threadIdx.x == 0)
 			scount = P.n_edits;
@@ -1694,7 +1699,7 @@ __global__ void __launch_bounds__(kAT) a_top(EditParams P0, const ALevel *__rest
 		const Entry *cur = sent[l & 1];
 		Entry *nxt = sent[(l + 1) & 1];
 		Pair base{0, 0};
-		for (u64 t0 = 0; t0 < (u64)n * 8u; t0 += kAT) {
+		for (u64 t0 = 0; t0 < (u64)n * 8u; t0 += kT) {
 			const u64 t = t0 + threadIdx.x;
 			const bool in = t < (u64)n * 8u;
 			PairOut o{0, 0, make_uint4(0, 0, 0, 0), kNull};
@@ -1721,7 +1726,7 @@ __global__ void __launch_bounds__(kAT) a_top(EditParams P0, const ALevel *__rest
 			}
 			sflag[threadIdx.x] = o.flag;
 			Pair tile;
-			Pair off = block_excl_scan2(Pair{o.flag & 1u, o.lcnt}, sh, tile); // synchronizes sflag
+			Pair off = block_excl_scan2<kT>(Pair{o.flag & 1u, o.lcnt}, sh, tile); // synchronizes sflag
 			if (in) {
 				u32 m8 = 0;
 				if ((t & 7u) == 0)
@@ -2654,14 +2659,250 @@ __global__ void __launch_bounds__(kAT) a_build_chain(EditParams P, u32 l, const 
 		} while (__syncthreads_or(todo));
 	}
 }
+// The levels [0, l_from] of a chained pass, each of at most kChainSmall entries, in one workgroup (a thread
+// per entry): the join over the versions' rows in LDS (children's results by slot, left there by the level
+// below), the find, the grouping of identical new contents and the appends, as a_build_chain, a_dedup and
+// a_walk do level by level in three launches of 5 us and more.
+constexpr u32 kChainSmall = 1024, kChainTab = 2048, kChainStage = 16384;
+struct ChainLds {
+	union {
+		u32 row[kChainSmall][8]; // a proceeding slot's result, until the joins are done
+		u32 content[kChainSmall][9];
+	};
+	unsigned char flag[kChainSmall][8]; // of the result: bit 0 a fresh append, bit 1 unchanged
+	union {
+		__align__(16) u32 stage[kChainStage]; // the scanned buckets' words
+		struct { // lowest entry per content; per bucket: its lowest group, its groups, how many
+			u32 tab[kChainTab], bkey[kChainTab], bmin[kChainTab], bhead[kChainTab], bn[kChainTab];
+		};
+	};
+	u32 hash[kChainSmall], bucket[kChainSmall], next[kChainSmall], csz[kChainSmall], res[kChainSmall];
+	u32 prev[kChainSmall], pmw[kChainSmall];
+	u32 top, appended;
+};
+static_assert(5 * kChainTab <= kChainStage && kChainTab >= 2 * kChainSmall && kChainTab == 1u << 11);
+__global__ void __launch_bounds__(kChainSmall) a_chain_small(EditParams P, const ALevel *__restrict__ lv,
+                                                             u32 *__restrict__ pm, int l_from, GroupTable G,
+                                                             u32 *__restrict__ acc) {
+	__shared__ ChainLds S;
+	const u32 e = threadIdx.x;
+	if (e == 0)
+		S.appended = 0;
+	JoinIn q{};
+	u32 sf = 0, pv = kNull;
+	auto load = [&](int l) {
+		const ALevel &A = lv[l];
+		if (e < pm[kPmHdr + l]) {
+			q = load_join(A, e);
+			sf = ldg(&A.ent[e].sf, 0);
+			pv = ldg(A.prev, e);
+		}
+	};
+	load(l_from);
+	for (int l = l_from; l >= 0; --l) {
+		const ALevel &A = lv[l];
+		const u32 n = min(pm[kPmHdr + l], kChainSmall);
+		const bool act = e < n;
+		const u32 pmk = q.pmw & 0xFFu;
+		if (act) {
+			S.prev[e] = pv;
+			S.pmw[e] = q.pmw;
+			if (l == l_from) {
+				const u32 cnt = (u32)__builtin_popcount(pmk);
+				uint2 cr[8];
+#pragma unroll
+				for (u32 j = 0; j < 8; ++j)
+					cr[j] = cnt ? chain_child(lv[l + 1], G, q.fc + min(j, cnt - 1u)) : make_uint2(kNull, 2u);
+				u32 rank = 0;
+#pragma unroll
+				for (u32 i = 0; i < 8; ++i)
+					if ((pmk >> i) & 1u) {
+						uint2 c = cr[0];
+#pragma unroll
+						for (u32 j = 1; j <= i; ++j)
+							c = rank == j ? cr[j] : c;
+						S.row[e][i] = c.x;
+						S.flag[e][i] = (unsigned char)c.y;
+						++rank;
+					}
+			}
+		}
+		__syncthreads();
+		// the join (chain_join)
+		u32 c[9], k = 0, h = 0, b = 0, bw = 0, r = kNull, rf = 0; // content, its size, hash, bucket; the result
+		bool fresh = false;
+		if (act) {
+			const u32 kv[8] = {q.k0.x, q.k0.y, q.k0.z, q.k0.w, q.k1.x, q.k1.y, q.k1.z, q.k1.w};
+			u32 nk[8], st[8], own = 0;
+#pragma unroll
+			for (u32 i = 0; i < 8; ++i) {
+				const bool pr = (pmk >> i) & 1u;
+				const u32 f = pr ? S.flag[e][i] : 2u;
+				const bool set = pr ? !(f & 2u) : ((q.pmw >> (8u + i)) & 1u) != 0u;
+				nk[i] = pr ? S.row[e][i] : kv[i];
+				st[i] = kv[i];
+				own |= (set ? 1u : 0u) << i;
+				fresh |= set && pr && (f & 1u);
+			}
+			const bool colored = (sf & kSfActive) != 0u;
+			u32 need = colored ? 0xFFu : own ? 0xFFu & ~own : 0u;
+			for (u32 v = need ? pv : kNull; v != kNull && need; v = S.prev[v]) {
+				const u32 vm = S.pmw[v];
+				for (u32 m = ((vm & 0xFFu) | (vm >> 8)) & need & 0xFFu; m; m &= m - 1u) {
+					const u32 i = (u32)__builtin_ctz(m);
+					u32 x, f = 0;
+					if ((vm >> i) & 1u) {
+						x = S.row[v][i];
+						f = S.flag[v][i];
+					} else
+						x = ldg(A.kids, 8ull * v + i);
+					if (f & 2u)
+						continue;
+					fresh |= !((own >> i) & 1u) && (f & 1u);
+					need &= ~(1u << i);
+#pragma unroll
+					for (u32 j = 0; j < 8; ++j)
+						st[j] = j == i ? x : st[j];
+				}
+			}
+			if (colored) {
+				bool bad = false;
+#pragma unroll
+				for (u32 i = 0; i < 8; ++i)
+					bad |= !((q.pmw >> (8u + i)) & 1u) && (st[i] == kNull) != (kv[i] == kNull);
+				if (bad)
+					chain_cut(pm, ldg(&A.ent[e].loff, 0));
+			}
+			u32 nm = 0;
+#pragma unroll
+			for (u32 i = 0; i < 8; ++i) {
+				nk[i] = (own >> i) & 1u ? nk[i] : st[i];
+				nm |= (nk[i] != kNull ? 1u : 0u) << i;
+			}
+			if (!own)
+				rf = 2u;
+			else if (nm) {
+				pack_inner(nm, nk, c);
+				k = (u32)__builtin_popcount(nm) + 1u;
+				h = murmur_regs(c, k);
+				b = P.c.level_base[l] + (h & ((1u << P.c.bucket_bits[l]) - 1u));
+			}
+		}
+		// the find among the bucket's existing nodes (a node with a fresh child is new)
+		bool todo = k != 0u;
+		do {
+			if (e == 0)
+				S.top = 0;
+			__syncthreads();
+			if (todo) {
+				if (fresh)
+					bw = ldg(P.bucket_words, b);
+				else
+					r = find_in_bucket_staged(P.words, P.bucket_words, P.c, b, c, k, headers_by_value(P.c, (u32)l), bw,
+					                          S.stage, &S.top, kChainStage);
+				todo = r == kFindRetry;
+			}
+		} while (__syncthreads_or(todo));
+		const bool need = k != 0u && r == kNull;
+		const u32 pidx = q.pidx, ptr = q.ptr;
+		if (l > 0)
+			load(l - 1); // in flight during the grouping
+		for (u32 i = e; i < 5u * kChainTab; i += kChainSmall)
+			S.stage[i] = i < 4u * kChainTab ? kNull : 0u;
+		if (need) {
+#pragma unroll
+			for (u32 j = 0; j < 9; ++j)
+				if (j < k)
+					S.content[e][j] = c[j];
+			S.csz[e] = k;
+			S.hash[e] = h;
+			S.bucket[e] = b;
+		}
+		__syncthreads();
+		u32 sl = ((h ^ (h >> 15)) * 0x2c1b3c6du) & (kChainTab - 1u);
+		if (need)
+			for (;;) { // identical contents share a slot, its lowest entry appends
+				const u32 x = atomicCAS(&S.tab[sl], kNull, e);
+				if (x == kNull)
+					break;
+				bool same = S.hash[x] == h && S.csz[x] == k;
+#pragma unroll
+				for (u32 j = 0; j < 9; ++j)
+					same = same && (j >= k || S.content[x][j] == c[j]);
+				if (same) {
+					atomicMin(&S.tab[sl], e);
+					break;
+				}
+				sl = (sl + 1u) & (kChainTab - 1u);
+			}
+		__syncthreads();
+		const u32 lead = need ? S.tab[sl] : kNull;
+		u32 m = (b * 0x9E3779B1u >> 7) & (kChainTab - 1u);
+		if (need && lead == e) {
+			for (;;) {
+				const u32 x = atomicCAS(&S.bkey[m], kNull, b);
+				if (x == kNull || x == b)
+					break;
+				m = (m + 1u) & (kChainTab - 1u);
+			}
+			atomicMin(&S.bmin[m], e);
+			atomicAdd(&S.bn[m], 1u);
+			S.next[e] = atomicExch(&S.bhead[m], e);
+		}
+		__syncthreads();
+		if (need && lead == e && S.bmin[m] == e) { // the bucket's new nodes in entry order
+			const u32 cnt = S.bn[m];
+			u32 done = 0;
+			if (cnt == 1u) {
+				const u32 f = append_regs(P.words, P.c, b, bw, c, k);
+				S.res[e] = f;
+				done += f != kNull ? 1u : 0u;
+			} else
+				for (u32 i = 0, last = e; i < cnt; ++i) {
+					u32 x = i ? kNull : e;
+					if (i)
+						for (u32 y = S.bhead[m]; y != kNull; y = S.next[y])
+							if (y > last && y < x)
+								x = y;
+					last = x;
+					const u32 f = append_to_bucket(P.words, P.c, b, bw, S.content[x], S.csz[x]);
+					S.res[x] = f;
+					done += f != kNull ? 1u : 0u;
+				}
+			stg(P.bucket_words, b, bw);
+			if (done)
+				atomicAdd(&S.appended, done);
+			if (done != cnt)
+				atomicOr(&P.meta[kMetaOverflow], 1u);
+		}
+		__syncthreads();
+		if (need) {
+			r = S.res[lead];
+			rf = r == kNull ? 2u : 1u;
+		}
+		if (act && l > 0) {
+			S.row[pidx >> 3][pidx & 7u] = r;
+			S.flag[pidx >> 3][pidx & 7u] = (unsigned char)rf;
+		} else if (act) { // the root's versions, for a_chain_end
+			stg(A.pend, e, 0u);
+			stg(A.status, e, rf & 2u ? ptr : r);
+		}
+	}
+	__syncthreads();
+	if (e == 0 && S.appended)
+		atomicAdd(&acc[kAccUpserts], S.appended);
+}
 // Before a chained pass's first append: the bucket counters, the pool's full-bucket flag (cleared, so that
 // the pass sees its own) and the append count are saved.
 __global__ void a_chain_begin(const u32 *__restrict__ bucket_words, u32 *__restrict__ saved, u64 n,
-                              u32 *__restrict__ meta, const u32 *__restrict__ acc) {
+                              u32 *__restrict__ meta, const u32 *__restrict__ acc, u32 *__restrict__ pm,
+                              const u32 *__restrict__ roots) {
 	const u64 t0 = (u64)blockIdx.x * blockDim.x + threadIdx.x;
 	for (u64 i = t0; i < n; i += (u64)gridDim.x * blockDim.x)
 		saved[i] = bucket_words[i];
 	if (t0 == 0) {
+		pm[kPmCroot] = roots[1];
+		pm[kPmNodes] = meta[kMetaColorNodes];
 		saved[n] = atomicAnd(&meta[kMetaOverflow], ~1u) & 1u;
 		saved[n + 1u] = acc[kAccUpserts];
 	}
@@ -2694,8 +2935,6 @@ __global__ void __launch_bounds__(kChainEdits) a_chain_end(EditParams P, const A
 			chain_cut(pm, k);
 		if (k == n - 1u) {
 			pm[kPmRoot] = ver[k].y & 2u ? at : ver[k].x;
-			pm[kPmCroot] = roots[1];
-			pm[kPmNodes] = P.meta[kMetaColorNodes];
 			if (P.meta[kMetaOverflow] & 1u) {
 				atomicAnd(&P.meta[kMetaOverflow], ~1u);
 				pm[kPmFull] = 1u;
@@ -2706,7 +2945,7 @@ __global__ void __launch_bounds__(kChainEdits) a_chain_end(EditParams P, const A
 	}
 }
 // The last kernel of a chained pass (one workgroup): the roots, color counters and statistics, if it held.
-__global__ void __launch_bounds__(kAT) a_chain_commit(EditParams P, const ALevel *__restrict__ lv,
+__global__ void __launch_bounds__(kChainSmall) a_chain_commit(EditParams P, const ALevel *__restrict__ lv,
                                                       const u32 *__restrict__ pm, u32 *__restrict__ roots,
                                                       u32 *__restrict__ acc, const u32 *__restrict__ saved, u64 n_saved) {
 	if (pm[kPmCut]) {
@@ -2718,7 +2957,7 @@ __global__ void __launch_bounds__(kAT) a_chain_commit(EditParams P, const ALevel
 	}
 	u32 jobs = 0; // the color leaves that colored edits enter
 	if (P.stateful)
-		for (u32 e = threadIdx.x; e < pm[kPmHdr + P.c.color_leaf]; e += kAT)
+		for (u32 e = threadIdx.x; e < pm[kPmHdr + P.c.color_leaf]; e += kChainSmall)
 			jobs += ldg(&lv[P.c.color_leaf].ent[e].sf, 0) & kSfActive ? 1u : 0u;
 #pragma unroll
 	for (u32 d = 32; d > 0; d >>= 1)
@@ -5457,9 +5696,6 @@ static void queue_chain_setnode(const Pool &p, const PassPlan &pp, const EditPar
 	const u32 leafL = p.dc.color_leaf;
 	const ChainColor K{B.d_lv, B.info, B.appo, 0u, (u32)p.cnode_cap};
 	u32 lb = leafL;
-	u64 widest = 1;
-	for (u32 l = 0; l < leafL; ++l)
-		widest = std::max(widest, pp.cap[l]);
 	while (lb > 1 && pp.cap[lb - 1] > kChainWide)
 		--lb;
 	for (u32 l = leafL; l-- > lb;)
@@ -5467,11 +5703,20 @@ static void queue_chain_setnode(const Pool &p, const PassPlan &pp, const EditPar
 	a_chain_top<<<1, kSetNodeThreads, 0, s>>>(P, K, lb, B.pm, B.roots, p.cleaf_cap);
 	for (u32 l = lb; l + 1 < leafL; ++l)
 		a_chain_down<<<grid_for(8 * pp.cap[l], kAT, 2048), kAT, 0, s>>>(P, K, l, B.pm);
-	a_chain_nodes<<<dim3(grid_for(8 * widest, kAT, 1024), leafL), kAT, 0, s>>>(P, K, B.pm);
+}
+static void queue_chain_nodes(const Pool &p, const PassPlan &pp, const EditParams &P, const AsyncBufs &B, hipStream_t s) {
+	const u32 leafL = p.dc.color_leaf;
+	const ChainColor K{B.d_lv, B.info, B.appo, 0u, (u32)p.cnode_cap};
+	u64 widest = 1;
+	for (u32 l = 0; l < leafL; ++l)
+		widest = std::max(widest, pp.cap[l]);
+	a_chain_nodes<<<dim3(grid_for(8 * widest, kAT, 128), leafL), kAT, 0, s>>>(P, K, B.pm);
 }
 
-// Queues one sync-free pass (no host synchronization).
-static int queue_pass(Pool &p, const PassPlan &pp, AsyncBufs &B, bool reserve = true) {
+// Queues one sync-free pass (no host synchronization). held (optional) is asked once the top-down, which
+// writes the pass's own buffers only, is queued: false leaves it at that.
+static int queue_pass(Pool &p, const PassPlan &pp, AsyncBufs &B, bool reserve = true,
+                      const std::function<bool()> &held = nullptr) {
 	const u32 L = p.dc.L, leafL = p.dc.color_leaf;
 	if (pp.stateful && lds_jobs(p.dc) && pp.count >= kNoEdit) // leaves record edits by 16-bit index
 		return set_error("hd_edit: a colored pass holds at most %u edits", kNoEdit - 1u), HD_ERR_ARG;
@@ -5489,7 +5734,7 @@ static int queue_pass(Pool &p, const PassPlan &pp, AsyncBufs &B, bool reserve = 
 	if (reserve)
 		HD_RET(gen_reserve(p, B, 1));
 	const auto top = pp.chained ? a_top<kTopChain> : pp.count > 1 ? a_top<kTopLists> : a_top<kTopOne>;
-	top<<<1, kAT, 0, p.stream>>>(P, B.d_lv, B.roots, B.pm, kPmHdr + 2 * L, top_end, B.ev, (u32)pp.ev_cap, B.gen_ctr);
+	top<<<1, pp.chained ? kTopThreads<kTopChain> : kAT, 0, p.stream>>>(P, B.d_lv, B.roots, B.pm, kPmHdr + 2 * L, top_end, B.ev, (u32)pp.ev_cap, B.gen_ctr);
 	// one 256-pair tile per block up to the block cap: a block's tiles are a chain of dependent round
 	// trips (entry, node words, color child), so a mid-size level spread over few blocks waits on
 	// them in turn (256 sphere edits on the 4096^3 terrain: 44.1 -> 41.0 ms per step vs 2048 pairs)
@@ -5499,9 +5744,11 @@ static int queue_pass(Pool &p, const PassPlan &pp, AsyncBufs &B, bool reserve = 
 		                                                                       B.ev, (u32)pp.ev_cap, B.bsum);
 		a_emit<<<G, kAT, 0, p.stream>>>(P, l, B.d_lv, B.pm, B.flag, B.lcnt, B.cstate, B.bsum);
 	}
+	if (held && !held())
+		return HD_OK;
 	if (pp.chained)
 		a_chain_begin<<<grid_for(p.total_buckets, kAT, 1024), kAT, 0, p.stream>>>(p.bucket_words, B.saved, p.total_buckets,
-		                                                                         p.meta, B.acc);
+		                                                                         p.meta, B.acc, B.pm, B.roots);
 	const bool colors = pp.stateful && pp.cap[leafL] > 0;
 	// A colored pass that proceeds only above the color leaves (its fills and clears land at or above
 	// them) has no color leaf job, yet the octree above the leaves may change (a fill color at a
@@ -5533,7 +5780,9 @@ static int queue_pass(Pool &p, const PassPlan &pp, AsyncBufs &B, bool reserve = 
 		a_leaf<kLeafNodes><<<leaf_grid, kAT, 0, p.stream>>>(P, B.d_lv, B.pm, B.lcol, B.lmask, B.lidx);
 	int l_from = -1; // levels [0, l_from] are small enough for a_bottom
 	const u64 small_level = std::min<u32>(g_tuning.small_level, kSmallLevel);
-	while (!pp.chained && l_from + 1 < (int)L && pp.cap[l_from + 1] <= small_level)
+	const u64 small = pp.chained ? kChainSmall : small_level;
+	const int small_end = pp.chained ? (int)L - 1 : (int)L; // (a chained pass's leaves take the grid kernels)
+	while (l_from + 1 < small_end && pp.cap[l_from + 1] <= small)
 		++l_from;
 	auto write_colors = [&](hipStream_t s) { // the encoded chunks to their places
 		const u32 G = grid_for(pp.cap[leafL], 1, 8192);
@@ -5570,7 +5819,8 @@ static int queue_pass(Pool &p, const PassPlan &pp, AsyncBufs &B, bool reserve = 
 		a_scan_app<<<grid_for(pp.cap[leafL], kScanTile, 1024), kScanThreads, 0, p.cstream>>>(leafL, B.pm, B.app,
 		                                                                                    B.appo, B.tsum);
 		a_scan_fix<<<grid_for(pp.cap[leafL], 256 * 8, 1024), 256, 0, p.cstream>>>(leafL, B.pm, B.appo, B.tsum);
-		if (pp.chained) { // written once the pass is known to hold
+		if (pp.chained) { // decided beside the node levels, written once the pass is known to hold
+			queue_chain_setnode(p, pp, P, B, p.cstream);
 			HD_TRY(hipEventRecord(p.ev_color, p.cstream));
 			return HD_OK;
 		}
@@ -5602,14 +5852,18 @@ static int queue_pass(Pool &p, const PassPlan &pp, AsyncBufs &B, bool reserve = 
 	if (!colors_queued)
 		HD_RET(queue_colors());
 	if (pp.chained) {
+		if (l_from >= 0)
+			a_chain_small<<<1, kChainSmall, 0, p.stream>>>(P, B.d_lv, B.pm, l_from, B.G, B.acc);
 		a_chain_end<<<1, kChainEdits, 0, p.stream>>>(P, B.d_lv, B.pm, B.G, B.roots, B.saved, p.total_buckets);
 		if (colors)
 			HD_TRY(hipStreamWaitEvent(p.stream, p.ev_color, 0));
-		if (pp.stateful)
+		else if (pp.stateful)
 			queue_chain_setnode(p, pp, P, B, p.stream);
+		if (pp.stateful)
+			queue_chain_nodes(p, pp, P, B, p.stream);
 		if (colors)
 			write_colors(p.stream);
-		a_chain_commit<<<1, kAT, 0, p.stream>>>(P, B.d_lv, B.pm, B.roots, B.acc, B.saved, p.total_buckets);
+		a_chain_commit<<<1, kChainSmall, 0, p.stream>>>(P, B.d_lv, B.pm, B.roots, B.acc, B.saved, p.total_buckets);
 		HD_TRY(hipGetLastError());
 		return HD_OK;
 	} else
@@ -5681,35 +5935,67 @@ static int edit_sequence(Pool &p, u32 root, u32 croot, const std::vector<hd_edit
 	a_set_roots<<<1, 64, 0, p.stream>>>(B.roots, root, croot, B.acc);
 	bool on_device = true;
 	std::vector<PassPlan> todo(plans.rbegin(), plans.rend()); // a stack, first pass on top
-	while (!todo.empty()) {
+	// A chained pass whose counters are on their way: whether it held is asked when the next pass's
+	// top-down is queued, so the host's work on the rest of that pass overlaps it.
+	PassPlan open;
+	hipError_t err = hipSuccess;
+	auto held = [&]() {
+		if (!open.count)
+			return true;
+		err = hipEventSynchronize(p.ev_pass);
+		return err == hipSuccess && !p.h_pass[kPmCut];
+	};
+	// It did not: the edits before the cut run again in one pass, then the others; or all one by one.
+	auto redo = [&]() {
+		a_chain_restore<<<grid_for(p.total_buckets, kAT, 1024), kAT, 0, p.stream>>>(p.bucket_words, B.saved,
+		                                                                           p.total_buckets);
+		std::vector<PassPlan> part;
+		if (p.h_pass[kPmFull])
+			for (u32 k = 0; k < open.count; ++k)
+				chain_split(open.first + k, 1, part);
+		else {
+			const u32 head = std::max(~p.h_pass[kPmCut], 1u);
+			chain_split(open.first, head, part);
+			chain_split(open.first + head, open.count - head, part);
+		}
+		for (auto it = part.rbegin(); it != part.rend(); ++it) {
+			plan_pass(p, flat.data(), *it);
+			todo.push_back(*it);
+		}
+		open = PassPlan{};
+	};
+	while (!todo.empty() || open.count) {
+		// (the top-down of a single pass writes the roots when the root does not proceed)
+		if (todo.empty() || !todo.back().async || !todo.back().chained) {
+			const bool ok = held();
+			HD_TRY(err);
+			if (!ok) {
+				redo();
+				continue;
+			}
+			open = PassPlan{};
+			if (todo.empty())
+				break;
+		}
 		const PassPlan pp = todo.back();
 		todo.pop_back();
 		if (pp.async) {
 			if (!on_device)
 				a_set_roots_keep<<<1, 64, 0, p.stream>>>(B.roots, root, croot);
 			on_device = true;
-			HD_RET(queue_pass(p, pp, B));
-			if (!pp.chained)
+			bool ok = true;
+			HD_RET(queue_pass(p, pp, B, true, [&]() { return ok = held(); }));
+			HD_TRY(err);
+			if (!ok) { // only this pass's top-down has been queued
+				todo.push_back(pp);
+				redo();
 				continue;
-			HD_TRY(hipMemcpyAsync(p.h_pass, B.pm, 4 * kPmHdr, hipMemcpyDeviceToHost, p.stream));
-			HD_TRY(hipStreamSynchronize(p.stream));
-			if (!p.h_pass[kPmCut])
-				continue;
-			// it did not hold: the edits before the cut in one pass, then the others; or one by one
-			a_chain_restore<<<grid_for(p.total_buckets, kAT, 1024), kAT, 0, p.stream>>>(p.bucket_words, B.saved,
-			                                                                           p.total_buckets);
-			std::vector<PassPlan> part;
-			if (p.h_pass[kPmFull])
-				for (u32 k = 0; k < pp.count; ++k)
-					chain_split(pp.first + k, 1, part);
-			else {
-				const u32 head = std::max(~p.h_pass[kPmCut], 1u);
-				chain_split(pp.first, head, part);
-				chain_split(pp.first + head, pp.count - head, part);
 			}
-			for (auto it = part.rbegin(); it != part.rend(); ++it) {
-				plan_pass(p, flat.data(), *it);
-				todo.push_back(*it);
+			open = PassPlan{};
+			if (pp.chained) {
+				HD_TRY(hipMemcpyAsync(p.h_pass, B.pm, 4 * kPmHdr, hipMemcpyDeviceToHost, p.stream));
+				HD_TRY(hipEventRecord(p.ev_pass, p.stream));
+				open = pp;
 			}
 		} else {
 			if (on_device) {

@@ -118,6 +118,7 @@ struct Pool {
 	// levels (joined before the next pass)
 	hipStream_t cstream = nullptr;
 	hipEvent_t ev_top = nullptr, ev_leaf = nullptr, ev_color = nullptr;
+	hipEvent_t ev_pass = nullptr; // a chained pass's counters are in h_pass
 	Scratch scratch;
 	// statistics of the last edit (host)
 	u64 last_entries = 0, last_upserts = 0, last_jobs = 0;

@@ -192,6 +192,8 @@ int hd_pool_create(const hd_config *cfg, hd_pool **out) {
 		return fail(e);
 	if ((e = hipEventCreateWithFlags(&p.ev_color, hipEventDisableTiming)) != hipSuccess)
 		return fail(e);
+	if ((e = hipEventCreateWithFlags(&p.ev_pass, hipEventDisableTiming)) != hipSuccess)
+		return fail(e);
 	if ((e = hipHostMalloc((void **)&p.h_pass, 64, hipHostMallocDefault)) != hipSuccess)
 		return fail(e);
 	if ((e = hipMalloc(&p.words, (words + kWordsPad) * 4)) != hipSuccess)
@@ -241,7 +243,7 @@ int hd_pool_destroy(hd_pool *h) {
 		(void)hipStreamDestroy(p.stream);
 	if (p.cstream)
 		(void)hipStreamDestroy(p.cstream);
-	for (hipEvent_t ev : {p.ev_top, p.ev_leaf, p.ev_color})
+	for (hipEvent_t ev : {p.ev_top, p.ev_leaf, p.ev_color, p.ev_pass})
 		if (ev)
 			(void)hipEventDestroy(ev);
 	delete h;
