@@ -2541,6 +2541,29 @@ __device__ inline uint2 chain_child(const ALevel &C, const GroupTable &G, u32 c)
 	const bool same = pend ? r == kNull && gf : st == pt, fresh = pend && r == kNull && !gf;
 	return make_uint2(!pend ? st : (r != kNull ? r : gr), (fresh ? 1u : 0u) | (same || c >= C.cap ? 2u : 0u));
 }
+// A colored edit's start state of entry e against the one that its top-down took: dif has the slots whose
+// child is null now but was not before the pass, or the other way round. A slot that the edit enters cuts
+// the pass there (what it did below depends on it); one that it covers whole depends on nothing; one that
+// it does not touch takes the edit's color if it is null (VBREditor's rule for empty space, main.cpp:51-53,
+// 117-119) and keeps its state else: corrected here for SetNode, which runs after the node levels.
+__device__ inline void chain_differs(const EditParams &P, u32 l, const ALevel &A, u32 e, u32 pmw, u32 dif,
+                                     u32 *__restrict__ pm) {
+	const u32 k = ldg(&A.ent[e].loff, 0);
+	const DevEditor ed = P.editor(k);
+	const u32 x = ldg(&A.ent[e].x, 0), y = ldg(&A.ent[e].y, 0), z = ldg(&A.ent[e].z, 0);
+	u32 bits = pmw;
+	for (u32 m = dif; m; m &= m - 1u) {
+		const u32 i = (u32)__builtin_ctz(m);
+		const EditType g = ed.geom(l + 1u, child_coord(x, i, 0), child_coord(y, i, 1), child_coord(z, i, 2));
+		if (g == kNotAffected) {
+			bits ^= 1u << (24u + i);
+			if (A.okids)
+				stg(A.okids, 8ull * e + i, cmake(kTagColor, color_to_rgb8(ed.color())));
+		} else if (g == kProceed)
+			chain_cut(pm, k);
+	}
+	stg(A.pmask, e, bits);
+}
 // The join of a chained pass (build_node with versions): a slot that the edit changed takes its result,
 // the others what the latest earlier version left there, or the node as it was before the pass. link(q):
 // {prev, pmask, first_child} of entry q.
@@ -2596,12 +2619,12 @@ __device__ inline Built chain_join(const EditParams &P, u32 l, const ALevel &A, 
 		v = t.x;
 	}
 	if (colored) { // (a slot that the edit covers whole does not depend on what was there)
-		bool bad = false;
+		u32 dif = 0;
 #pragma unroll
 		for (u32 i = 0; i < 8; ++i)
-			bad |= !((q.pmw >> (8u + i)) & 1u) && (st[i] == kNull) != (kv[i] == kNull);
-		if (bad)
-			chain_cut(pm, ldg(&A.ent[e].loff, 0));
+			dif |= (!((q.pmw >> (8u + i)) & 1u) && (st[i] == kNull) != (kv[i] == kNull) ? 1u : 0u) << i;
+		if (dif)
+			chain_differs(P, l, A, e, q.pmw, dif, pm);
 	}
 	if (!own) { // unchanged
 		stg(A.pend, e, 0u);
@@ -2766,12 +2789,12 @@ __global__ void __launch_bounds__(kChainSmall) a_chain_small(EditParams P, const
 				}
 			}
 			if (colored) {
-				bool bad = false;
+				u32 dif = 0;
 #pragma unroll
 				for (u32 i = 0; i < 8; ++i)
-					bad |= !((q.pmw >> (8u + i)) & 1u) && (st[i] == kNull) != (kv[i] == kNull);
-				if (bad)
-					chain_cut(pm, ldg(&A.ent[e].loff, 0));
+					dif |= (!((q.pmw >> (8u + i)) & 1u) && (st[i] == kNull) != (kv[i] == kNull) ? 1u : 0u) << i;
+				if (dif)
+					chain_differs(P, (u32)l, A, e, q.pmw, dif, pm);
 			}
 			u32 nm = 0;
 #pragma unroll
@@ -4758,21 +4781,31 @@ __device__ inline u32 chain_color(const EditParams &P, u32 k) {
 // color state for its own color, or the other way round, than it finds.
 __device__ inline void chain_decide(const EditParams &P, const ChainColor &K, u32 l, u32 e, u32 i, u32 *__restrict__ pm) {
 	const ALevel &A = K.lv[l];
+	// (what does not depend on one another is loaded at once: an entry costs three round trips)
 	const u32 lane = threadIdx.x & 63u, sf = ldg(&A.ent[e].sf, 0), own = ldg(&A.ent[e].octree, 0);
+	const u32 k = ldg(&A.ent[e].loff, 0), m = ldg(A.pmask, e), fc = ldg(A.first_child, e), prev = ldg(A.prev, e);
+	const u32 kid = ldg(A.kids, 8ull * e + i), ok = ldg(A.okids, 8ull * e + i);
 	u32 r = kColorKeep, c = 0;
 	if ((sf & kSfActive) && (sf & kSfFinal))
 		r = own;
 	else if (sf & kSfActive) {
-		const u32 m = ldg(A.pmask, e), kid = ldg(A.kids, 8ull * e + i), k = ldg(&A.ent[e].loff, 0);
-		const u32 was = chain_before(P, K, l, e, i, own);
-		u32 ch = was;
-		if (!chain_slot(P, K, l, e, i, sf, ch))
-			ch = was;
-		if (((m >> i) & 1u) && l + 1u < P.c.color_leaf)
-			c = ldg(K.lv[l + 1u].ccnt, ldg(A.first_child, e) + (u32)__builtin_popcount(m & 0xFFu & ((1u << i) - 1u)));
-		const u32 mine = chain_color(P, k);
-		if (kid != kNull && !((m >> (8u + i)) & 1u) && (was == mine) != (color_child(P.cnodes, own, i) == mine) &&
-		    mine != kColorNull)
+		const bool jobs = l + 1u == P.c.color_leaf, pr = (m >> i) & 1u;
+		const u32 ci = fc + (u32)__builtin_popcount(m & 0xFFu & ((1u << i) - 1u));
+		const u32 mine = chain_color(P, k), before = color_child(P.cnodes, own, i);
+		u32 ch = ok;
+		bool set = ((m >> (24u + i)) & 1u) != 0u;
+		if (pr && jobs) {
+			ch = chain_job_state(P, K, ci);
+			set = true;
+		} else if (pr) {
+			const u32 cr = ldg(K.lv[l + 1u].ores, ci);
+			c = ldg(K.lv[l + 1u].ccnt, ci);
+			ch = cr == kColorNewNode ? cmake(kTagNode, K.node_cap + ci) : cr;
+			set = cr != kColorKeep;
+		}
+		const u32 was = prev == kNull ? before : chain_before(P, K, l, e, i, own);
+		ch = set ? ch : was;
+		if (kid != kNull && !((m >> (8u + i)) & 1u) && (was == mine) != (before == mine) && mine != kColorNull)
 			chain_cut(pm, k);
 #pragma unroll
 		for (u32 d = 1; d < 8; d <<= 1)
@@ -5819,8 +5852,7 @@ static int queue_pass(Pool &p, const PassPlan &pp, AsyncBufs &B, bool reserve = 
 		a_scan_app<<<grid_for(pp.cap[leafL], kScanTile, 1024), kScanThreads, 0, p.cstream>>>(leafL, B.pm, B.app,
 		                                                                                    B.appo, B.tsum);
 		a_scan_fix<<<grid_for(pp.cap[leafL], 256 * 8, 1024), 256, 0, p.cstream>>>(leafL, B.pm, B.appo, B.tsum);
-		if (pp.chained) { // decided beside the node levels, written once the pass is known to hold
-			queue_chain_setnode(p, pp, P, B, p.cstream);
+		if (pp.chained) { // written once the pass is known to hold
 			HD_TRY(hipEventRecord(p.ev_color, p.cstream));
 			return HD_OK;
 		}
@@ -5857,10 +5889,10 @@ static int queue_pass(Pool &p, const PassPlan &pp, AsyncBufs &B, bool reserve = 
 		a_chain_end<<<1, kChainEdits, 0, p.stream>>>(P, B.d_lv, B.pm, B.G, B.roots, B.saved, p.total_buckets);
 		if (colors)
 			HD_TRY(hipStreamWaitEvent(p.stream, p.ev_color, 0));
-		else if (pp.stateful)
+		if (pp.stateful) { // (its decisions need to know which nodes the edits found empty)
 			queue_chain_setnode(p, pp, P, B, p.stream);
-		if (pp.stateful)
 			queue_chain_nodes(p, pp, P, B, p.stream);
+		}
 		if (colors)
 			write_colors(p.stream);
 		a_chain_commit<<<1, kChainSmall, 0, p.stream>>>(P, B.d_lv, B.pm, B.roots, B.acc, B.saved, p.total_buckets);
@@ -6048,30 +6080,54 @@ static bool chains(const Pool &p, const hd_edit_desc &d) {
 		return false;
 	return !is_stateful(d) || (d.color.has_value && !d.color.bits_per_weight && lds_jobs(p.dc) && p.dc.color_leaf > 0);
 }
-// Whether two edits may reach the same node of size S or below: its cube would meet both shapes, so
-// their S-aligned bounds meet and their distance is at most the cube's diagonal.
+// Whether an edit reaches the node of size S at lo: sphere_node / aabb_node do not rule it out.
+static bool reaches(const hd_edit_desc &d, const i64 (&lo)[3], i64 S) {
+	u64 n2 = 0;
+	for (int i = 0; i < 3; ++i) {
+		if (d.kind <= HD_EDIT_SPHERE_PAINT) {
+			const i64 a = lo[i] - (i64)d.p0[i], b = lo[i] + S - (i64)d.p0[i];
+			n2 += a > 0 ? (u64)(a * a) : b < 0 ? (u64)(b * b) : 0u;
+		} else if (lo[i] + S <= (i64)d.p0[i] || lo[i] >= (i64)d.p1[i])
+			return false;
+	}
+	return d.kind > HD_EDIT_SPHERE_PAINT || n2 <= d.r2;
+}
+// Whether two edits may reach the same node of size S (so also whether they may share a smaller one): the
+// nodes that meet both shapes' bounds are tried one by one, when they are few. Shapes further apart than a
+// node's diagonal share none.
 static bool may_share_nodes(const hd_edit_desc &a, const hd_edit_desc &b, i64 S) {
 	auto ball = [](const hd_edit_desc &d) { return d.kind <= HD_EDIT_SPHERE_PAINT; };
-	auto radius = [](const hd_edit_desc &d) { return std::sqrt((double)d.r2) + 1.0; };
+	auto radius = [&](const hd_edit_desc &d) { return ball(d) ? std::sqrt((double)d.r2) + 1.0 : 0.0; };
+	i64 n0[3], n1[3]; // the nodes whose closed cubes meet both bounds
 	double d2 = 0;
 	for (int i = 0; i < 3; ++i) {
 		double lo[2], hi[2]; // the shapes' closed bounds, spheres as their centre
-		i64 c0[2], c1[2];    // the nodes whose closed cubes meet them
+		n0[i] = 0, n1[i] = INT64_MAX;
 		for (int k = 0; k < 2; ++k) {
 			const hd_edit_desc &d = k ? b : a;
 			lo[k] = (double)d.p0[i];
 			hi[k] = ball(d) ? lo[k] : std::max(lo[k], (double)d.p1[i]);
-			const double r = ball(d) ? radius(d) : 0.0;
-			c0[k] = (i64)std::floor((lo[k] - r) / (double)S) - 1;
-			c1[k] = (i64)std::floor((hi[k] + r) / (double)S);
+			n0[i] = std::max(n0[i], (i64)std::floor((lo[k] - radius(d)) / (double)S) - 1);
+			n1[i] = std::min(n1[i], (i64)std::floor((hi[k] + radius(d)) / (double)S));
 		}
-		if (c1[0] < c0[1] || c1[1] < c0[0])
+		if (n1[i] < n0[i])
 			return false;
 		const double g = std::max(0.0, std::max(lo[0] - hi[1], lo[1] - hi[0]));
 		d2 += g * g;
 	}
-	const double reach = (ball(a) ? radius(a) : 0.0) + (ball(b) ? radius(b) : 0.0) + (double)S * std::sqrt(3.0) + 1.0;
-	return d2 <= reach * reach;
+	const double reach = radius(a) + radius(b) + (double)S * std::sqrt(3.0) + 1.0;
+	if (d2 > reach * reach)
+		return false;
+	if ((double)(n1[0] - n0[0] + 1) * (double)(n1[1] - n0[1] + 1) * (double)(n1[2] - n0[2] + 1) > 8192.0)
+		return true;
+	for (i64 z = n0[2]; z <= n1[2]; ++z)
+		for (i64 y = n0[1]; y <= n1[1]; ++y)
+			for (i64 x = n0[0]; x <= n1[0]; ++x) {
+				const i64 lo[3] = {x * S, y * S, z * S};
+				if (reaches(a, lo, S) && reaches(b, lo, S))
+					return true;
+			}
+	return false;
 }
 // The passes of a plain call: runs of consecutive edits of which no two may reach the same leaf (with
 // colors: the same color leaf), each run one chained pass; the others one by one.
