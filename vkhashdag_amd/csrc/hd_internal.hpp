@@ -111,6 +111,7 @@ struct Pool {
 	u32 *cnodes = nullptr, *cleaves = nullptr; // color octree nodes (8 u32 each) and VBR leaf words
 	u64 cnode_cap = 0, cleaf_cap = 0;
 	u32 *hm_mn = nullptr, *hm_mx = nullptr;
+	u64 hm_total = 0; // heights in each of them
 	DevHeightmap hm{};
 	DevHeightmap *d_hm = nullptr; // device copy of hm (editors read it through a pointer)
 	hipStream_t stream = nullptr;
