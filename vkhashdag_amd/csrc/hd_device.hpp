@@ -302,6 +302,40 @@ struct DevEditor {
 			return aabb_voxel(x, y, z);
 		return column_voxel(x, y, z);
 	}
+	// in_range of the 2 x 2 voxels (x + i, y + j, z), bit i + 2 j (x, y even)
+	__device__ u32 in_range4(u32 x, u32 y, u32 z) const {
+		if (is_sphere()) { // |a - b| < 2^32, and sphere_voxel's sums are taken modulo 2^64 too
+			const u32 c0 = d.p0[0], c1 = d.p0[1], c2 = d.p0[2];
+			const u32 dx0 = x > c0 ? x - c0 : c0 - x, dx1 = x + 1u > c0 ? x + 1u - c0 : c0 - x - 1u;
+			const u32 dy0 = y > c1 ? y - c1 : c1 - y, dy1 = y + 1u > c1 ? y + 1u - c1 : c1 - y - 1u;
+			const u32 dz = z > c2 ? z - c2 : c2 - z;
+			const u64 zz = (u64)dz * dz, y0 = (u64)dy0 * dy0 + zz, y1 = (u64)dy1 * dy1 + zz;
+			const u64 x0 = (u64)dx0 * dx0, x1 = (u64)dx1 * dx1;
+			return (x0 + y0 <= d.r2 ? 1u : 0u) | (x1 + y0 <= d.r2 ? 2u : 0u) | (x0 + y1 <= d.r2 ? 4u : 0u) |
+			       (x1 + y1 <= d.r2 ? 8u : 0u);
+		}
+		u32 m = (x >= d.p0[0] && x < d.p1[0] ? 5u : 0u) | (x + 1u >= d.p0[0] && x + 1u < d.p1[0] ? 10u : 0u);
+		m &= (y >= d.p0[1] && y < d.p1[1] ? 3u : 0u) | (y + 1u >= d.p0[1] && y + 1u < d.p1[1] ? 12u : 0u);
+		if (is_box())
+			return z >= d.p0[2] && z < d.p1[2] ? m : 0u;
+		if (!m)
+			return 0u;
+		return m & ((z < hm->h(x, y) ? 1u : 0u) | (z < hm->h(x + 1u, y) ? 2u : 0u) | (z < hm->h(x, y + 1u) ? 4u : 0u) |
+		            (z < hm->h(x + 1u, y + 1u) ? 8u : 0u));
+	}
+	// edit_voxel / edit_voxel_vbr_asg of those four, v their occupancy: the new one; asg |= the voxels
+	// the edit assigns its color.
+	__device__ u32 edit_voxel4(u32 x, u32 y, u32 z, u32 v, u32 &asg) const {
+		if (!stateful()) {
+			if (is_paint())
+				return v;
+			const u32 in = in_range4(x, y, z);
+			return is_dig() ? v & ~in : v | in;
+		}
+		const u32 in = in_range4(x, y, z);
+		asg = in | (~v & 15u);
+		return is_paint() ? v : v | in;
+	}
 	// StatelessEditorWrapper path (Editor.hpp:42-55)
 	__device__ EditType edit_node(u32 level, u32 x, u32 y, u32 z) const {
 		EditType t = geom(level, x, y, z);
