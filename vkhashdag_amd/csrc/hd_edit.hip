@@ -3258,112 +3258,100 @@ __global__ void a_job_ranges(const ALevel *__restrict__ lv, const u32 *__restric
 	}
 }
 
-// LDS color jobs: one workgroup per writer job rebuilds the job's colors in LDS (job_rebuild) and
-// encodes them (a_job_encode, a_job_rest). Every load of a phase is independent of the others in
-// it: a rebuild costs about three memory round trips.
-constexpr u32 kJobHdr = 3072; // staged header words (larger chunks are decoded voxel by voxel); also the
+// Color jobs of at most kJobV voxels: one workgroup per writer job rebuilds the job's colors, each thread the
+// kSeg consecutive voxels of its segment in registers (job_rebuild), and encodes them (a_job_encode,
+// a_job_rest). Every load of a phase is independent of the others in it.
+// A segment lies inside one 4^3 leaf (64 voxels in Morton order), so its colors are one push, one fill or a
+// few runs of the old chunk, and then what one leaf's edits assigned. With the colors voxel by voxel in LDS
+// (24 KB of writes, coverage bits and strided reads a job) four jobs fitted a CU; now six do.
+// (868k jobs of 4096 mixed edits 10.2 -> 3.9 ms; the jobs of about 27 chained edits 189 -> 74 us.)
+constexpr u32 kJobHdr = 3072; // staged header words (larger chunks are decoded from memory); also the
                               // largest encoded chunk staged here (larger ones go to a_job_rest)
-// A voxel's VBRColor in LDS: colors, and weight | bits_per_weight << 8 | has_value << 15 in 16 bits
-// (hd_edit accepts bits_per_weight <= 3), so that four jobs fit a CU's LDS.
-__device__ inline u32 pack_wb16(u32 wb) { return (wb & 0xFFu) | (((wb >> 8) & 0x7Fu) << 8) | (((wb >> 16) & 1u) << 15); }
-__device__ inline u32 unpack_wb16(u32 w) { return (w & 0xFFu) | (((w >> 8) & 0x7Fu) << 8) | ((w >> 15) << 16); }
+constexpr u32 kSeg = kJobV / kEncThreads, kSegLeaf = 64u / kSeg;
+static_assert(kSeg == 16 && kSegLeaf * kSeg == 64, "a segment's records are two 16-byte loads inside one leaf");
+// A voxel's VBRColor weight word in 16 bits: weight | bits_per_weight << 8 (hd_edit accepts bits_per_weight
+// <= 3; whether the voxel has a value is not encoded).
+__device__ inline u32 pack_wb16(u32 wb) { return (wb & 0xFFu) | (((wb >> 8) & 0x7Fu) << 8); }
 static_assert(kJobHdr <= kEncTmp, "a staged chunk fits its kEncTmp-word slot");
 static_assert(kJobHdr % kEncThreads == 0 && kEncThreads >= 72, "staged words split evenly; one push per thread");
 struct JobLds {
-	u32 colc[kJobV];
-	unsigned short colw[kJobV];
 	union {
 		u32 hdr[kJobHdr];
 		u32 stmp[kJobHdr];
 	};
-	union { // the rebuild's records (dead once the encode starts) / the encode's wave totals
-		struct {
-			u32 cov[kJobV / 32];
-			uint4 fill[kJobV / 64 + 8]; // pushes: {voxel offset, colors, wb, voxel count}
-			u32 nfill;
-			u32 lbase[kJobV / 64];      // per leaf of the job: its first voxel, or kNull without assigned colors
-		};
-		EncScan sh[kEncThreads / 64];
-	};
+	// pushes on the job's children (8) and grandchildren (64, at 8): {colors, wb | 1 << 31}, 0 where none
+	uint2 push[8 + kJobV / 64];
+	u32 leaf[kJobV / 64]; // per 64 voxels: the job's leaf with assigned colors, or kNull
+	uint2 last[kEncThreads]; // each segment's last color
+	unsigned short colw[kJobV];
+	EncScan sh[kEncThreads / 64];
 };
-__device__ inline void job_set(JobLds &S, u32 v, Color c) {
-	S.colc[v] = c.colors;
-	S.colw[v] = (unsigned short)pack_wb16(c.wb);
+__device__ inline u32 opaque(u32 x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+	asm volatile("" : "+v"(x));
+#endif
+	return x;
 }
-// enc_load over the job's LDS colors.
-// A thread's voxels of a job (v0 .. v0 + n - 1): which start a header, and the totals for the
-// block scan. The colors stay in LDS; the writers read them again.
-struct JobEnc {
-	u32 v0, n, heads;
+// A thread's segment: its voxels' colors, which start a header, and the totals for the block scan. The weight
+// words of a weighted segment (few colors have weights) lie in LDS: the thread's own kSeg of them.
+struct JobSeg {
+	u32 v0, c[kSeg], heads;
 	EncScan x;
-};
-// kFull: V == kJobV, so every thread holds exactly kEncPer voxels.
-template <bool kFull> __device__ inline void enc_scan_job(const JobLds &S, u32 V, JobEnc &R) {
-	const u32 per = kFull ? kEncPer : (V + kEncThreads - 1) / kEncThreads;
-	R.v0 = threadIdx.x * per;
-	const u32 v1 = kFull ? R.v0 + kEncPer : min(V, R.v0 + per);
-	R.n = R.v0 < v1 ? v1 - R.v0 : 0u;
-	u32 pc = 0, pb = 0;
-	if (R.n && R.v0)
-		pc = S.colc[R.v0 - 1], pb = (S.colw[R.v0 - 1] >> 8) & 0x7Fu;
-	R.heads = 0;
-	R.x = EncScan{0, 0};
-	auto step = [&](u32 k, u32 c, u32 w16) {
-		const u32 v = R.v0 + k, b = (w16 >> 8) & 0x7Fu;
-		if (v == 0 || (v & 0x3FFFu) == 0 || c != pc || b != pb)
-			R.heads |= 1u << k;
-		R.x.bits += b;
-		pc = c;
-		pb = b;
-	};
-	if (kFull || R.n == kEncPer) {
-		const uint4 *qc = reinterpret_cast<const uint4 *>(S.colc + R.v0);
-		const uint4 *qw = reinterpret_cast<const uint4 *>(S.colw + R.v0);
-#pragma unroll
-		for (u32 q = 0; q < kEncPer / 8; ++q) { // 8 voxels a step: their colors and weight words
-			const uint4 c0 = qc[2 * q], c1 = qc[2 * q + 1], w = qw[q];
-			const u32 cs[8] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z, c1.w}, ws[4] = {w.x, w.y, w.z, w.w};
-#pragma unroll
-			for (u32 j = 0; j < 8; ++j)
-				step(8 * q + j, cs[j], (ws[j >> 1] >> (16 * (j & 1))) & 0xFFFFu);
-		}
-	} else {
-#pragma unroll
-		for (u32 k = 0; k < kEncPer; ++k)
-			if (k < R.n)
-				step(k, S.colc[R.v0 + k], S.colw[R.v0 + k]);
+	bool weighted; // some weight word is not 0
+	unsigned short *w;
+	__device__ u32 wb(u32 k) const { return weighted ? w[k] : 0u; }
+	__device__ void set_weights(u32 m, u32 wb16) { // of the voxels of mask m
+		if (wb16 == 0u && !weighted)
+			return;
+#pragma unroll 1
+		for (u32 k = 0; k < kSeg; ++k)
+			w[k] = (m >> k) & 1u ? (unsigned short)wb16 : (weighted ? w[k] : (unsigned short)0u);
+		weighted = true;
 	}
-	R.x.heads = (u32)__builtin_popcount(R.heads);
-}
-// Rebuilds job e's colors in S (every thread of the block calls it): the colors pushed onto its
-// terminal subtrees (pev records of the pairs whose pmask push bit is set) and the colors its leaves'
-// edits assigned (lcol / lmask) are written first and marked covered (pushes cover terminal
-// subtrees, leaves proceeding ones: disjoint); the job's current colors (DAGColorPool's leaf decode,
-// headers staged in LDS) fill the rest. Returns with S complete and visible to the block; E and jh
-// are the job's entry and the header of its current chunk.
+	__device__ void set(u32 m, u32 colors, u32 wb16) {
+#pragma unroll
+		for (u32 k = 0; k < kSeg; ++k)
+			c[k] = (m >> k) & 1u ? colors : c[k];
+		set_weights(m, wb16);
+	}
+	__device__ void fill(u32 colors, u32 wb16) {
+#pragma unroll
+		for (u32 k = 0; k < kSeg; ++k)
+			c[k] = colors;
+		weighted = false;
+		set_weights((1u << kSeg) - 1u, wb16);
+	}
+};
+// Rebuilds job e's colors into R (every thread of the block calls it): the job's current colors (DAGColorPool's
+// leaf decode, headers staged in LDS), over them the colors pushed onto its terminal subtrees (pev records of
+// the pairs whose pmask push bit is set) and over those the colors its leaves' edits assigned (lidx; outside
+// a folded pass the three are disjoint: pushes cover terminal subtrees, leaves proceeding ones. A folded
+// pass can push a color on a proceeding child, the edit that reset it, and again on its children or assign
+// leaf colors inside it). Then the segment's headers. E and jh are the job's entry and the header of its
+// current chunk; S.hdr is free when it returns.
 __device__ inline void job_rebuild(const EditParams &P, const ALevel *__restrict__ lv, const uint4 *__restrict__ jrange,
                                    const unsigned short *__restrict__ lidx, const uint2 *__restrict__ ecol, u32 V, u32 e,
-                                   JobLds &S, Entry &E, uint4 &jh) {
+                                   JobLds &S, Entry &E, uint4 &jh, JobSeg &R) {
 	const u32 leafL = P.c.color_leaf, L = P.c.L, vl = P.c.voxel_level;
 	const u32 *cleaves = P.cleaves;
 	const Entry *ent = lv[leafL].ent;
 	const u32 below = L - 1u - leafL; // node levels from the job down to the leaves (0, 1 or 2)
+	// (opaque, so that what is derived from it is not kept in registers over the job loop)
+	const u32 t0 = opaque(threadIdx.x);
 	__syncthreads(); // the previous job's readers are done with S
-	for (u32 w = threadIdx.x; w < V / 32u; w += kEncThreads)
-		S.cov[w] = 0u;
-	if (threadIdx.x == 0)
-		S.nfill = 0;
-	E = ent[e];
-	const uint4 jr = jrange[2ull * e];
-	jh = jrange[2ull * e + 1u];
+	if (t0 < 8u + kJobV / 64)
+		S.push[t0] = make_uint2(0u, 0u);
+	if (t0 < kJobV / 64)
+		S.leaf[t0] = kNull;
+	E = ldg(ent, e);
+	const uint4 jr = ldg(jrange, 2ull * e);
+	jh = ldg(jrange, 2ull * e + 1u);
 	__syncthreads();
 	const bool chunk = ctag(E.octree) == kTagLeaf;
 	const u32 idx = cdata(E.octree), M = jh.x, B0 = jh.y, W0 = jh.w;
-	// pushes (the job's own 8 pairs, then the pairs of its entries one level down: at most 72),
-	// the leaves' records, the chunk's headers and its weight words when they fit beside them (at
-	// most 384 words for 4096 voxels of <= 3 bits) and the leaves' colors: every load is issued
-	// before the first LDS store, so they share one round trip
-	const u32 t0 = threadIdx.x;
+	// pushes (the job's own 8 pairs, then the pairs of its entries one level down: at most 72), the leaves
+	// and the chunk's headers and its weight words when they fit beside them (at most 384 words for 4096
+	// voxels of <= 3 bits): every load is issued before the first LDS store, so they share one round trip
 	const u32 np0 = below ? 8u : 0u, np1 = below > 1u ? 8u * (jr.y - jr.x) : 0u;
 	u32 pmw = 0, pl = leafL;
 	uint4 q = make_uint4(0, 0, 0, 0);
@@ -3393,134 +3381,152 @@ __device__ inline void job_rebuild(const EditParams &P, const ALevel *__restrict
 #pragma unroll
 	for (u32 r = 0; r < kHdrPer; ++r) {
 		const u32 k = t0 + r * kEncThreads;
-		if (k < nk)
-			hw[r] = cleaves[idx + 4u + k];
+		if (r * kEncThreads < nk && k < nk)
+			hw[r] = ldg(cleaves, (u64)idx + 4u + k);
 	}
-	constexpr u32 kPer = kJobV / kEncThreads;
-	// which edit assigned each leaf voxel's color last: a thread's r-th voxel lies in leaf
-	// wave + 4 r (wave-uniform)
-	const u32 wv = __builtin_amdgcn_readfirstlane(t0 >> 6);
-	u32 ix[kPer];
-#pragma unroll
-	for (u32 r = 0; r < kPer; ++r)
-		ix[r] = wv + r * (kEncThreads / 64u) < nl ? (u32)ldg(lidx, 64ull * llo + t0 + r * kEncThreads) : kNoEdit;
-	if (t0 < np0 + np1 && ((pmw >> (16u + (t0 & 7u))) & 1u))
-		S.fill[atomicAdd(&S.nfill, 1u)] = make_uint4(q.x, q.y, q.z, 1u << (3u * (vl - (pl + 1u))));
-	if (t0 < nl) {
+	if (t0 < np0 + np1 && ((pmw >> (16u + (t0 & 7u))) & 1u)) {
+		const u32 sh = 3u * (vl - (pl + 1u)); // 64 or 512 voxels
+		S.push[sh == 6u ? 8u + (q.x >> 6) : q.x >> 9] = make_uint2(q.y, q.z | 1u << 31);
+	}
+	if (t0 < nl && leaf_writes_colors(P, lv, LE)) {
 		const u32 m2 = (1u << P.leaf_bits >> 2) - 1u;
-		// a leaf's lane is the Morton index of its voxel inside the 4^3 leaf
-		S.lbase[t0] = leaf_writes_colors(P, lv, LE) ? morton3(LE.x & m2, LE.y & m2, LE.z & m2) << 6 : kNull;
+		S.leaf[morton3(LE.x & m2, LE.y & m2, LE.z & m2)] = t0;
 	}
 #pragma unroll
 	for (u32 r = 0; r < kHdrPer; ++r) {
 		const u32 k = t0 + r * kEncThreads;
-		if (k < nk)
+		if (r * kEncThreads < nk && k < nk)
 			S.hdr[k] = hw[r];
 	}
 	__syncthreads();
-	// the assigning edits' colors from the pass's table (their loads overlap the pushes below)
-	uint2 ac[kPer];
-#pragma unroll
-	for (u32 r = 0; r < kPer; ++r) {
-		const u32 li = wv + r * (kEncThreads / 64u);
-		ac[r] = make_uint2(0u, 0u);
-		if (ix[r] != kNoEdit && li < nl && S.lbase[li] != kNull)
-			ac[r] = ldg(ecol, ix[r]);
-	}
-	// the pushed and assigned colors, marked covered. A folded pass can push a color on a proceeding
-	// child (the edit that reset it) and again on its children or assign leaf colors inside it: the
-	// larger pushes go first, the leaves last.
-	const u32 big = 1u << (3u * (vl - (leafL + 1u)));
-	for (u32 pass = 0; pass < 2; ++pass) {
-		for (u32 f = 0; f < S.nfill; ++f) {
-			const uint4 q = S.fill[f];
-			if ((q.w >= big) != (pass == 0))
-				continue;
-			for (u32 v = threadIdx.x; v < q.w; v += kEncThreads)
-				job_set(S, q.x + v, Color{q.y, q.z});
-			if (q.w >= 32u)
-				for (u32 w = (q.x >> 5) + threadIdx.x; w < (q.x + q.w) >> 5; w += kEncThreads)
-					S.cov[w] = 0xFFFFFFFFu;
-			else if (threadIdx.x == 0)
-				atomicOr(&S.cov[q.x >> 5], ((1u << q.w) - 1u) << (q.x & 31u));
+	R.v0 = t0 * kSeg;
+	R.w = S.colw + R.v0;
+	R.heads = 0;
+	R.x = EncScan{0, 0};
+	const bool on = R.v0 < V;
+	if (on) {
+		// which edit assigned each voxel's color last: 16 indices, in flight during the decode
+		const u32 li = S.leaf[t0 / kSegLeaf];
+		uint4 ia = make_uint4(~0u, ~0u, ~0u, ~0u), ib = ia;
+		if (li != kNull) {
+			const uint4 *src = reinterpret_cast<const uint4 *>(lidx) + 8ull * (llo + li) + 2u * (t0 % kSegLeaf);
+			ia = ldg(src, 0);
+			ib = ldg(src, 1);
 		}
-		if (P.folded)
-			__syncthreads();
-	}
-#pragma unroll
-	for (u32 r = 0; r < kPer; ++r) {
-		const u32 li = wv + r * (kEncThreads / 64u), lane = t0 & 63u;
-		if (ix[r] != kNoEdit && li < nl && S.lbase[li] != kNull) {
-			const u32 at = S.lbase[li] | lane;
-			Color c{ac[r].x, ac[r].y};
-			if (ac[r].y >> 24) { // a column fill: the voxel's absolute position from its Morton index in the job
-				const u32 bits = P.leaf_bits;
-				const u32 vx = (E.x << bits) | morton_compact(at), vy = (E.y << bits) | morton_compact(at >> 1),
-				          vz = (E.z << bits) | morton_compact(at >> 2);
-				c = Color::rgb8(P.editor(ix[r]).column_rgb8(vx, vy, vz));
-			}
-			job_set(S, at, c);
-			atomicOr(&S.cov[at >> 5], 1u << (at & 31u));
-		}
-	}
-	__syncthreads();
-	// the current colors of the voxels not covered above
-	if (!chunk || M == 0u || B0 == 0u) {
-		const Color fill = chunk ? Color::none() : get_fill(E.octree);
-		for (u32 v = threadIdx.x; v < V; v += kEncThreads)
-			if (!((S.cov[v >> 5] >> (v & 31u)) & 1u))
-				job_set(S, v, fill);
-	} else if (!staged_hdr) {
-		for (u32 v = threadIdx.x; v < V; v += kEncThreads)
-			if (!((S.cov[v >> 5] >> (v & 31u)) & 1u))
-				job_set(S, v, chunk_voxel(cleaves, idx, v));
-	} else {
-		const u32 *mac = S.hdr, *hd = S.hdr + 2u * M, wo = idx + 4u + 2u * M + 2u * B0;
-		for (u32 v0 = threadIdx.x * kDenseRun; v0 < V; v0 += kEncThreads * kDenseRun) {
+		uint2 ps = S.push[8u + t0 / kSegLeaf];
+		if (!(ps.y >> 31))
+			ps = S.push[t0 / (8u * kSegLeaf)];
+		if (ps.y >> 31)
+			R.fill(ps.x, pack_wb16(ps.y));
+		else if (!chunk || M == 0u || B0 == 0u)
+			R.fill(chunk ? 0u : get_fill(E.octree).colors, 0u);
+		else {
 			// V <= 4096 < 2^14: one macro block; the last header with voxoff <= v0, then forward
-			const u32 ws = mac[1];
-			u32 lo = mac[0], cnt = (M > 1u ? mac[2] : B0) - lo;
-			const u32 lb = lo + cnt;
-			const u32 fb = lo;
+			const u64 at = (u64)idx + 4u;
+			auto H = [&](u32 i) { return staged_hdr ? S.hdr[i] : ldg(cleaves, at + i); };
+			const u32 ho = 2u * M, wo = 2u * (M + B0), ws = H(1), fb = H(0), lb = M > 1u ? H(2) : B0;
+			u32 lo = fb, cnt = lb - fb;
 			while (cnt > 0) {
 				const u32 step = cnt >> 1;
-				if ((hd[2u * (lo + step) + 1u] >> 18) <= v0)
+				if ((H(ho + 2u * (lo + step) + 1u) >> 18) <= R.v0)
 					lo += step + 1u, cnt -= step + 1u;
 				else
 					cnt = step;
 			}
-			u32 h = lo > fb ? lo - 1u : fb;
-			for (u32 k = 0; k < kDenseRun && v0 + k < V; ++k) {
-				const u32 v = v0 + k;
-				while (h + 1u < lb && (hd[2u * (h + 1u) + 1u] >> 18) <= v)
-					++h;
-				if ((S.cov[v >> 5] >> (v & 31u)) & 1u)
-					continue;
-				Color c;
-				const u32 hc = hd[2u * h], hp = hd[2u * h + 1u], bpw = (hp >> 16) & 3u;
-				if (bpw == 0)
-					c = Color{hc, 1u << 16};
-				else {
-					const u32 bit = ws + (hp & 0xFFFFu) + (v - (hp >> 18)) * bpw, o = bit & 31u;
-					u32 w, w1 = 0u;
-					if (staged_w) {
-						w = S.hdr[2u * (M + B0) + (bit >> 5)];
+			u32 h = lo > fb ? lo - 1u : fb, hp = H(ho + 2u * h + 1u);
+			R.fill(0u, 0u);
+			for (u32 from = 0;;) { // header h's run starts at the segment's voxel `from`
+				const u32 hc = H(ho + 2u * h), hn = h + 1u < lb ? H(ho + 2u * h + 3u) : ~0u;
+				const u32 bpw = (hp >> 16) & 3u;
+#pragma unroll
+				for (u32 k = 0; k < kSeg; ++k)
+					R.c[k] = k >= from ? hc : R.c[k];
+				if (bpw || R.weighted) {
+					R.set_weights(((1u << kSeg) - 1u) & ~((1u << from) - 1u), bpw << 8);
+					const u32 to = hn == ~0u ? kSeg : min((hn >> 18) - R.v0, kSeg);
+#pragma unroll 1
+					for (u32 k = from; bpw && k < to; ++k) {
+						const u32 bit = ws + (hp & 0xFFFFu) + (R.v0 + k - (hp >> 18)) * bpw, o = bit & 31u, i = wo + (bit >> 5);
+						u32 w = (staged_w ? S.hdr[i] : ldg(cleaves, at + i)) >> o;
 						if (o + bpw > 32u)
-							w1 = S.hdr[2u * (M + B0) + (bit >> 5) + 1u];
-					} else {
-						w = cleaves[wo + (bit >> 5)];
-						if (o + bpw > 32u)
-							w1 = cleaves[wo + (bit >> 5) + 1u];
+							w |= (staged_w ? S.hdr[i + 1u] : ldg(cleaves, at + i + 1u)) << (32u - o);
+						R.w[k] = (unsigned short)((w & ((1u << bpw) - 1u)) | (bpw << 8));
 					}
-					w = (w >> o) | (o + bpw > 32u ? w1 << (32u - o) : 0u);
-					w &= (1u << bpw) - 1u;
-					c = Color{hc, w | (bpw << 8) | (1u << 16)};
 				}
-				job_set(S, v, c);
+				if (hn == ~0u || (hn >> 18) >= R.v0 + kSeg)
+					break;
+				from = max(hn >> 18, R.v0) - R.v0;
+				hp = hn;
+				++h;
 			}
 		}
-	}
+		// the assigned colors from the pass's table, one edit of the segment's at a time (mostly there is one)
+		const u32 ix[kSeg / 2] = {ia.x, ia.y, ia.z, ia.w, ib.x, ib.y, ib.z, ib.w};
+		auto id = [&](u32 k) { return (ix[k >> 1] >> (16u * (k & 1u))) & 0xFFFFu; };
+		u32 todo = 0;
+#pragma unroll
+		for (u32 k = 0; k < kSeg; ++k)
+			todo |= id(k) != kNoEdit ? 1u << k : 0u;
+		while (todo) {
+			u32 f = 0, sel = 0;
+#pragma unroll
+			for (u32 k = kSeg; k-- > 0;)
+				f = (todo >> k) & 1u ? id(k) : f;
+			const uint2 ec = ldg(ecol, f);
+#pragma unroll
+			for (u32 k = 0; k < kSeg; ++k)
+				sel |= id(k) == f ? 1u << k : 0u;
+			todo &= ~sel;
+			u32 cc = ec.x, cw = pack_wb16(ec.y);
+			if (ec.y >> 24) { // a column fill (one color per 4^3 block): the segment's position in the world
+				const u32 bits = P.leaf_bits;
+				cc = P.editor(f).column_rgb8((E.x << bits) | morton_compact(R.v0), (E.y << bits) | morton_compact(R.v0 >> 1),
+				                             (E.z << bits) | morton_compact(R.v0 >> 2));
+				cw = 0;
+			}
+			R.set(sel, cc, cw);
+		}
+		S.last[t0] = make_uint2(R.c[kSeg - 1], R.wb(kSeg - 1) >> 8);
+	} else
+		R.fill(0u, 0u); // no voxels: no headers and no weights
 	__syncthreads();
+	if (on) {
+		const uint2 before = S.last[t0 ? t0 - 1u : 0u];
+		R.heads = R.c[0] != before.x || R.wb(0) >> 8 != before.y ? 1u : 0u;
+#pragma unroll
+		for (u32 k = 1; k < kSeg; ++k)
+			R.heads |= R.c[k] != R.c[k - 1] ? 1u << k : 0u;
+		if (R.weighted)
+#pragma unroll 1
+			for (u32 k = 0, b = R.wb(0) >> 8; k < kSeg; ++k) {
+				const u32 bk = R.wb(k) >> 8;
+				R.heads |= bk != b ? 1u << k : 0u;
+				R.x.bits += bk;
+				b = bk;
+			}
+		R.heads |= t0 ? 0u : 1u; // (no other voxel starts a macro block)
+	}
+	R.x.heads = (u32)__builtin_popcount(R.heads);
+}
+// The segment's headers and weights into the chunk at out (word 6: its headers, then W weight words, zeroed);
+// run: the headers and weight bits before it.
+template <class Out, class Or> __device__ inline void job_write(const JobSeg &R, EncScan run, u32 wo, Out out, Or out_or) {
+#pragma unroll
+	for (u32 k = 0; k < kSeg; ++k) {
+		const u32 wb = R.wb(k), bpw = wb >> 8;
+		if ((R.heads >> k) & 1u) {
+			out(6u + 2u * run.heads, R.c[k]);
+			out(7u + 2u * run.heads, ((R.v0 + k) << 18) | (bpw << 16) | run.bits);
+			run.heads += 1u;
+		}
+		if (bpw) {
+			const u32 w = wb & ((1u << bpw) - 1u), o = run.bits & 31u;
+			out_or(wo + (run.bits >> 5), w << o);
+			if (o + bpw > 32u)
+				out_or(wo + (run.bits >> 5) + 1u, w >> (32u - o));
+		}
+		run.bits += bpw;
+	}
 }
 // Staging words per job of a sync-free pass with LDS jobs (on average: each workgroup fills its
 // share of the area in turn); a chunk that no longer fits goes to a_job_rest like one larger than
@@ -3530,8 +3536,7 @@ constexpr u32 kEtmpJobWords = 512;
 // a_encode_size does (SetLeaf's size decision). A chunk of at most kJobHdr words is staged in the
 // workgroup's share of etmp (etmp_cap words); a larger one, or one that no longer fits, is listed for
 // a_job_rest, which rebuilds and encodes it in place once the append offsets are known.
-template <bool kFull>
-__global__ void __launch_bounds__(kEncThreads, 4) a_job_encode(EditParams P, const ALevel *__restrict__ lv,
+__global__ void __launch_bounds__(kEncThreads, 6) a_job_encode(EditParams P, const ALevel *__restrict__ lv,
                                                              u32 *__restrict__ pm, const uint4 *__restrict__ jrange,
                                                              const unsigned short *__restrict__ lidx,
                                                              const uint2 *__restrict__ ecol, u32 V,
@@ -3549,52 +3554,29 @@ __global__ void __launch_bounds__(kEncThreads, 4) a_job_encode(EditParams P, con
 	u32 used = 0;
 	for (u32 c0 = blockIdx.x; c0 < n; c0 += gridDim.x * kJobChunk)
 	for (u64 m = writer_chunk(ent, n, c0, &s_wm, [&](u32 e) { app[e] = 0; }); m; m &= m - 1ull) {
-		const u32 e = c0 + (u32)__builtin_ctzll(m) * gridDim.x;
-		__syncthreads(); // the previous job's readers are done with S
+		const u32 e = __builtin_amdgcn_readfirstlane(c0 + (u32)__builtin_ctzll(m) * gridDim.x);
 		Entry E;
 		uint4 jh;
-		job_rebuild(P, lv, jrange, lidx, ecol, V, e, S, E, jh);
+		JobSeg R;
+		job_rebuild(P, lv, jrange, lidx, ecol, V, e, S, E, jh, R);
 		const bool chunk = ctag(E.octree) == kTagLeaf;
 		const u32 block = jh.z;
-		// encode: a_encode_size's register path over the LDS colors
-		JobEnc R;
-		enc_scan_job<kFull>(S, V, R);
 		EncScan tot;
-		EncScan run = block_excl_scan(R.x, S.sh, tot);
+		const EncScan run = block_excl_scan(R.x, S.sh, tot);
 		const u32 B = tot.heads, W = (tot.bits + 31u) >> 5, ds = 6u + 2u * B + W;
 		const bool staged = ds <= kJobHdr && used + ds <= per_block; // block-uniform
 		const u32 off = blk_base + used;
 		used += staged ? ds : 0u;
 		if (staged) {
-			const u32 bo = 6u, wo = bo + 2u * B;
-			for (u32 w = threadIdx.x; w < W; w += kEncThreads)
-				S.stmp[wo + w] = 0u;
-			if (threadIdx.x == 0) {
-				S.stmp[0] = 0u;
-				S.stmp[1] = 1u;
-				S.stmp[2] = B;
-				S.stmp[3] = W;
-				S.stmp[4] = 0u;
-				S.stmp[5] = 0u;
+			const u32 wo = 6u + 2u * B;
+			if (threadIdx.x < 6u) // one macro block
+				S.stmp[threadIdx.x] = threadIdx.x == 1u ? 1u : (threadIdx.x == 2u ? B : (threadIdx.x == 3u ? W : 0u));
+			if (W) { // block-uniform
+				for (u32 w = threadIdx.x; w < W; w += kEncThreads)
+					S.stmp[wo + w] = 0u;
+				__syncthreads();
 			}
-			__syncthreads();
-#pragma unroll
-			for (u32 k = 0; k < kEncPer; ++k)
-				if (kFull || k < R.n) {
-					const u32 v = R.v0 + k, wb = unpack_wb16(S.colw[v]), bpw = (wb >> 8) & 0xFFu;
-					if ((R.heads >> k) & 1u) {
-						S.stmp[bo + 2u * run.heads] = S.colc[v];
-						S.stmp[bo + 2u * run.heads + 1u] = (v << 18) | (bpw << 16) | run.bits;
-						run.heads += 1u;
-					}
-					if (bpw) {
-						const u32 w = wb & ((1u << bpw) - 1u), o = run.bits & 31u;
-						atomicOr(&S.stmp[wo + (run.bits >> 5)], w << o);
-						if (o + bpw > 32u)
-							atomicOr(&S.stmp[wo + (run.bits >> 5) + 1u], w >> (32u - o));
-					}
-					run.bits += bpw;
-				}
+			job_write(R, run, wo, [&](u32 i, u32 x) { S.stmp[i] = x; }, [&](u32 i, u32 x) { atomicOr(&S.stmp[i], x); });
 			__syncthreads();
 			for (u32 w = threadIdx.x; w < ds; w += kEncThreads)
 				etmp[(u64)off + w] = S.stmp[w];
@@ -3622,7 +3604,6 @@ __global__ void __launch_bounds__(kEncThreads, 4) a_job_encode(EditParams P, con
 // give the same colors and size) and encoded straight into the color leaves at the offset the
 // append scan gave, or over the old chunk when it fits in place (the rebuild has read it whole
 // before the first store). One workgroup per job.
-template <bool kFull>
 __global__ void __launch_bounds__(kEncThreads, 3) a_job_rest(EditParams P, const ALevel *__restrict__ lv,
                                                            const u32 *__restrict__ pm, const uint4 *__restrict__ jrange,
                                                            const unsigned short *__restrict__ lidx,
@@ -3636,23 +3617,21 @@ __global__ void __launch_bounds__(kEncThreads, 3) a_job_rest(EditParams P, const
 	const u32 nrest = pm[kPmCut] ? 0u : pm[kPmRest]; // (a chained pass that did not hold writes nothing)
 	for (u32 i = blockIdx.x; i < nrest; i += gridDim.x) {
 		const u32 e = rest[i];
-		__syncthreads(); // the previous job's readers are done with S
 		Entry E;
 		uint4 jh;
-		job_rebuild(P, lv, jrange, lidx, ecol, V, e, S, E, jh);
-		JobEnc R;
-		enc_scan_job<kFull>(S, V, R);
+		JobSeg R;
+		job_rebuild(P, lv, jrange, lidx, ecol, V, e, S, E, jh, R);
 		EncScan tot;
-		EncScan run = block_excl_scan(R.x, S.sh, tot);
+		const EncScan run = block_excl_scan(R.x, S.sh, tot);
 		const u32 ds = info[4 * e], as = info[4 * e + 1], inplace = info[4 * e + 2] & 1u;
 		const u32 idx = inplace ? cdata(E.octree) : leaf_base + appo[e];
 		u32 result = E.octree;
 		if (inplace || (u64)idx + as <= leaf_cap) {
 			u32 *Lw = P.cleaves;
 			const u32 B = tot.heads, W = (tot.bits + 31u) >> 5;
-			const u32 mo = idx + 4u, bo = mo + 2u, wo = bo + 2u * B; // one macro block (V <= 2^14)
+			const u32 mo = idx + 4u, wo = 6u + 2u * B; // one macro block (V <= 2^14)
 			for (u32 w = threadIdx.x; w < W; w += kEncThreads)
-				Lw[wo + w] = 0u;
+				Lw[idx + wo + w] = 0u;
 			if (threadIdx.x == 0) {
 				Lw[mo] = 0u;
 				Lw[mo + 1u] = 0u;
@@ -3663,23 +3642,7 @@ __global__ void __launch_bounds__(kEncThreads, 3) a_job_rest(EditParams P, const
 					Lw[idx] = as;
 			}
 			__syncthreads();
-#pragma unroll
-			for (u32 k = 0; k < kEncPer; ++k)
-				if (kFull || k < R.n) {
-					const u32 v = R.v0 + k, wb = unpack_wb16(S.colw[v]), bpw = (wb >> 8) & 0xFFu;
-					if ((R.heads >> k) & 1u) {
-						Lw[bo + 2u * run.heads] = S.colc[v];
-						Lw[bo + 2u * run.heads + 1u] = (v << 18) | (bpw << 16) | run.bits;
-						run.heads += 1u;
-					}
-					if (bpw) {
-						const u32 w = wb & ((1u << bpw) - 1u), o = run.bits & 31u;
-						atomicOr(&Lw[wo + (run.bits >> 5)], w << o);
-						if (o + bpw > 32u)
-							atomicOr(&Lw[wo + (run.bits >> 5) + 1u], w >> (32u - o));
-					}
-					run.bits += bpw;
-				}
+			job_write(R, run, wo, [&](u32 i, u32 x) { Lw[idx + i] = x; }, [&](u32 i, u32 x) { atomicOr(&Lw[idx + i], x); });
 			if (!inplace)
 				for (u32 w = ds + threadIdx.x; w < as; w += kEncThreads)
 					Lw[idx + w] = 0u;
@@ -5897,8 +5860,7 @@ static int queue_pass(Pool &p, const PassPlan &pp, AsyncBufs &B, bool reserve = 
 		const u32 G = grid_for(pp.cap[leafL], 1, 8192);
 		a_encode_write<<<G, kEncThreads, 0, s>>>(P, B.d_lv, B.pm, B.dense, V, B.info, B.appo, p.cleaf_cap, B.etmp);
 		if (ljobs) {
-			const auto rest = V == kJobV ? a_job_rest<true> : a_job_rest<false>;
-			rest<<<std::min(G, 1024u), kEncThreads, 0, s>>>(P, B.d_lv, B.pm, B.jrange, B.lidx, B.ecol, V, B.info, B.appo,
+			a_job_rest<<<std::min(G, 1024u), kEncThreads, 0, s>>>(P, B.d_lv, B.pm, B.jrange, B.lidx, B.ecol, V, B.info, B.appo,
 			                                               p.cleaf_cap, B.rest);
 		}
 	};
@@ -5916,8 +5878,7 @@ static int queue_pass(Pool &p, const PassPlan &pp, AsyncBufs &B, bool reserve = 
 		if (ljobs) {
 			a_job_ranges<<<grid_for(std::max<u64>(pp.cap[leafL], pp.count), 256, 4096), 256, 0, p.cstream>>>(
 			    B.d_lv, B.pm, leafL, L, p.cleaves, B.jrange, P.edits, pp.count, B.ecol);
-			const auto job = V == kJobV ? a_job_encode<true> : a_job_encode<false>;
-			job<<<G, kEncThreads, 0, p.cstream>>>(P, B.d_lv, B.pm, B.jrange, B.lidx, B.ecol, V, B.info, B.app, B.etmp,
+			a_job_encode<<<G, kEncThreads, 0, p.cstream>>>(P, B.d_lv, B.pm, B.jrange, B.lidx, B.ecol, V, B.info, B.app, B.etmp,
 			                                      B.etmp_cap, B.rest);
 		}
 		else {
