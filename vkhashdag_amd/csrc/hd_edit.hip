@@ -1962,7 +1962,8 @@ __global__ void a_push(const PushEvent *__restrict__ ev, const u32 *__restrict__
 }
 
 // ---- leaves + bottom-up DAG
-// OR over the 8 lanes of a half row / the other half row's value (a group: one row of 16 lanes)
+constexpr u32 kLeafLanes = 16, kLeafPer = 64 / kLeafLanes; // a group: one row of 16 lanes; a leaf's voxels per lane
+// OR over the 8 lanes of a half row / the other half row's value
 template <int kCtrl> __device__ inline u32 row_move(u32 x) {
 	return (u32)__builtin_amdgcn_mov_dpp((int)x, kCtrl, 0xF, 0xF, true);
 }
@@ -2001,6 +2002,46 @@ __device__ inline u32 group_find_leaf(const u32 *__restrict__ W, const u32 *__re
 			return (u32)(base + i0 + 4u * first + ((hita >> first) & 1u ? 0u : 2u));
 		}
 		x = y;
+	}
+	return kNull;
+}
+
+// The inner node of n words at `node` (LDS) among the bucket's existing ones, by a group of 16 lanes, 64 words a
+// step, where headers are told by value (headers_by_value): the first place whose n words equal the node is
+// find_node's answer (find_in_words_hv). Buckets of 64 words or more.
+__device__ inline u32 group_find_inner(const u32 *__restrict__ W, const u32 *__restrict__ bucket_words,
+                                       const DevConfig &c, u32 bucket, const u32 *node, u32 n, u32 g, u32 row) {
+	const u64 base = (u64)bucket << c.wbpb();
+	const uint4 *W4 = reinterpret_cast<const uint4 *>(W + base);
+	uint4 x = ldg(W4, g), y = make_uint4(0u, 0u, 0u, 0u);
+	if (c.words_per_bucket() >= 128u)
+		y = ldg(W4, 16u + g);
+	const u32 bw = ldg(bucket_words, bucket), h0 = node[0], h1 = node[1];
+	for (u32 i0 = 0; i0 < bw; i0 += 64u) { // two steps' words are in flight
+		uint4 z = make_uint4(0u, 0u, 0u, 0u);
+		if (i0 + 128u < bw) // (whole 64-word steps stay inside the bucket)
+			z = ldg(W4, (i0 >> 2) + 32u + g);
+		const u32 j = i0 + 4u * g, next = row_move<0x101>(x.x); // row_shl 1: the lane after's first word
+		u32 cand = (x.x == h0 && x.y == h1 ? 1u : 0u) | (x.y == h0 && x.z == h1 ? 2u : 0u) |
+		           (x.z == h0 && x.w == h1 ? 4u : 0u) | (x.w == h0 && (g == 15u || next == h1) ? 8u : 0u);
+		if ((__ballot(cand != 0u) >> (16u * row)) & 0xFFFFu) {
+			u32 pos = kNull;
+			for (; cand && pos == kNull; cand &= cand - 1u) {
+				const u32 at = j + (u32)__builtin_ctz(cand);
+				bool eq = at + n <= bw;
+				if (eq)
+#pragma unroll
+					for (u32 k = 1; k < 9; ++k)
+						if (k < n)
+							eq = eq && ldg(W, base + at + k) == node[k];
+				pos = eq ? at : kNull;
+			}
+			const u32 hit = (u32)(__ballot(pos != kNull) >> (16u * row)) & 0xFFFFu;
+			if (hit)
+				return (u32)base + (u32)__shfl((int)pos, (int)(16u * row + (u32)__builtin_ctz(hit)));
+		}
+		x = y;
+		y = z;
 	}
 	return kNull;
 }
@@ -2061,7 +2102,6 @@ __device__ inline bool leaf_writes_colors(const EditParams &P, const ALevel *__r
 // of the color and a mask bit); the color job reads the color from that edit.
 enum : u32 { kLeafAll = 0, kLeafNodes = 1, kLeafColors = 2 };
 constexpr u32 kNoEdit = 0xFFFFu; // a pass with LDS color jobs holds fewer edits
-constexpr u32 kLeafLanes = 16, kLeafPer = 64 / kLeafLanes;
 template <u32 kMode>
 __global__ void __launch_bounds__(kAT) a_leaf(EditParams P, const ALevel *__restrict__ lv, const u32 *__restrict__ pm,
                                               Color *__restrict__ lcol, u64 *__restrict__ lmask,
@@ -2268,16 +2308,16 @@ __device__ inline Built join_entry(const EditParams &P, u32 l, const ALevel &A, 
 	}
 	return o;
 }
-// The find of a joined entry among its bucket's existing nodes. Returns false when the
-// workgroup's stage was full (the find runs again after a reset; the join is kept).
-__device__ inline bool find_entry(const EditParams &P, u32 l, const ALevel &A, u32 e, const Built &o, u32 *stage,
-                                  u32 *top, u32 cap) {
-	u32 bw;
-	const u32 f = o.need ? kNull // a fresh child: a new node
-	                     : find_in_bucket_staged(P.words, P.bucket_words, P.c, o.b, o.c, o.k, headers_by_value(P.c, l),
-	                                             bw, stage, top, cap);
-	if (f == kFindRetry)
-		return false;
+// The finds of a workgroup's joined entries among their buckets' existing nodes: the entries' nodes are queued in
+// LDS and each group of 16 lanes takes one at a time. (Each thread copied its own entry's bucket to an LDS
+// stage and scanned it there: a few buckets filled the stage, the other threads waited for the next round.
+// The first level above the leaves of 4096 mixed edits, in a world after 20 such batches: 10.4 -> 6.7 ms beside the
+// color stream; the levels of about 27 chained edits 31 -> 18 us each.)
+struct FindLds {
+	u32 node[kAT][9], e[kAT], b[kAT], k[kAT], n;
+};
+// Entry e's join: what is known of it is written, and the find is queued. (A fresh child: a new node.)
+__device__ inline void queue_find(const EditParams &P, u32 l, const ALevel &A, u32 e, const Built &o, FindLds &S) {
 #pragma unroll
 	for (u32 j = 0; j < 9; ++j)
 		if (j < o.k)
@@ -2285,8 +2325,41 @@ __device__ inline bool find_entry(const EditParams &P, u32 l, const ALevel &A, u
 	stg(A.pend, e, 1u);
 	stg(A.csize, e, o.k);
 	stg(A.bucket, e, o.b);
-	stg(A.res, e, f);
-	return true;
+	if (o.need)
+		stg(A.res, e, kNull);
+	else if (P.c.wbpb() < 6 || !headers_by_value(P.c, l))
+		stg(A.res, e, find_in_global(P.words, P.c, (u64)o.b << P.c.wbpb(), ldg(P.bucket_words, o.b), o.c, o.k));
+	else {
+		const u32 i = atomicAdd(&S.n, 1u);
+#pragma unroll
+		for (u32 j = 0; j < 9; ++j)
+			S.node[i][j] = o.c[j];
+		S.e[i] = e, S.b[i] = o.b, S.k[i] = o.k;
+	}
+}
+// Entries a workgroup takes at a time: a group of lanes has one find each where the level leaves the chip idle.
+__device__ inline u32 build_chunk(u32 n) { return min(max((n + gridDim.x - 1u) / gridDim.x, kAT / kLeafLanes), kAT); }
+template <class Join>
+__device__ inline void build_level(const EditParams &P, u32 l, const ALevel &A, u32 n, FindLds &S, Join join) {
+	const u32 chunk = build_chunk(n), g = threadIdx.x & (kLeafLanes - 1u), row = (threadIdx.x & 63u) / kLeafLanes;
+	for (u64 e0 = (u64)blockIdx.x * chunk; e0 < n; e0 += (u64)gridDim.x * chunk) { // uniform trip count
+		if (threadIdx.x == 0)
+			S.n = 0;
+		__syncthreads();
+		const u64 e = e0 + threadIdx.x;
+		if (threadIdx.x < chunk && e < n) {
+			const Built o = join((u32)e);
+			if (o.k)
+				queue_find(P, l, A, (u32)e, o, S);
+		}
+		__syncthreads();
+		for (u32 i = threadIdx.x / kLeafLanes; i < S.n; i += kAT / kLeafLanes) {
+			const u32 f = group_find_inner(P.words, P.bucket_words, P.c, S.b[i], S.node[i], S.k[i], g, row);
+			if (g == 0)
+				stg(A.res, S.e[i], f);
+		}
+		__syncthreads();
+	}
 }
 
 // Joins entry e (pending, not in the pool) to its content's group; the creator queues the group
@@ -2529,31 +2602,11 @@ __device__ inline u32 walk_entry(const EditParams &P, u32 l, const ALevel &A, co
 	return appended;
 }
 
-// kCap: staging words per workgroup. Entries whose buckets do not fit the stage wait for the next
-// round, so a larger stage takes fewer rounds; 10240 words (40 KiB) fit beside three color-job
-// workgroups on a CU, for the batched passes whose color jobs run beside their node levels.
-template <u32 kCap>
 __global__ void __launch_bounds__(kAT) a_build(EditParams P, u32 l, const ALevel *__restrict__ lv,
-                                               const u32 *__restrict__ pm, GroupTable G) {
-	__shared__ __align__(16) u32 stage[kCap];
-	__shared__ u32 top;
+                                               u32 *__restrict__ pm, GroupTable G) {
+	__shared__ FindLds S;
 	const ALevel A = lv[l], C = lv[l + 1];
-	const u32 n = pm[kPmHdr + l];
-	for (u32 e0 = blockIdx.x * blockDim.x; e0 < n; e0 += gridDim.x * blockDim.x) { // uniform trip count
-		const u32 e = e0 + threadIdx.x;
-		Built o{};
-		o.k = 0;
-		if (e < n)
-			o = join_entry(P, l, A, C, G, e);
-		bool todo = o.k != 0;
-		do { // an entry whose bucket found the stage full looks again after the reset
-			if (threadIdx.x == 0)
-				top = 0;
-			__syncthreads();
-			if (todo)
-				todo = !find_entry(P, l, A, e, o, stage, &top, kCap);
-		} while (__syncthreads_or(todo));
-	}
+	build_level(P, l, A, pm[kPmHdr + l], S, [&](u32 e) { return join_entry(P, l, A, C, G, e); });
 }
 // child_result_fresh of a chained pass: x the result, y bit 0 a fresh append, bit 1 unchanged (the
 // node's version before the edit, whatever x says: also when its bucket was full).
@@ -2678,12 +2731,10 @@ __device__ inline Built chain_join(const EditParams &P, u32 l, const ALevel &A, 
 // a_build of a chained pass. The links of a level near the root (at most kLinkEntries entries, long
 // version chains) are staged in LDS; below, a node has a version or two.
 constexpr u32 kLinkEntries = 512;
-template <u32 kCap>
 __global__ void __launch_bounds__(kAT) a_build_chain(EditParams P, u32 l, const ALevel *__restrict__ lv,
                                                      u32 *__restrict__ pm, GroupTable G) {
-	__shared__ __align__(16) u32 stage[kCap];
+	__shared__ FindLds S;
 	__shared__ uint4 links[kLinkEntries];
-	__shared__ u32 top;
 	const ALevel A = lv[l], C = lv[l + 1];
 	const u32 n = pm[kPmHdr + l];
 	auto load = [&](u32 q) { return make_uint4(ldg(A.prev, q), ldg(A.pmask, q), ldg(A.first_child, q), 0u); };
@@ -2691,21 +2742,9 @@ __global__ void __launch_bounds__(kAT) a_build_chain(EditParams P, u32 l, const 
 		for (u32 i = threadIdx.x; i < n; i += kAT)
 			links[i] = load(i);
 	__syncthreads();
-	for (u32 e0 = blockIdx.x * blockDim.x; e0 < n; e0 += gridDim.x * blockDim.x) { // uniform trip count
-		const u32 e = e0 + threadIdx.x;
-		Built o{};
-		o.k = 0;
-		if (e < n)
-			o = chain_join(P, l, A, C, G, e, pm, [&](u32 q) { return n <= kLinkEntries ? links[q] : load(q); });
-		bool todo = o.k != 0;
-		do { // an entry whose bucket found the stage full looks again after the reset
-			if (threadIdx.x == 0)
-				top = 0;
-			__syncthreads();
-			if (todo)
-				todo = !find_entry(P, l, A, e, o, stage, &top, kCap);
-		} while (__syncthreads_or(todo));
-	}
+	build_level(P, l, A, n, S, [&](u32 e) {
+		return chain_join(P, l, A, C, G, e, pm, [&](u32 q) { return n <= kLinkEntries ? links[q] : load(q); });
+	});
 }
 // The levels [0, l_from] of a chained pass, each of at most kChainSmall entries, in one workgroup (a thread
 // per entry): the join over the versions' rows in LDS (children's results by slot, left there by the level
@@ -5907,12 +5946,9 @@ static int queue_pass(Pool &p, const PassPlan &pp, AsyncBufs &B, bool reserve = 
 		HD_RET(queue_colors());
 	for (int l = (int)L - 1; l > l_from; --l) {
 		u32 G = grid_for(pp.cap[l], kAT, 4096);
-		if (l + 1 < (int)L && pp.chained)
-			a_build_chain<16384><<<G, kAT, 0, p.stream>>>(P, (u32)l, B.d_lv, B.pm, B.G);
-		else if (l + 1 < (int)L)
-			// a single-edit pass has few color jobs beside it: twice the stage (256 sphere edits on
-			// the 4096^3 terrain: 41.1 -> 40.3 ms per step; the 4096-edit batch 1 % slower with it)
-			(pp.count == 1 ? a_build<20480> : a_build<10240>)<<<G, kAT, 0, p.stream>>>(P, (u32)l, B.d_lv, B.pm, B.G);
+		if (l + 1 < (int)L)
+			(pp.chained ? a_build_chain : a_build)<<<grid_for(pp.cap[l], kAT / kLeafLanes, 4096), kAT, 0, p.stream>>>(
+			    P, (u32)l, B.d_lv, B.pm, B.G);
 		a_dedup<<<G, kAT, 0, p.stream>>>(P, (u32)l, B.d_lv, B.pm, B.G, B.bcnt, B.head, B.blist);
 		a_walk<<<G, kAT, 0, p.stream>>>(P, (u32)l, B.d_lv, B.pm, B.G, B.bcnt, B.head, B.blist, B.acc);
 		if (!colors_queued && l <= color_after)
