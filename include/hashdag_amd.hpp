@@ -435,16 +435,8 @@ public:
 	// NodePoolTraversal::Traversal<float>(root, o, d): the hit position in [0,1]^3 or nullopt.
 	inline std::optional<std::array<float, 3>> Traversal(NodePointer root, const std::array<float, 3> &o,
 	                                                     const std::array<float, 3> &d) const {
-		void *buf = nullptr;
-		if (hd_device_alloc(sizeof(float) * 10, &buf) != HD_OK)
-			return std::nullopt;
-		float host[6] = {o[0], o[1], o[2], d[0], d[1], d[2]}, out[4] = {0, 0, 0, 0};
-		float *dev = static_cast<float *>(buf);
-		bool ok = hd_memcpy_h2d(dev, host, sizeof(host)) == HD_OK &&
-		          hd_traversal(m_pool, *root, dev, dev + 3, 1, dev + 6) == HD_OK &&
-		          hd_memcpy_d2h(out, dev + 6, sizeof(out)) == HD_OK;
-		hd_device_free(buf);
-		if (!ok || out[3] == 0.0f)
+		float out[4] = {0, 0, 0, 0};
+		if (hd_traversal_host(m_pool, *root, o.data(), d.data(), 1, out) != HD_OK || out[3] == 0.0f)
 			return std::nullopt;
 		return std::array<float, 3>{out[0], out[1], out[2]};
 	}

@@ -258,6 +258,9 @@ int hd_timer_end(hd_pool *pool, float *ms);
 /* NodePoolTraversal::Traversal<float> (NodePoolTraversal.hpp:93-256) for n rays given as device
  * arrays o[3n], d[3n]; out: device float[4n] = hit position in [0,1]^3 + hit flag. */
 int hd_traversal(hd_pool *pool, uint32_t root, const float *o, const float *d, uint64_t n, float *out);
+/* The same for at most HD_TRAVERSAL_HOST_RAYS rays in host memory (a pick): no device buffers and no copies. */
+#define HD_TRAVERSAL_HOST_RAYS 1024
+int hd_traversal_host(hd_pool *pool, uint32_t root, const float *o, const float *d, uint64_t n, float *out);
 
 /* ---- frames captured as hipGraphs: up to max_passes passes of pairwise-disjoint edits (max_edits
  * each, every edit within max_radius voxels: sphere radius or box half-extent) followed by one

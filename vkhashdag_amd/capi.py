@@ -135,6 +135,7 @@ def lib():
             "hd_trace_beam_sizes": (C.c_int, [VP, U32, VP]),
             "hd_trace_beam_async": (C.c_int, [VP, U32, U32, VP, VP, VP, U32, U32, U32, VP, VP]),
             "hd_traversal": (C.c_int, [VP, U32, VP, VP, U64, VP]),
+            "hd_traversal_host": (C.c_int, [VP, U32, VP, VP, U64, VP]),
             "hd_device_alloc": (C.c_int, [U64, C.POINTER(VP)]),
             "hd_device_free": (C.c_int, [VP]),
             "hd_memcpy_h2d": (C.c_int, [VP, VP, U64]),
@@ -163,6 +164,9 @@ def lib():
 def check(rc):
     if rc != 0:
         raise HDError(f"hd error {rc}: {lib().hd_last_error().decode()}")
+
+
+TRAVERSAL_HOST_RAYS = 1024  # HD_TRAVERSAL_HOST_RAYS
 
 
 class DeviceBuffer:
@@ -400,6 +404,11 @@ class DevicePool:
         o = np.ascontiguousarray(o, np.float32).reshape(-1, 3)
         d = np.ascontiguousarray(d, np.float32).reshape(-1, 3)
         n = len(o)
+        if n <= TRAVERSAL_HOST_RAYS and len(d) >= n:
+            out = np.empty((n, 4), np.float32)
+            check(lib().hd_traversal_host(self.h, self.root if root is None else root, o.ctypes.data, d.ctypes.data, n,
+                                          out.ctypes.data))
+            return out
         bo, bd, bout = DeviceBuffer(o.nbytes), DeviceBuffer(d.nbytes), DeviceBuffer(n * 16)
         bo.upload(o)
         bd.upload(d)

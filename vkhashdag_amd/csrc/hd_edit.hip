@@ -4989,6 +4989,19 @@ __global__ void a_set_roots_keep(u32 *roots, u32 root, u32 croot) {
 	roots[0] = root;
 	roots[1] = croot;
 }
+// A call's level table and edits, passed by value: two copies from pageable memory and the wait for them held
+// the host for about 40 us (with the table of per-level buffers, one edit in a 4096^3 world 220 -> 153 us).
+constexpr u32 kPutLevels = 12, kPutEdits = 16;
+struct PutSetup {
+	u32 lv[kPutLevels * sizeof(ALevel) / 4], edits[kPutEdits * sizeof(hd_edit_desc) / 4], n_lv, n_edits;
+};
+static_assert(sizeof(ALevel) % 4 == 0 && sizeof(hd_edit_desc) % 4 == 0 && sizeof(PutSetup) <= 3584);
+__global__ void __launch_bounds__(256) a_put_setup(PutSetup a, u32 *__restrict__ lv, u32 *__restrict__ edits) {
+	for (u32 i = threadIdx.x; i < a.n_lv * (u32)(sizeof(ALevel) / 4); i += 256)
+		lv[i] = a.lv[i];
+	for (u32 i = threadIdx.x; i < a.n_edits * (u32)(sizeof(hd_edit_desc) / 4); i += 256)
+		edits[i] = a.edits[i];
+}
 __global__ void a_fill_u32(u32 *p, u64 n, u32 v) {
 	for (u64 i = (u64)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (u64)gridDim.x * blockDim.x)
 		p[i] = v;
@@ -5404,10 +5417,7 @@ static u64 async_budget(const Pool &p) {
 	size_t free_b = 0, total_b = 0;
 	if (hipMemGetInfo(&free_b, &total_b) != hipSuccess)
 		return kAsyncBudget;
-	u64 held = 0;
-	for (const auto &kv : p.scratch.bufs)
-		held += kv.second.bytes;
-	return std::min<u64>(kAsyncBudget, ((u64)free_b + held) / 4 * 3);
+	return std::min<u64>(kAsyncBudget, ((u64)free_b + p.scratch.held()) / 4 * 3);
 }
 
 // Upper bounds on the proceeding nodes of a pass, per level. A node proceeds only where some
@@ -5629,6 +5639,8 @@ struct AsyncBufs {
 };
 constexpr u32 kMaxEmitBlocks = 1024;
 
+enum : u32 { kLvEnt, kLvLists, kLvKids, kLvFchild, kLvPmask, kLvPrev, kLvOkids, kLvStatus, kLvPend, kLvRes, kLvSlot, kLvLpos, kLvBucket, kLvContent, kLvCsize, kLvPev, kLvOres, kLvCcnt, kLvCbase, kLvOwn, kLvCount };
+static_assert(kLvCount <= kLevelBufs);
 // Buffers for the largest bounds of the call's sync-free passes (allocated before any pass is
 // queued: a growing buffer would be freed under queued work).
 static int async_setup(Pool &p, const std::vector<PassPlan> &plans, const std::vector<hd_edit_desc> &flat,
@@ -5651,48 +5663,54 @@ static int async_setup(Pool &p, const std::vector<PassPlan> &plans, const std::v
 		ev = std::max(ev, pp.ev_cap);
 		stateful |= pp.stateful;
 	}
+	LevelBufs &bufs = p.scratch.levels[pre];
+	auto get = [&](u32 l, u32 which, u64 count, auto **out) -> int {
+		DevBuf &b = bufs.b[l][which];
+		HD_RET(b.ensure(std::max<u64>(count, 1) * sizeof(**out)));
+		*out = b.as<std::remove_reference_t<decltype(**out)>>();
+		return HD_OK;
+	};
 	B.lv.assign(L, ALevel{});
 	for (u32 l = 0; l < L; ++l) {
 		ALevel &A = B.lv[l];
 		const u64 c = std::max<u64>(cap[l], 1);
 		A.cap = (u32)cap[l];
 		A.list_cap = (u32)lcap[l];
-		HD_RET(buf(p, (pre + "ent").c_str(), l, c, &A.ent));
-		HD_RET(buf(p, (pre + "lists").c_str(), l, std::max<u64>(lcap[l], 1), &A.lists));
+		HD_RET(get(l, kLvEnt, c, &A.ent));
+		HD_RET(get(l, kLvLists, std::max<u64>(lcap[l], 1), &A.lists));
 		if (l + 1 < L) {
-			HD_RET(buf(p, (pre + "kids").c_str(), l, 8 * c, &A.kids));
-			HD_RET(buf(p, (pre + "fchild").c_str(), l, c, &A.first_child));
-			HD_RET(buf(p, (pre + "pmask").c_str(), l, c, &A.pmask));
+			HD_RET(get(l, kLvKids, 8 * c, &A.kids));
+			HD_RET(get(l, kLvFchild, c, &A.first_child));
+			HD_RET(get(l, kLvPmask, c, &A.pmask));
 			if (chained)
-				HD_RET(buf(p, (pre + "prev").c_str(), l, c, &A.prev));
+				HD_RET(get(l, kLvPrev, c, &A.prev));
 			if (stateful && l < leafL)
-				HD_RET(buf(p, (pre + "okids").c_str(), l, 8 * c, &A.okids));
+				HD_RET(get(l, kLvOkids, 8 * c, &A.okids));
 		}
-		HD_RET(buf(p, (pre + "status").c_str(), l, c, &A.status));
-		HD_RET(buf(p, (pre + "pend").c_str(), l, c, &A.pend));
-		HD_RET(buf(p, (pre + "res").c_str(), l, c, &A.res));
-		HD_RET(buf(p, (pre + "slot").c_str(), l, c, &A.slot));
-		HD_RET(buf(p, (pre + "lpos").c_str(), l, c, &A.lpos));
-		HD_RET(buf(p, (pre + "bucket").c_str(), l, c, &A.bucket));
-		HD_RET(buf(p, (pre + "content").c_str(), l, c * (l + 1 < L ? 9 : 2), &A.content));
+		HD_RET(get(l, kLvStatus, c, &A.status));
+		HD_RET(get(l, kLvPend, c, &A.pend));
+		HD_RET(get(l, kLvRes, c, &A.res));
+		HD_RET(get(l, kLvSlot, c, &A.slot));
+		HD_RET(get(l, kLvLpos, c, &A.lpos));
+		HD_RET(get(l, kLvBucket, c, &A.bucket));
+		HD_RET(get(l, kLvContent, c * (l + 1 < L ? 9 : 2), &A.content));
 		if (l + 1 < L)
-			HD_RET(buf(p, (pre + "csize").c_str(), l, c, &A.csize));
+			HD_RET(get(l, kLvCsize, c, &A.csize));
 		if (stateful && lds_jobs(p.dc) && l >= leafL && l + 1 < L)
-			HD_RET(buf(p, (pre + "pev").c_str(), l, 8 * c, &A.pev));
+			HD_RET(get(l, kLvPev, 8 * c, &A.pev));
 		if (stateful && l <= leafL) {
-			HD_RET(buf(p, (pre + "ores").c_str(), l, c, &A.ores));
-			HD_RET(buf(p, (pre + "ccnt").c_str(), l, c, &A.ccnt));
-			HD_RET(buf(p, (pre + "cbase").c_str(), l, c, &A.cbase));
-			HD_RET(buf(p, (pre + "own").c_str(), l, c, &A.own));
+			HD_RET(get(l, kLvOres, c, &A.ores));
+			HD_RET(get(l, kLvCcnt, c, &A.ccnt));
+			HD_RET(get(l, kLvCbase, c, &A.cbase));
+			HD_RET(get(l, kLvOwn, c, &A.own));
 		}
 	}
 	if (chained)
 		HD_RET(p.scratch.get<u32>(pre + "saved", p.total_buckets + 2, &B.saved));
 	HD_RET(p.scratch.get<ALevel>(pre + "levels", L, &B.d_lv));
-	HD_TRY(hipMemcpyAsync(B.d_lv, B.lv.data(), L * sizeof(ALevel), hipMemcpyHostToDevice, p.stream));
 	HD_RET(p.scratch.get<u32>(pre + "pm", kPmHdr + 2 * L, &B.pm));
-	HD_RET(p.scratch.get<u32>(pre + "roots", 2, &B.roots));
-	HD_RET(p.scratch.get<u32>(pre + "acc", kAccCount, &B.acc));
+	HD_RET(p.scratch.get<u32>(pre + "roots", 2 + kAccCount, &B.roots)); // one copy reads both
+	B.acc = B.roots + 2;
 	HD_RET(p.scratch.get<u32>(pre + "flag", maxpairs, &B.flag));
 	HD_RET(p.scratch.get<u32>(pre + "lcnt", maxpairs, &B.lcnt));
 	HD_RET(p.scratch.get<uint4>(pre + "cstate", maxpairs, &B.cstate));
@@ -5720,7 +5738,19 @@ static int async_setup(Pool &p, const std::vector<PassPlan> &plans, const std::v
 		HD_RET(p.scratch.get<uint2>(pre + "ecol", max_count, &B.ecol));
 	}
 	HD_RET(p.scratch.get<hd_edit_desc>(pre + "edits", std::max<size_t>(flat.size(), 1), &B.edits));
-	HD_TRY(hipMemcpyAsync(B.edits, flat.data(), flat.size() * sizeof(hd_edit_desc), hipMemcpyHostToDevice, p.stream));
+	// the level table and a few edits as the arguments of kernels; more edits by a copy
+	const bool few = flat.size() <= kPutEdits;
+	for (u32 l0 = 0; l0 < L; l0 += kPutLevels) {
+		PutSetup a;
+		a.n_lv = std::min(kPutLevels, L - l0);
+		a.n_edits = few && l0 == 0 ? (u32)flat.size() : 0u;
+		std::memcpy(a.lv, &B.lv[l0], a.n_lv * sizeof(ALevel));
+		std::memcpy(a.edits, flat.data(), a.n_edits * sizeof(hd_edit_desc));
+		a_put_setup<<<1, 256, 0, p.stream>>>(a, (u32 *)(B.d_lv + l0), (u32 *)B.edits);
+	}
+	HD_TRY(hipGetLastError());
+	if (!few)
+		HD_TRY(hipMemcpyAsync(B.edits, flat.data(), flat.size() * sizeof(hd_edit_desc), hipMemcpyHostToDevice, p.stream));
 	// group table: 2x the largest level; generations make clearing unnecessary except on growth
 	u64 maxcap = 1;
 	for (u32 l = 0; l < L; ++l)
@@ -5761,7 +5791,8 @@ static int async_setup(Pool &p, const std::vector<PassPlan> &plans, const std::v
 		a_fill_u32<<<g, 256, 0, p.stream>>>(B.head, p.total_buckets, kNull);
 		HD_TRY(hipGetLastError());
 	}
-	HD_TRY(hipStreamSynchronize(p.stream)); // the host staging arrays may go out of scope
+	if (!few)
+		HD_TRY(hipStreamSynchronize(p.stream)); // the host staging array may go out of scope
 	return HD_OK;
 }
 
@@ -6131,9 +6162,8 @@ static int edit_sequence(Pool &p, u32 root, u32 croot, const std::vector<hd_edit
 			HD_RET(edit_pass(p, root, croot, flat.data() + pp.first, pp.count, &root, &croot));
 		}
 	}
-	u32 out[2 + kAccCount];
-	HD_TRY(hipMemcpyAsync(out, B.roots, 8, hipMemcpyDeviceToHost, p.stream));
-	HD_TRY(hipMemcpyAsync(out + 2, B.acc, 4 * kAccCount, hipMemcpyDeviceToHost, p.stream));
+	const u32 *out = p.h_pass; // (no chained pass is open)
+	HD_TRY(hipMemcpyAsync(p.h_pass, B.roots, 4 * (2 + kAccCount), hipMemcpyDeviceToHost, p.stream));
 	HD_TRY(hipStreamSynchronize(p.stream));
 	if (on_device)
 		root = out[0], croot = out[1];
@@ -6422,6 +6452,10 @@ struct FrameState {
 					it = p->scratch.bufs.erase(it);
 				} else
 					++it;
+			if (auto it = p->scratch.levels.find(pre); it != p->scratch.levels.end()) {
+				it->second.release();
+				p->scratch.levels.erase(it);
+			}
 		}
 	}
 };
@@ -6509,7 +6543,7 @@ static int frame_create(Pool &p, const hd_frame_config &cfg, u32 root, u32 croot
 		HD_TRY(hipEventCreateWithFlags(&F.copied[k], hipEventDisableTiming));
 		HD_TRY(hipEventRecord(F.copied[k], p.stream));
 	}
-	HD_TRY(hipHostMalloc((void **)&F.h_roots, 8 + 4 * kAccCount, hipHostMallocDefault));
+	HD_TRY(hipHostMalloc((void **)&F.h_roots, 4 * (2 + kAccCount + HD_MAX_LEVELS), hipHostMallocDefault));
 	std::memset(F.h_views[0], 0, cfg.n_views * sizeof(hd_view));
 	std::memset(F.h_tiles[0], 0, (cfg.n_views + 1) * 4);
 	HD_TRY(hipMemcpyAsync(F.d_views, F.h_views[0], cfg.n_views * sizeof(hd_view), hipMemcpyHostToDevice, p.stream));
@@ -6695,13 +6729,15 @@ extern "C" int hd_frame_wait(hd_frame *f, uint32_t *root_out, uint32_t *color_ro
 		return set_error("hd_frame_wait: null argument"), HD_ERR_ARG;
 	FrameState &F = f->F;
 	Pool &p = *F.p;
-	HD_TRY(hipMemcpyAsync(F.h_roots, F.B.roots, 8, hipMemcpyDeviceToHost, p.stream));
-	HD_TRY(hipMemcpyAsync(F.h_roots + 2, F.B.acc, 4 * kAccCount, hipMemcpyDeviceToHost, p.stream));
+	u32 *filled = F.h_roots + 2 + kAccCount;
+	HD_TRY(hipMemcpyAsync(F.h_roots, F.B.roots, 4 * (2 + kAccCount), hipMemcpyDeviceToHost, p.stream));
+	if (F.cfg.flags & HD_FRAME_GC)
+		HD_TRY(hipMemcpyAsync(filled, p.d_filled, p.dc.L * 4, hipMemcpyDeviceToHost, p.stream));
 	HD_TRY(hipStreamSynchronize(p.stream));
 	if (F.h_roots[2 + kAccOverflow])
 		return set_error("hd_frame_wait: a level outgrew its bound (internal error)"), HD_ERR_CAPACITY;
 	if (F.cfg.flags & HD_FRAME_GC) { // the captured GC found the filled chain again on the device
-		HD_TRY(hipMemcpy(p.filled.data(), p.d_filled, p.dc.L * 4, hipMemcpyDeviceToHost));
+		std::copy(filled, filled + p.dc.L, p.filled.begin());
 	}
 	if (root_out)
 		*root_out = F.h_roots[0];

@@ -6,6 +6,7 @@
 
 #include <cstdio>
 #include <map>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -56,18 +57,43 @@ struct DevBuf {
 	}
 };
 
-// Named scratch buffers, grown on demand and kept for the pool's lifetime.
+// Named scratch buffers, grown on demand and kept for the pool's lifetime. A sync-free pass's per-level
+// buffers lie in a table for each user of them (a call's 200 names took 60 us to look up).
+constexpr u32 kLevelBufs = 20;
+struct LevelBufs {
+	DevBuf b[HD_MAX_LEVELS][kLevelBufs];
+	void release() {
+		for (auto &l : b)
+			for (DevBuf &x : l)
+				x.release();
+	}
+};
 struct Scratch {
 	std::map<std::string, DevBuf> bufs;
+	std::map<std::string, LevelBufs> levels;
 	template <typename T> int get(const std::string &name, size_t count, T **out) {
-		HD_RET(bufs[name].ensure(count * sizeof(T)));
-		*out = bufs[name].as<T>();
+		DevBuf &b = bufs[name];
+		HD_RET(b.ensure(count * sizeof(T)));
+		*out = b.as<T>();
 		return HD_OK;
+	}
+	u64 held() const {
+		u64 n = 0;
+		for (const auto &kv : bufs)
+			n += kv.second.bytes;
+		for (const auto &kv : levels)
+			for (const auto &l : kv.second.b)
+				for (const DevBuf &x : l)
+					n += x.bytes;
+		return n;
 	}
 	void release() {
 		for (auto &kv : bufs)
 			kv.second.release();
 		bufs.clear();
+		for (auto &kv : levels)
+			kv.second.release();
+		levels.clear();
 	}
 };
 
@@ -82,6 +108,8 @@ enum Meta : u32 {
 // Zero words allocated past the pool so a node can be read whole (up to 9 words) without a
 // bounds test, wherever in the pool it starts.
 constexpr u64 kWordsPad = 16;
+
+constexpr u64 kHostRays = HD_TRAVERSAL_HOST_RAYS;
 
 struct Pool;
 // Device buffers of a node-pool GC (hd_gc.hip), sized by the pool's configuration: per level a
@@ -127,6 +155,10 @@ struct Pool {
 	double last_ms = 0;
 	u32 edit_gen = 0; // generation of the sync-free pass's group table (hd_edit.hip)
 	u32 *h_pass = nullptr; // pinned: a chained pass's counters, read back after its top-down
+	// pinned: hd_traversal_host's rays and hits (kHostRays of them), which the kernel reads and writes in
+	// place; in the same allocation as h_pass. The lock holds for a call.
+	float *h_rays = nullptr;
+	std::mutex rays_mu;
 	GcPlan gc_plan;   // hd_gc's buffers
 };
 

@@ -217,8 +217,9 @@ int hd_pool_create(const hd_config *cfg, hd_pool **out) {
 		return fail(e);
 	if ((e = hipEventCreateWithFlags(&p.ev_pass, hipEventDisableTiming)) != hipSuccess)
 		return fail(e);
-	if ((e = hipHostMalloc((void **)&p.h_pass, 64, hipHostMallocDefault)) != hipSuccess)
+	if ((e = hipHostMalloc((void **)&p.h_pass, 64 + kHostRays * 40, hipHostMallocDefault)) != hipSuccess)
 		return fail(e);
+	p.h_rays = (float *)(p.h_pass + 16);
 	if ((e = hipMalloc(&p.words, (words + kWordsPad) * 4)) != hipSuccess)
 		return fail(e);
 	if ((e = hipMalloc(&p.bucket_words, buckets * 4)) != hipSuccess)

@@ -499,6 +499,41 @@ __global__ void __launch_bounds__(kThreads) k_traversal(const u32 *__restrict__ 
 	out[4 * i + 3] = h.hit ? 1.0f : 0.0f;
 }
 
+// A call's views, tile prefix and beam prefix for the trace kernels: up to kPutViews views go to the device as
+// the arguments of a one-workgroup kernel; more take a copy each. (A small copy from pageable memory holds the
+// host for about 10 us: a 255 x 201 frame 107 -> 102 us.)
+constexpr u32 kPutViews = 16;
+struct PutViews {
+	u32 views[kPutViews * sizeof(hd_view) / 4], tiles[kPutViews + 1], beams[kPutViews + 1];
+};
+__global__ void __launch_bounds__(64) k_put_views(PutViews a, u32 n, u32 *__restrict__ views, u32 *__restrict__ tiles,
+                                                  u32 *__restrict__ beams) {
+	for (u32 i = threadIdx.x; i < n * (u32)(sizeof(hd_view) / 4); i += 64)
+		views[i] = a.views[i];
+	for (u32 i = threadIdx.x; i <= n; i += 64) {
+		tiles[i] = a.tiles[i];
+		if (beams)
+			beams[i] = a.beams[i];
+	}
+}
+static int put_views(hipStream_t s, const hd_view *views, const u32 *tiles, const u32 *beams, u32 n, hd_view *dv, u32 *dt,
+                     u32 *db) {
+	if (n <= kPutViews) {
+		PutViews a;
+		std::memcpy(a.views, views, n * sizeof(hd_view));
+		std::memcpy(a.tiles, tiles, (n + 1) * 4);
+		std::memcpy(a.beams, beams, (n + 1) * 4);
+		k_put_views<<<1, 64, 0, s>>>(a, n, (u32 *)dv, dt, db);
+		HD_TRY(hipGetLastError());
+		return HD_OK;
+	}
+	HD_TRY(hipMemcpyAsync(dv, views, n * sizeof(hd_view), hipMemcpyHostToDevice, s));
+	HD_TRY(hipMemcpyAsync(dt, tiles, (n + 1) * 4, hipMemcpyHostToDevice, s));
+	if (db)
+		HD_TRY(hipMemcpyAsync(db, beams, (n + 1) * 4, hipMemcpyHostToDevice, s));
+	return HD_OK;
+}
+
 // The frame kernel at the tuned tile (tiles counted with the same tile by trace_tile_count).
 // The march keeps one stack word per node level and thread in LDS (pushes and pops stay at scales
 // >= the leaf scale, so the slots are scale - leaf_scale in [0, levels)); sizing the stack to the
@@ -558,13 +593,11 @@ extern "C" int hd_trace(hd_pool *h, uint32_t root, uint32_t color_root, const hd
 	float *beam = nullptr;
 	HD_RET(p.scratch.get<hd_view>("trace_views", n_views, &dv));
 	HD_RET(p.scratch.get<u32>("trace_tiles", n_views + 1, &dt));
-	HD_TRY(hipMemcpyAsync(dv, views, n_views * sizeof(hd_view), hipMemcpyHostToDevice, p.stream));
-	HD_TRY(hipMemcpyAsync(dt, tiles.data(), (n_views + 1) * 4, hipMemcpyHostToDevice, p.stream));
 	if (beams[n_views]) {
 		HD_RET(p.scratch.get<u32>("trace_beam_start", n_views + 1, &db));
 		HD_RET(p.scratch.get<float>("trace_beam", beams[n_views], &beam));
-		HD_TRY(hipMemcpyAsync(db, beams.data(), (n_views + 1) * 4, hipMemcpyHostToDevice, p.stream));
 	}
+	HD_RET(put_views(p.stream, views, tiles.data(), beams.data(), n_views, dv, dt, db));
 	TraceArgs A{p.words, p.cnodes, p.cleaves, root,   color_root, p.dc.L, p.dc.color_leaf,
 	            dv,      dt,       n_views,   rgba, records, nullptr, nullptr, beam, db};
 	if (beams[n_views])
@@ -628,6 +661,25 @@ extern "C" int hd_traversal(hd_pool *h, uint32_t root, const float *o, const flo
 	                                                                                         d, n, out);
 	HD_TRY(hipGetLastError());
 	HD_TRY(hipStreamSynchronize(p.stream));
+	return HD_OK;
+}
+
+// A pick: the kernel reads the rays from pinned host memory and writes the hits there. (Three device
+// allocations, two copies in and one out took 56 of a one-ray call's 82 us: 26 us without them. Each ray
+// crosses the bus once either way.)
+extern "C" int hd_traversal_host(hd_pool *h, uint32_t root, const float *o, const float *d, uint64_t n, float *out) {
+	if (!h || (n && (!o || !d || !out)))
+		return set_error("hd_traversal_host: null argument"), HD_ERR_ARG;
+	if (n > kHostRays)
+		return set_error("hd_traversal_host: %llu rays, at most %llu", (unsigned long long)n,
+		                 (unsigned long long)kHostRays), HD_ERR_CAPACITY;
+	Pool &p = h->p;
+	std::lock_guard<std::mutex> lock(p.rays_mu);
+	float *po = p.h_rays, *pd = po + 3 * kHostRays, *hits = pd + 3 * kHostRays;
+	std::memcpy(po, o, n * 12);
+	std::memcpy(pd, d, n * 12);
+	HD_RET(hd_traversal(h, root, po, pd, n, hits));
+	std::memcpy(out, hits, n * 16);
 	return HD_OK;
 }
 
@@ -704,10 +756,7 @@ extern "C" int hd_trace_noalloc(hd_pool *h, uint32_t root, uint32_t color_root, 
 	hd_view *dv = reinterpret_cast<hd_view *>(base);
 	u32 *dt = base + kNoAllocViewWords, *db = dt + kNoAllocViews + 1;
 	float *beam = reinterpret_cast<float *>(base + kNoAllocBeamOff);
-	HD_TRY(hipMemcpyAsync(dv, views, n_views * sizeof(hd_view), hipMemcpyHostToDevice, p.stream));
-	HD_TRY(hipMemcpyAsync(dt, tiles, (n_views + 1) * 4, hipMemcpyHostToDevice, p.stream));
-	if (n_beam)
-		HD_TRY(hipMemcpyAsync(db, beams, (n_views + 1) * 4, hipMemcpyHostToDevice, p.stream));
+	HD_RET(put_views(p.stream, views, tiles, beams, n_views, dv, dt, n_beam ? db : nullptr));
 	TraceArgs A{p.words, p.cnodes, p.cleaves, root,   color_root,          p.dc.L,         p.dc.color_leaf,
 	            dv,      dt,       n_views,   rgba,   records,             nullptr,        nullptr,
 	            n_beam ? beam : nullptr,     n_beam ? db : nullptr};
