@@ -334,35 +334,56 @@ struct NoiseArgs {
 	double base, lacunarity, gain, norm;
 	u64 consts[32];
 };
+// A wavefront takes 64 columns of kNoiseRun rows at a time: the lattice rows around a point are those of the
+// point before it in all but one of (rows per cell) steps, so a point costs a few of the 24 lattice hashes of six octaves
+// (two 64-bit products each): a 2048^2 field 125 -> 41 us.
 // Grid-stride: the min / max atomics of all workgroups meet on two addresses and take about 10 ns each (one
-// pair per wavefront of a 2048^2 field took 1.3 of the kernel's 1.49 ms; 125 us with a pair per workgroup).
-constexpr u32 kNoiseThreads = 256, kNoiseGrid = 1024;
+// pair per wavefront of a 2048^2 field took 1.3 of the kernel's 1.49 ms; 125 us with a pair per workgroup then).
+constexpr u32 kNoiseThreads = 256, kNoiseGrid = 1024, kNoiseRun = 16;
 __global__ void __launch_bounds__(kNoiseThreads) k_noise(NoiseArgs a, double *__restrict__ acc,
                                                          unsigned long long *__restrict__ minmax) {
-	const u64 n = (u64)a.res * a.res;
+	const u32 side = (a.res + 63u) / 64u, waves = kNoiseThreads / 64;
+	const double inv = 1.0 / (double)a.res; // (a power of two)
 	unsigned long long lo = ~0ull, hi = 0ull;
-	for (u64 i = (u64)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (u64)gridDim.x * blockDim.x) {
-		double v = 0.0;
-		const u32 x = (u32)(i % a.res), y = (u32)(i / a.res);
-		const double xs = ((double)x + 0.5) / (double)a.res, ys = ((double)y + 0.5) / (double)a.res;
-		double amp = 1.0, freq = a.base;
-		for (u32 o = 0; o < a.octaves; ++o) {
-			const double fx = xs * freq, fy = ys * freq;
-			const double ix = floor(fx), iy = floor(fy);
-			double tx = fx - ix, ty = fy - iy;
-			tx = tx * tx * (3.0 - 2.0 * tx);
-			ty = ty * ty * (3.0 - 2.0 * ty);
-			const u64 x0 = (u64)ix, y0 = (u64)iy, c = a.consts[o];
-			const double top = lattice(x0, y0, c) * (1.0 - tx) + lattice(x0 + 1, y0, c) * tx;
-			const double bot = lattice(x0, y0 + 1, c) * (1.0 - tx) + lattice(x0 + 1, y0 + 1, c) * tx;
-			v = v + amp * (top * (1.0 - ty) + bot * ty);
-			amp *= a.gain;
-			freq *= a.lacunarity;
+	for (u64 t = blockIdx.x; t < (u64)side * side; t += gridDim.x) { // tiles of 64 x 64
+		const u32 x = (u32)(t % side) * 64u + (threadIdx.x & 63u);
+		const double xs = ((double)x + 0.5) * inv;
+		for (u32 y0 = (u32)(t / side) * 64u + (threadIdx.x >> 6) * kNoiseRun; y0 < (u32)(t / side + 1u) * 64u && y0 < a.res;
+		     y0 += waves * kNoiseRun) {
+			double v[kNoiseRun], amp = 1.0, freq = a.base;
+#pragma unroll
+			for (u32 k = 0; k < kNoiseRun; ++k)
+				v[k] = 0.0;
+			for (u32 o = 0; o < a.octaves; ++o) {
+				const double fx = xs * freq, ix = floor(fx);
+				double tx = fx - ix, cell = -1.0, top = 0.0, bot = 0.0;
+				tx = tx * tx * (3.0 - 2.0 * tx);
+				const u64 cx = (u64)ix, c = a.consts[o];
+				auto row = [&](u64 cy) { return lattice(cx, cy, c) * (1.0 - tx) + lattice(cx + 1, cy, c) * tx; };
+#pragma unroll
+				for (u32 k = 0; k < kNoiseRun; ++k) {
+					const double fy = ((double)(y0 + k) + 0.5) * inv * freq, iy = floor(fy);
+					double ty = fy - iy;
+					ty = ty * ty * (3.0 - 2.0 * ty);
+					if (iy != cell) { // (the same for the wavefront)
+						top = iy == cell + 1.0 && cell >= 0.0 ? bot : row((u64)iy);
+						bot = row((u64)iy + 1);
+						cell = iy;
+					}
+					v[k] = v[k] + amp * (top * (1.0 - ty) + bot * ty);
+				}
+				amp *= a.gain;
+				freq *= a.lacunarity;
+			}
+#pragma unroll
+			for (u32 k = 0; k < kNoiseRun; ++k)
+				if (x < a.res && y0 + k < a.res) {
+					const double w = v[k] / a.norm;
+					acc[(u64)(y0 + k) * a.res + x] = w;
+					lo = min(lo, (unsigned long long)__double_as_longlong(w));
+					hi = max(hi, (unsigned long long)__double_as_longlong(w));
+				}
 		}
-		v = v / a.norm;
-		acc[i] = v;
-		lo = min(lo, (unsigned long long)__double_as_longlong(v));
-		hi = max(hi, (unsigned long long)__double_as_longlong(v));
 	}
 	// non-negative doubles order like their bit patterns: the workgroup's min / max, then one atomic each
 	for (u32 d = 32; d >= 1; d >>= 1) {
@@ -430,7 +451,8 @@ extern "C" int hd_pool_value_noise_heightmap(hd_pool *h, uint32_t octaves, uint6
 			break;
 	}
 	HD_RET(heightmap_buffers(p, total));
-	k_noise<<<std::min(div_up(n, kNoiseThreads), kNoiseGrid), kNoiseThreads, 0, p.stream>>>(a, acc, mm);
+	const u32 side = div_up(res, 64);
+	k_noise<<<(u32)std::min<u64>((u64)side * side, kNoiseGrid), kNoiseThreads, 0, p.stream>>>(a, acc, mm);
 	HD_TRY(hipGetLastError());
 	k_noise_heights<<<div_up(n, 256), 256, 0, p.stream>>>(res, zlo, zhi, acc, mm, p.hm_mn, p.hm_mx);
 	HD_TRY(hipGetLastError());
