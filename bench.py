@@ -660,7 +660,7 @@ def edit_roofline(args, edit_gpu_ms):
             "traffic_source": EDIT_TRAFFIC_PROFILE if tr.get("traffic_bytes_per_step") else None,
             "algorithmic_bytes_per_step": per_step_bytes, "algorithmic_source": EDIT_BYTES_PROFILE,
             "device_ms_per_step": t * 1e3,
-            "note": "latency-bound: ~10 dependent launches per edit, each a few memory round trips"}
+            "note": "latency-bound: about 40 dependent launches per pass of some 30 edits, each a few memory round trips"}
 
 
 TRAFFIC_PROFILE = "profiles/k_trace_4096_terrain_1080p.md"

@@ -153,9 +153,11 @@ int hd_pool_clear_overflow(hd_pool *pool);
 
 /* Edit modes. */
 enum {
-	HD_MODE_PLAIN = 0,  /* one level-synchronous pass per edit, edits applied in order: the result
-	                       (pool words, bucket counters, color arrays, roots) equals NodePoolBase::Edit
-	                       applied to each edit in turn (NodePool.hpp:405-417) */
+	HD_MODE_PLAIN = 0,  /* edits applied in order: the result (pool words, bucket counters, color arrays,
+	                       roots) equals NodePoolBase::Edit applied to each edit in turn
+	                       (NodePool.hpp:405-417). Runs of consecutive edits that share no color leaf go
+	                       through one level-synchronous pass that keeps a version of each node per edit;
+	                       the others take a pass each */
 	HD_MODE_BATCHED = 1 /* folded passes: runs of up to 4096 consecutive edits, overlapping ones
 	                       included, each applied by one level-synchronous pass whose nodes carry the
 	                       edits that touch them in submission order, folded from the last edit that

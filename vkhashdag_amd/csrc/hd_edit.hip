@@ -7,7 +7,8 @@
 //   top-down   k_root, then per level k_expand (one lane per (node, child): classify with the
 //              editor, fill / clear / keep / proceed) + stable compaction (k_emit) so every level's
 //              frontier is in the reference's DFS order;
-//   leaves     k_leaf: one wavefront per 4^3 leaf, one lane per voxel, __ballot builds the mask;
+//   leaves     k_leaf: one wavefront per 4^3 leaf, one lane per voxel, __ballot builds the mask (a_leaf
+//              of the sync-free passes: 16 lanes, four voxels each);
 //   bottom-up  k_build packs changed inner nodes; k_dedup / k_find / stable sort by bucket /
 //              k_append / k_resolve give find-or-insert whose appends land in each bucket in DFS
 //              order -- the pool words equal the reference's single-threaded Edit;
