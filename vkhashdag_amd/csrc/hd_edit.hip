@@ -810,7 +810,9 @@ constexpr u32 kAT = 256;       // threads per block of the sync-free kernels
 constexpr u32 kTopPairs = 4096; // a level whose 8 n pairs fit this bound expands inside a_top
 constexpr u32 kGather = 32;    // bucket lists up to this length are sorted in registers
 constexpr u32 kWalkList = 64;  // groups per bucket listed by arrival for the walker
-constexpr u32 kWalkShort = 16; // at most this many: one thread walks the bucket from registers
+// At most this many: one thread walks the bucket from registers; more take the wavefront (4096 mixed edits in a
+// changed world, the walks of a pass: 16 2.13 ms, 8 1.42 ms, 4 1.22 ms; of 256 edits 12.8, -, 12.4 us each).
+constexpr u32 kWalkShort = 4;
 
 struct Pair {
 	u32 a, b;
@@ -2564,9 +2566,7 @@ __device__ inline u32 walk_entry(const EditParams &P, u32 l, const ALevel &A, co
 	const u32 b = A.bucket[e], k = bcnt[b];
 	const u32 bw0 = ldg(P.bucket_words, b);
 	u32 appended = 0;
-	if (k <= 4u)
-		appended = walk_short<4>(P, leaf, A, G, b, k, bw0, blist);
-	else if (k <= kWalkShort)
+	if (k <= kWalkShort)
 		appended = walk_short<kWalkShort>(P, leaf, A, G, b, k, bw0, blist);
 	else if (k <= kWalkList) {
 		wb = b, wk = k;
