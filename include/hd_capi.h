@@ -180,6 +180,11 @@ int hd_edit(hd_pool *pool, uint32_t root, uint32_t color_root, const hd_edit_des
  * for serving loops that must not stall on device allocation. Blocking. */
 int hd_edit_reserve(hd_pool *pool, const hd_edit_desc *edits, uint32_t n, uint32_t mode);
 
+/* The passes that a plain hd_edit of these edits is planned as on a pool of this configuration that holds no
+ * buffers yet: counts[k] (room for n) consecutive edits each, *n_passes of them; more than one edit: a pass of
+ * versions. What the world holds may split such a pass further. Works without a device. */
+int hd_edit_plan(const hd_config *cfg, const hd_edit_desc *edits, uint32_t n, uint32_t *counts, uint32_t *n_passes);
+
 /* Editor decisions: hashdag::EditType (Editor.hpp:18), same order. */
 enum { HD_EDIT_TYPE_NOT_AFFECTED = 0, HD_EDIT_TYPE_PROCEED = 1, HD_EDIT_TYPE_FILL = 2, HD_EDIT_TYPE_CLEAR = 3 };
 

@@ -116,6 +116,7 @@ def lib():
             "hd_pool_clear_overflow": (C.c_int, [VP]),
             "hd_edit": (C.c_int, [VP, U32, U32, VP, U32, U32, P32, P32]),
             "hd_edit_reserve": (C.c_int, [VP, VP, U32, U32]),
+            "hd_edit_plan": (C.c_int, [VP, VP, U32, VP, C.POINTER(U32)]),
             "hd_gc": (C.c_int, [VP, VP, U32]),
             "hd_edit_host": (C.c_int, [VP, U32, C.POINTER(hd_host_editor), P32]),
             "hd_trace": (C.c_int, [VP, U32, U32, VP, U32, VP, VP]),
@@ -204,21 +205,34 @@ def make_view(vb, width, height, flags=0, out_offset=0) -> hd_view:
     return v
 
 
+def _config(cfg: PoolConfig) -> hd_config:
+    c = hd_config()
+    c.word_bits_per_page = cfg.word_bits_per_page
+    c.page_bits_per_bucket = cfg.page_bits_per_bucket
+    c.node_levels = cfg.node_levels
+    for i, b in enumerate(cfg.bucket_bits):
+        c.bucket_bits[i] = b
+    c.color_leaf_level = cfg.color_leaf_level
+    c.color_keep_history = int(cfg.keep_history)
+    c.color_node_capacity = cfg.color_node_capacity
+    c.color_leaf_capacity = cfg.color_leaf_capacity
+    return c
+
+
+def edit_plan(cfg: PoolConfig, edits) -> list:
+    """hd_edit_plan: how many consecutive edits each pass of a plain call takes. Needs no device."""
+    e = np.ascontiguousarray(np.atleast_1d(edits).astype(EDIT_DTYPE))
+    counts, n = np.zeros(max(len(e), 1), np.uint32), U32(0)
+    check(lib().hd_edit_plan(C.byref(_config(cfg)), e.ctypes.data, len(e), counts.ctypes.data, C.byref(n)))
+    return [int(k) for k in counts[: n.value]]
+
+
 class DevicePool:
     """A device-resident HashDAG node pool + color pool (DAGNodePool + DAGColorPool semantics)."""
 
     def __init__(self, cfg: PoolConfig, heights=None):
         self.cfg = cfg
-        c = hd_config()
-        c.word_bits_per_page = cfg.word_bits_per_page
-        c.page_bits_per_bucket = cfg.page_bits_per_bucket
-        c.node_levels = cfg.node_levels
-        for i, b in enumerate(cfg.bucket_bits):
-            c.bucket_bits[i] = b
-        c.color_leaf_level = cfg.color_leaf_level
-        c.color_keep_history = int(cfg.keep_history)
-        c.color_node_capacity = cfg.color_node_capacity
-        c.color_leaf_capacity = cfg.color_leaf_capacity
+        c = _config(cfg)
         h = VP()
         check(lib().hd_pool_create(C.byref(c), C.byref(h)))
         self.h = h.value

@@ -6197,9 +6197,10 @@ static void batched_plans(const Pool &p, const hd_edit_desc *edits, u32 n, std::
 			plans.push_back(pp);
 		}
 }
-// Whether an edit may share a chained pass at all: no column fill, colors (if any) plain RGB8.
+// Whether an edit may share a chained pass at all: no column fill, colors (if any) plain RGB8, and inner
+// levels to link versions of (in a pool of one level the root is a leaf, which no two edits may share).
 static bool chains(const Pool &p, const hd_edit_desc &d) {
-	if (d.kind == HD_EDIT_COLUMN_FILL)
+	if (d.kind == HD_EDIT_COLUMN_FILL || p.dc.L < 2)
 		return false;
 	return !is_stateful(d) || (d.color.has_value && !d.color.bits_per_weight && lds_jobs(p.dc) && p.dc.color_leaf > 0);
 }
@@ -6702,6 +6703,21 @@ extern "C" int hd_edit_reserve(hd_pool *h, const hd_edit_desc *edits, uint32_t n
 			return set_error("edit %u: bits_per_weight %u > 3", i, edits[i].color.bits_per_weight), HD_ERR_ARG;
 	}
 	return edit_reserve(h->p, edits, n, mode);
+}
+
+extern "C" int hd_edit_plan(const hd_config *cfg, const hd_edit_desc *edits, uint32_t n, uint32_t *counts,
+                            uint32_t *n_passes) {
+	if (!cfg || (n && (!edits || !counts)) || !n_passes)
+		return set_error("hd_edit_plan: null argument"), HD_ERR_ARG;
+	Pool p;
+	HD_RET(set_config(p, *cfg));
+	std::vector<hd_edit_desc> flat;
+	std::vector<PassPlan> plans;
+	plain_plans(p, edits, n, flat, plans);
+	*n_passes = (uint32_t)plans.size();
+	for (size_t k = 0; k < plans.size(); ++k)
+		counts[k] = plans[k].count;
+	return HD_OK;
 }
 
 // ---- frames (hipGraph): the C-ABI

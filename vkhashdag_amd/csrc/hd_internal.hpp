@@ -172,6 +172,7 @@ struct Tuning {
 };
 extern Tuning g_tuning; // hd_pool.hip
 
+int set_config(Pool &p, const hd_config &cfg); // hd_pool.hip: checks it and takes it over, no device
 int make_filled(Pool &p);               // hd_pool.hip
 void launch_refill(Pool &p, hipStream_t s); // hd_pool.hip: the chain found again when d_filled misses a node, queued only
 // A whole GC queued on stream s over device roots (remapped in place); the filled chain is a root

@@ -149,6 +149,42 @@ static int live_offsets(Pool &p, u64 **d_off, u64 *total) {
 	return HD_OK;
 }
 
+// Checks a configuration and takes it over (no device).
+int set_config(Pool &p, const hd_config &cfg) {
+	if (cfg.node_levels == 0 || cfg.node_levels > HD_MAX_LEVELS - 1 || cfg.word_bits_per_page < 4 ||
+	    cfg.color_leaf_level > cfg.node_levels - 1 || cfg.node_levels + 1 > 22)
+		return set_error("invalid hd_config"), HD_ERR_ARG;
+	u64 buckets = 0;
+	for (u32 l = 0; l < cfg.node_levels; ++l) {
+		if (cfg.bucket_bits[l] > 30)
+			return set_error("bucket_bits too large"), HD_ERR_ARG;
+		buckets += 1ull << cfg.bucket_bits[l];
+	}
+	u64 words = buckets << (cfg.word_bits_per_page + cfg.page_bits_per_bucket);
+	if (words - 1 > 0xFFFFFFFEull) // Config::Validate (Config.hpp:48-56)
+		return set_error("pool exceeds 2^32-1 words"), HD_ERR_ARG;
+	if (cfg.color_node_capacity >= (1ull << 30) - 1 || cfg.color_leaf_capacity > (1ull << 30))
+		return set_error("color capacities exceed 30-bit color pointers (DAGColorPool.hpp:24)"), HD_ERR_ARG;
+	p.cfg = cfg;
+	p.dc.wbpp = cfg.word_bits_per_page;
+	p.dc.pbpb = cfg.page_bits_per_bucket;
+	p.dc.L = cfg.node_levels;
+	p.dc.color_leaf = cfg.color_leaf_level;
+	p.dc.voxel_level = cfg.node_levels + 1;
+	p.dc.keep_history = cfg.color_keep_history;
+	u32 base = 0;
+	for (u32 l = 0; l < cfg.node_levels; ++l) {
+		p.dc.bucket_bits[l] = cfg.bucket_bits[l];
+		p.dc.level_base[l] = base;
+		base += 1u << cfg.bucket_bits[l];
+	}
+	p.total_buckets = buckets;
+	p.total_words = words;
+	p.cnode_cap = cfg.color_node_capacity;
+	p.cleaf_cap = cfg.color_leaf_capacity;
+	return HD_OK;
+}
+
 } // namespace hd
 
 using namespace hd;
@@ -158,47 +194,15 @@ extern "C" {
 const char *hd_last_error(void) { return g_err; }
 
 int hd_pool_create(const hd_config *cfg, hd_pool **out) {
-	if (!cfg || !out || cfg->node_levels == 0 || cfg->node_levels > HD_MAX_LEVELS - 1 || cfg->word_bits_per_page < 4 ||
-	    cfg->color_leaf_level > cfg->node_levels - 1 || cfg->node_levels + 1 > 22) {
-		set_error("invalid hd_config");
-		return HD_ERR_ARG;
-	}
-	u64 buckets = 0;
-	for (u32 l = 0; l < cfg->node_levels; ++l) {
-		if (cfg->bucket_bits[l] > 30) {
-			set_error("bucket_bits too large");
-			return HD_ERR_ARG;
-		}
-		buckets += 1ull << cfg->bucket_bits[l];
-	}
-	u64 words = buckets << (cfg->word_bits_per_page + cfg->page_bits_per_bucket);
-	if (words - 1 > 0xFFFFFFFEull) { // Config::Validate (Config.hpp:48-56)
-		set_error("pool exceeds 2^32-1 words");
-		return HD_ERR_ARG;
-	}
-	if (cfg->color_node_capacity >= (1ull << 30) - 1 || cfg->color_leaf_capacity > (1ull << 30)) {
-		set_error("color capacities exceed 30-bit color pointers (DAGColorPool.hpp:24)");
-		return HD_ERR_ARG;
-	}
+	if (!cfg || !out)
+		return set_error("invalid hd_config"), HD_ERR_ARG;
 	auto *h = new hd_pool();
 	Pool &p = h->p;
-	p.cfg = *cfg;
-	p.dc.wbpp = cfg->word_bits_per_page;
-	p.dc.pbpb = cfg->page_bits_per_bucket;
-	p.dc.L = cfg->node_levels;
-	p.dc.color_leaf = cfg->color_leaf_level;
-	p.dc.voxel_level = cfg->node_levels + 1;
-	p.dc.keep_history = cfg->color_keep_history;
-	u32 base = 0;
-	for (u32 l = 0; l < cfg->node_levels; ++l) {
-		p.dc.bucket_bits[l] = cfg->bucket_bits[l];
-		p.dc.level_base[l] = base;
-		base += 1u << cfg->bucket_bits[l];
+	if (const int rc = set_config(p, *cfg); rc != HD_OK) {
+		delete h;
+		return rc;
 	}
-	p.total_buckets = buckets;
-	p.total_words = words;
-	p.cnode_cap = cfg->color_node_capacity;
-	p.cleaf_cap = cfg->color_leaf_capacity;
+	const u64 words = p.total_words, buckets = p.total_buckets;
 	auto fail = [&](hipError_t e) {
 		set_error("hd_pool_create: %s", hipGetErrorString(e));
 		hd_pool_destroy(h);
