@@ -31,7 +31,7 @@ namespace {
 
 constexpr u32 kGcThreads = 256;
 constexpr u32 kGcGrid = 2048;    // workgroups of the grid-stride kernels (bounded dispatch)
-constexpr u32 kGcSortCap = 1024; // nodes a bucket can receive without overflowing (2-word nodes)
+constexpr u32 kGcSortCap = 1024; // nodes that a wavefront sorts in LDS
 
 __device__ inline u32 low_mask(u32 k) { return k >= 32u ? ~0u : ((1u << k) - 1u); }
 
@@ -194,17 +194,20 @@ __global__ void k_gc_pack_leaves(u32 *__restrict__ words, u32 *__restrict__ buck
 	}
 	bucket_words[gb] = bw;
 }
+// The nodes that a new bucket of a level receives, in the order of arrival: the first cap in a list of the
+// bucket's own, the others in a chain (head: the latest one's old offset + 1; next, at half its old offset: the
+// one before it). cap is what a bucket of 2-word nodes holds, so only a bucket that overflows has a chain.
+struct GcLists {
+	u32 cap, *cnt, *head, *list, *next;
+};
 // The live nodes of an inner level: each one's children remapped (cnewp: the new pointers of the level
 // below), the node written to the stage at its old offset (the pack rewrites the pool's words in place),
-// re-hashed (:147-148) and listed in its new bucket, unordered (cap entries per bucket; more 2-word
-// nodes than the bucket holds: the reference's cache overflows). Thread 0 moves the filled chain's
-// entry of the level below.
+// re-hashed (:147-148) and listed in its new bucket, unordered. Thread 0 moves the filled chain's entry of
+// the level below.
 __global__ void __launch_bounds__(kGcThreads) k_gc_key(const u32 *__restrict__ words, const u32 *__restrict__ bits,
                                                        const u32 *__restrict__ bucket_words, DevConfig c, u32 level,
                                                        u64 base, u64 cbase, u64 cwords, const u32 *__restrict__ cnewp,
-                                                       u32 cap, u32 *__restrict__ stage, u32 *__restrict__ cnt,
-                                                       u32 *__restrict__ list, u32 *__restrict__ newp,
-                                                       u32 *__restrict__ filled, u32 *__restrict__ meta) {
+                                                       u32 *__restrict__ stage, GcLists B, u32 *__restrict__ filled) {
 	if ((threadIdx.x | blockIdx.x) == 0 && filled) {
 		const u64 o = (u64)filled[level + 1u] - cbase;
 		if (o < cwords)
@@ -226,17 +229,15 @@ __global__ void __launch_bounds__(kGcThreads) k_gc_key(const u32 *__restrict__ w
 		for (u32 j = 0; j < 8; ++j)
 			buf[j + 1] = np[j];
 		const u32 kb = murmur_regs(buf, k + 1u) & ((1u << c.bucket_bits[level]) - 1u);
-		const u32 lp = atomicAdd(&cnt[kb], 1u);
+		const u32 lp = atomicAdd(&B.cnt[kb], 1u);
 #pragma unroll
 		for (u32 j = 0; j < 9; ++j)
 			if (j <= k)
 				stage[(u64)o + j] = buf[j];
-		if (lp < cap)
-			list[(u64)kb * cap + lp] = o;
-		else {
-			newp[o >> 1] = kNull;
-			atomicOr(&meta[kMetaOverflow], 4u);
-		}
+		if (lp < B.cap)
+			B.list[(u64)kb * B.cap + lp] = o;
+		else
+			B.next[o >> 1] = atomicExch(&B.head[kb], o + 1u);
 	});
 }
 // One node of a new bucket written at word `at` of the bucket (kNull: the bucket was full).
@@ -306,21 +307,22 @@ __device__ inline u32 gc_pack_small(u32 *__restrict__ words, const DevConfig &c,
 		gc_place(words, stage, wbase, o, sz, at, newp);
 	return bw;
 }
-// A bucket of 65 to kGcSortCap nodes (one wavefront): bitonic sort in LDS (so / sp), places one by one.
-__device__ inline u32 gc_pack_large(u32 *__restrict__ words, const DevConfig &c, const u32 *__restrict__ stage, u64 wbase,
-                                    u32 m, const u32 *__restrict__ list, u32 *__restrict__ newp, u32 *__restrict__ meta,
-                                    u32 lane, u32 *so, u32 *sp) {
-	__builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-	__builtin_amdgcn_wave_barrier(); // the previous bucket's readers of so / sp are done
-	__builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-	u32 P = 1;
-	while (P < m)
-		P <<= 1;
-	for (u32 k = lane; k < P; k += 64)
-		so[k] = k < m ? list[k] : ~0u;
+__device__ inline void gc_wave_sync() {
 	__builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
 	__builtin_amdgcn_wave_barrier();
 	__builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+// The m nodes in so (LDS, at most kGcSortCap; one wavefront) into a bucket filled to bw: bitonic sort,
+// places one by one (sp). Returns what the bucket is filled to.
+__device__ inline u32 gc_pack_sorted(u32 *__restrict__ words, const DevConfig &c, const u32 *__restrict__ stage, u64 wbase,
+                                     u32 m, u32 bw, u32 *__restrict__ newp, u32 *__restrict__ meta, u32 lane, u32 *so,
+                                     u32 *sp) {
+	u32 P = 1;
+	while (P < m)
+		P <<= 1;
+	for (u32 k = m + lane; k < P; k += 64)
+		so[k] = ~0u;
+	gc_wave_sync();
 	for (u32 size = 2; size <= P; size <<= 1) // bitonic sort, ascending
 		for (u32 stride = size >> 1; stride > 0; stride >>= 1) {
 			for (u32 k = lane; k < P; k += 64) {
@@ -334,16 +336,11 @@ __device__ inline u32 gc_pack_large(u32 *__restrict__ words, const DevConfig &c,
 					}
 				}
 			}
-			__builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-			__builtin_amdgcn_wave_barrier();
-			__builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+			gc_wave_sync();
 		}
 	for (u32 k = lane; k < m; k += 64)
 		sp[k] = (u32)__builtin_popcount(stage[so[k]] & 0xFFu) + 1u; // node sizes
-	__builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-	__builtin_amdgcn_wave_barrier();
-	__builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-	u32 bw = 0;
+	gc_wave_sync();
 	if (lane == 0) { // positions in pointer order; a page tail a node skips is zero (the cache's resize)
 		for (u32 k = 0; k < m; ++k) {
 			const u32 sz = sp[k], at = gc_next(c, bw, sz);
@@ -357,12 +354,62 @@ __device__ inline u32 gc_pack_large(u32 *__restrict__ words, const DevConfig &c,
 			bw = at + sz;
 		}
 	}
-	__builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-	__builtin_amdgcn_wave_barrier();
-	__builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+	gc_wave_sync();
 	for (u32 k = lane; k < m; k += 64)
 		gc_place(words, stage, wbase, so[k], (u32)__builtin_popcount(stage[so[k]] & 0xFFu) + 1u, sp[k], newp);
 	return __builtin_amdgcn_readfirstlane(bw);
+}
+// A bucket of 65 to kGcSortCap listed nodes (one wavefront).
+__device__ inline u32 gc_pack_large(u32 *__restrict__ words, const DevConfig &c, const u32 *__restrict__ stage, u64 wbase,
+                                    u32 m, const u32 *__restrict__ list, u32 *__restrict__ newp, u32 *__restrict__ meta,
+                                    u32 lane, u32 *so, u32 *sp) {
+	gc_wave_sync(); // the previous bucket's readers of so / sp are done
+	for (u32 k = lane; k < m; k += 64)
+		so[k] = list[k];
+	return gc_pack_sorted(words, c, stage, wbase, m, 0u, newp, meta, lane, so, sp);
+}
+// Any number of nodes, listed and chained (one wavefront): range after range of old offsets, each narrow
+// enough for the LDS sort. level_words: the offsets lie below it.
+__device__ inline u32 gc_pack_ranges(u32 *__restrict__ words, const DevConfig &c, const u32 *__restrict__ stage, u64 wbase,
+                                     u32 m, const u32 *__restrict__ list, const GcLists &B, u32 head, u64 level_words,
+                                     u32 *__restrict__ newp, u32 *__restrict__ meta, u32 lane, u32 *so, u32 *sp) {
+	u64 width = level_words;
+	for (u32 k = m; k > kGcSortCap / 2u; k >>= 1)
+		width >>= 1;
+	u32 bw = 0, left = m;
+	for (u64 lo = 0; left && lo < level_words;) {
+		// (nodes are two words or more, so a range of 2 kGcSortCap offsets always fits)
+		width = max(width, (u64)kGcSortCap);
+		u32 n = 0;
+		gc_wave_sync();
+		for (u32 k0 = 0; k0 < min(m, B.cap); k0 += 64u) {
+			const u32 k = k0 + lane, o = k < min(m, B.cap) ? list[k] : 0u;
+			const bool in = k < min(m, B.cap) && o >= lo && o < lo + width;
+			const u64 b = __ballot(in);
+			const u32 at = n + (u32)__popcll(b & ((1ull << lane) - 1ull));
+			if (in && at < kGcSortCap)
+				so[at] = o;
+			n += (u32)__popcll(b);
+		}
+		for (u32 q = head; q; q = B.next[(q - 1u) >> 1]) { // (the same on every lane)
+			const u32 o = q - 1u;
+			if (o >= lo && o < lo + width) {
+				if (lane == 0 && n < kGcSortCap)
+					so[n] = o;
+				++n;
+			}
+		}
+		if (n > kGcSortCap) {
+			width >>= 1;
+			continue;
+		}
+		if (n)
+			bw = gc_pack_sorted(words, c, stage, wbase, n, bw, newp, meta, lane, so, sp);
+		left -= n;
+		lo += width;
+		width = min(2u * width, level_words);
+	}
+	return bw;
 }
 // The new buckets of an inner level, kPackBuckets per wavefront: their nodes sorted by old pointer,
 // placed one after another with page-tail padding (lf_gc_shrink_inner_bucket's cache, :105-182, and
@@ -370,31 +417,38 @@ __device__ inline u32 gc_pack_large(u32 *__restrict__ words, const DevConfig &c,
 // count cleared for the next level. The wave reads its buckets' counts at once and skips the empty ones.
 constexpr u32 kPackBuckets = 4;
 __global__ void __launch_bounds__(kGcThreads) k_gc_pack_inner(u32 *__restrict__ words, u32 *__restrict__ bucket_words,
-                                                              DevConfig c, u32 level, u32 cap,
-                                                              const u32 *__restrict__ stage, u32 *__restrict__ cnt,
-                                                              const u32 *__restrict__ list, u32 *__restrict__ newp,
-                                                              u32 *__restrict__ meta) {
+                                                              DevConfig c, u32 level, const u32 *__restrict__ stage,
+                                                              GcLists B, u32 *__restrict__ newp, u32 *__restrict__ meta) {
 	__shared__ u32 s_off[kGcThreads / 64][kGcSortCap];
 	__shared__ u32 s_pos[kGcThreads / 64][kGcSortCap];
 	const u32 lane = threadIdx.x & 63u, w = threadIdx.x >> 6, nb = 1u << c.bucket_bits[level];
 	for (u64 b0 = ((u64)blockIdx.x * (kGcThreads / 64) + w) * kPackBuckets; b0 < nb;
 	     b0 += (u64)gridDim.x * (kGcThreads / 64) * kPackBuckets) {
 		const bool in = lane < kPackBuckets && b0 + lane < nb;
-		const u32 mm = in ? min(cnt[b0 + lane], cap) : 0u;
+		const u32 mm = in ? B.cnt[b0 + lane] : 0u;
 		u32 bw = 0;
 		for (u64 todo = __ballot(mm != 0u); todo; todo &= todo - 1ull) {
 			const int k = __builtin_ctzll(todo);
 			const u32 m = (u32)__builtin_amdgcn_readlane((int)mm, k), b = (u32)b0 + (u32)k;
 			const u64 wbase = (u64)(c.level_base[level] + b) << c.wbpb();
-			const u32 *ls = list + (u64)b * cap;
-			const u32 r = m <= 64u ? gc_pack_small(words, c, stage, wbase, m, ls, newp, meta, lane)
-			                       : gc_pack_large(words, c, stage, wbase, m, ls, newp, meta, lane, s_off[w], s_pos[w]);
+			const u32 *ls = B.list + (u64)b * B.cap;
+			u32 r;
+			if (m <= min(64u, B.cap))
+				r = gc_pack_small(words, c, stage, wbase, m, ls, newp, meta, lane);
+			else if (m <= min(kGcSortCap, B.cap))
+				r = gc_pack_large(words, c, stage, wbase, m, ls, newp, meta, lane, s_off[w], s_pos[w]);
+			else {
+				r = gc_pack_ranges(words, c, stage, wbase, m, ls, B, m > B.cap ? B.head[b] : 0u,
+				                   1ull << (c.bucket_bits[level] + c.wbpb()), newp, meta, lane, s_off[w], s_pos[w]);
+				if (lane == 0)
+					B.head[b] = 0u;
+			}
 			bw = (int)lane == k ? r : bw;
 		}
 		if (in) {
 			bucket_words[c.level_base[level] + b0 + lane] = bw;
 			if (mm)
-				cnt[b0 + lane] = 0u;
+				B.cnt[b0 + lane] = 0u;
 		}
 	}
 }
@@ -427,13 +481,13 @@ int GcPlan::prepare(Pool &p, const char *prefix) {
 		max_words = std::max(max_words, V.words);
 		max_buckets = std::max(max_buckets, V.buckets);
 	}
-	// a bucket holds at most wpb / 2 nodes: a list of min(kGcSortCap, wpb) tells an overflowing one
-	cap = std::min(kGcSortCap, wpb);
+	cap = wpb / 2; // (of 2-word nodes)
 	HD_RET(p.scratch.get<u32>(pre + "gc_newp0", max_words / 2 + 1, &newp[0]));
 	HD_RET(p.scratch.get<u32>(pre + "gc_newp1", max_words / 2 + 1, &newp[1]));
 	HD_RET(p.scratch.get<u32>(pre + "gc_stage", max_words + 16, &stage));
 	HD_RET(p.scratch.get<u32>(pre + "gc_list", max_buckets * cap, &list));
-	HD_RET(p.scratch.get<u32>(pre + "gc_cnt", max_buckets, &cnt));
+	HD_RET(p.scratch.get<u32>(pre + "gc_next", max_words / 2 + 1, &next));
+	HD_RET(p.scratch.get<u32>(pre + "gc_cnt", 2 * max_buckets, &cnt)); // and the chains' heads
 	return HD_OK;
 }
 
@@ -449,7 +503,7 @@ int gc_queue(Pool &p, const GcPlan &G, hipStream_t s, u32 *d_roots, u32 n_roots,
 		max_buckets = std::max(max_buckets, G.lv[l].buckets);
 	}
 	k_gc_clear<<<std::min(grid(p.total_buckets), kGcGrid), kGcThreads, 0, s>>>(p.bucket_words, p.dc, p.total_buckets, B,
-	                                                                          G.cnt, max_buckets);
+	                                                                          G.cnt, 2 * max_buckets);
 	k_gc_mark_roots<<<grid(n_roots + L), kGcThreads, 0, s>>>(d_roots, n_roots, has_filled ? p.d_filled : nullptr, p.dc, B);
 	auto waves = [&](u32 l) { return std::min(grid(G.lv[l].buckets / kWaveBuckets * 64), kGcGrid); };
 	for (u32 l = 0; l + 1 < L; ++l) {
@@ -459,14 +513,15 @@ int gc_queue(Pool &p, const GcPlan &G, hipStream_t s, u32 *d_roots, u32 n_roots,
 	}
 	k_gc_pack_leaves<<<grid(G.lv[L - 1].buckets), kGcThreads, 0, s>>>(p.words, p.bucket_words, p.dc, L - 1,
 	                                                                 G.lv[L - 1].bits, G.newp[(L - 1) & 1], p.meta);
+	const GcLists lists{G.cap, G.cnt, G.cnt + max_buckets, G.list, G.next};
 	for (int l = (int)L - 2; l >= 0; --l) {
 		const GcPlan::Level &V = G.lv[l], &C = G.lv[l + 1];
 		u32 *newp = G.newp[l & 1];
 		k_gc_key<<<waves((u32)l), kGcThreads, 0, s>>>(p.words, V.bits, p.bucket_words, p.dc, (u32)l, V.base, C.base,
-		                                              C.words, G.newp[(l + 1) & 1], G.cap, G.stage, G.cnt, G.list, newp,
-		                                              has_filled ? p.d_filled : nullptr, p.meta);
+		                                              C.words, G.newp[(l + 1) & 1], G.stage, lists,
+		                                              has_filled ? p.d_filled : nullptr);
 		k_gc_pack_inner<<<grid((V.buckets + kPackBuckets - 1) / kPackBuckets * 64), kGcThreads, 0, s>>>(
-		    p.words, p.bucket_words, p.dc, (u32)l, G.cap, G.stage, G.cnt, G.list, newp, p.meta);
+		    p.words, p.bucket_words, p.dc, (u32)l, G.stage, lists, newp, p.meta);
 	}
 	k_gc_roots<<<grid(n_roots + 1), kGcThreads, 0, s>>>(d_roots, n_roots, has_filled ? p.d_filled : nullptr, G.newp[0],
 	                                                    G.lv[0].base, G.lv[0].words);

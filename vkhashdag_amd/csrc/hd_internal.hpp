@@ -114,8 +114,8 @@ constexpr u64 kHostRays = HD_TRAVERSAL_HOST_RAYS;
 struct Pool;
 // Device buffers of a node-pool GC (hd_gc.hip), sized by the pool's configuration: per level a
 // bitmap of live node starts over the level's words; new pointers at half the old offset for two
-// adjacent levels; one level's remapped nodes, the new buckets' node lists (cap entries each) and
-// counts.
+// adjacent levels; one level's remapped nodes, the new buckets' node lists (cap entries each), the chains of
+// what exceeds them, counts and the chains' heads.
 struct GcPlan {
 	struct Level {
 		u32 *bits = nullptr;
@@ -123,7 +123,7 @@ struct GcPlan {
 	};
 	std::vector<Level> lv;
 	u32 *newp[2] = {nullptr, nullptr};
-	u32 *stage = nullptr, *list = nullptr, *cnt = nullptr, cap = 0;
+	u32 *stage = nullptr, *list = nullptr, *next = nullptr, *cnt = nullptr, cap = 0;
 	int prepare(Pool &p, const char *prefix);
 };
 
