@@ -1,0 +1,192 @@
+// The host side of plain edits (hd_edit.hip: planning, buffers, the order of passes) on a stand-in for the HIP
+// runtime: nothing runs, launches are reported by name, device memory is addresses only, and what the host
+// reads back is what a test says. Compiled for the host alone; no device is needed.
+//     edit_host_check NAME   runs one test (exit status 0: passed)
+#include "../../vkhashdag_amd/csrc/hd_edit.hip"
+
+#include <cstdarg>
+#include <cstdio>
+#include <functional>
+#include <map>
+#include <set>
+#include <string>
+
+using namespace hd;
+
+struct Fake {
+	u64 free_bytes = 256ull << 30, next = 1ull << 40, allocs = 0;
+	bool same_address = false; // an allocation gets the address that was freed last, whatever its size
+	u64 freed = 0;
+	std::map<u64, u64> held; // address, bytes
+	std::map<const void *, std::string> names;
+	std::function<void(const std::string &, void **)> launch;
+	std::function<bool(void *, const void *, size_t)> read; // device to host: true if it filled the destination
+} fake;
+
+extern "C" {
+hipError_t hipMalloc(void **p, size_t n) {
+	if (n > fake.free_bytes)
+		return hipErrorOutOfMemory;
+	const u64 at = fake.same_address && fake.freed ? fake.freed : fake.next;
+	fake.freed = 0;
+	fake.next += (n + (1u << 21)) & ~((1ull << 21) - 1u);
+	fake.free_bytes -= n;
+	fake.held[at] = n;
+	++fake.allocs;
+	*p = (void *)at;
+	return hipSuccess;
+}
+hipError_t hipFree(void *p) {
+	if (!p)
+		return hipSuccess;
+	const auto it = fake.held.find((u64)p);
+	if (it == fake.held.end())
+		printf("hipFree of %p, which is not held\n", p), exit(1);
+	fake.free_bytes += it->second;
+	fake.freed = it->first;
+	fake.held.erase(it);
+	return hipSuccess;
+}
+hipError_t hipMemGetInfo(size_t *free_b, size_t *total) { return *free_b = fake.free_bytes, *total = 288ull << 30, hipSuccess; }
+hipError_t hipMemcpyAsync(void *dst, const void *src, size_t n, hipMemcpyKind kind, hipStream_t) {
+	if (kind == hipMemcpyDeviceToHost && !(fake.read && fake.read(dst, src, n)))
+		memset(dst, 0, n);
+	return hipSuccess;
+}
+hipError_t hipLaunchKernel(const void *f, dim3, dim3, void **args, size_t, hipStream_t) {
+	if (fake.launch)
+		fake.launch(fake.names[f], args);
+	return hipSuccess;
+}
+void __hipRegisterFunction(void **, const void *f, char *, const char *name, unsigned, void *, void *, dim3 *, dim3 *, int *) {
+	fake.names[f] = name;
+}
+void **__hipRegisterFatBinary(const void *) { return nullptr; }
+void __hipUnregisterFatBinary(void **) {}
+hipError_t __hipPushCallConfiguration(dim3, dim3, size_t, hipStream_t) { return hipSuccess; }
+hipError_t __hipPopCallConfiguration(dim3 *g, dim3 *b, size_t *n, hipStream_t *s) {
+	return *g = *b = dim3(1), *n = 0, *s = nullptr, hipSuccess;
+}
+hipError_t hipMemsetAsync(void *, int, size_t, hipStream_t) { return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned) { return hipSuccess; }
+hipError_t hipEventCreateWithFlags(hipEvent_t *, unsigned) { return hipSuccess; }
+hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
+hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+const char *hipGetErrorString(hipError_t) { return "an error"; }
+hipError_t hipGetLastError() { return hipSuccess; }
+hipError_t hipDeviceGetAttribute(int *, hipDeviceAttribute_t, int) { return hipErrorInvalidValue; }
+hipError_t hipGetDevice(int *d) { return *d = 0, hipSuccess; }
+hipError_t hipGetDevicePropertiesR0600(hipDeviceProp_tR0600 *, int) { return hipErrorInvalidValue; }
+int hipGetStreamDeviceId(hipStream_t) { return 0; }
+hipError_t hipGraphDestroy(hipGraph_t) { return hipSuccess; }
+hipError_t hipGraphExecDestroy(hipGraphExec_t) { return hipSuccess; }
+hipError_t hipGraphInstantiate(hipGraphExec_t *, hipGraph_t, hipGraphNode_t *, char *, size_t) { return hipSuccess; }
+hipError_t hipGraphLaunch(hipGraphExec_t, hipStream_t) { return hipSuccess; }
+hipError_t hipStreamBeginCapture(hipStream_t, hipStreamCaptureMode) { return hipSuccess; }
+hipError_t hipStreamEndCapture(hipStream_t, hipGraph_t *) { return hipSuccess; }
+hipError_t hipHostFree(void *p) { return free(p), hipSuccess; }
+hipError_t hipHostMalloc(void **p, size_t n, unsigned) { return *p = calloc(1, n), hipSuccess; }
+}
+
+namespace hd {
+Tuning g_tuning;
+void set_error(const char *fmt, ...) {
+	va_list ap;
+	va_start(ap, fmt);
+	vprintf(fmt, ap);
+	va_end(ap);
+	printf("\n");
+}
+int set_config(Pool &, const hd_config &) { return HD_ERR_ARG; }
+int make_filled(Pool &) { return HD_OK; }
+int GcPlan::prepare(Pool &, const char *) { return HD_ERR_ARG; }
+int gc_queue(Pool &, const GcPlan &, hipStream_t, u32 *, u32, bool) { return HD_ERR_ARG; }
+int trace_on_stream(Pool &, hipStream_t, u32, u32, const hd_view *, const u32 *, u32, u32, u32 *, const u32 *) {
+	return HD_ERR_ARG;
+}
+} // namespace hd
+
+#define CHECK(x)                                                                                                   \
+	do {                                                                                                           \
+		if (!(x))                                                                                                  \
+			printf("%s:%d: %s does not hold\n", __FILE__, __LINE__, #x), exit(1);                                   \
+	} while (0)
+
+static void make_pool(Pool &p, u32 voxel_level, u32 color_leaf) {
+	p.dc = DevConfig{};
+	p.dc.wbpp = 9, p.dc.pbpb = 2, p.dc.L = voxel_level - 1, p.dc.voxel_level = voxel_level, p.dc.color_leaf = color_leaf;
+	for (u32 l = 0; l < p.dc.L; ++l)
+		p.dc.bucket_bits[l] = 10, p.dc.level_base[l] = l << 10;
+	p.total_buckets = (u64)p.dc.L << 10;
+	p.total_words = p.total_buckets << 11;
+	p.cnode_cap = 1u << 24, p.cleaf_cap = 1u << 28;
+	p.h_pass = (u32 *)calloc(16, 4);
+}
+static hd_edit_desc ball(u32 x, u32 y, u32 z, u32 r, bool colored) {
+	hd_edit_desc d{};
+	d.kind = HD_EDIT_SPHERE_FILL, d.p0[0] = x, d.p0[1] = y, d.p0[2] = z, d.r2 = (u64)r * r;
+	d.colored = colored, d.color.colors = 0x010203u * (x + y + z) & 0xFFFFFFu, d.color.has_value = colored;
+	return d;
+}
+// The pass whose top-down was launched last.
+struct Pass {
+	u32 first = 0, count = 0;
+	bool chained = false;
+};
+static Pass top_down(const std::string &kernel, void **args, const hd_edit_desc *base) {
+	const EditParams &P = *(const EditParams *)args[0];
+	(void)kernel;
+	return Pass{(u32)(P.edits - base), P.n_edits, kernel.find("a_topILj2E") != std::string::npos};
+}
+
+// ---- a piece of a pass that did not hold stays sync-free when the device's memory is gone meanwhile
+static void test_piece() {
+	setenv("HD_EDIT_STAGING_WORDS", "1", 1); // (the buffers held are then much smaller than the plan counts)
+	Pool p;
+	make_pool(p, 12, 8);
+	std::vector<hd_edit_desc> e;
+	for (u32 k = 0; k < 64; ++k)
+		e.push_back(ball(256 + 512 * (k % 8), 256 + 512 * (k / 8), 2048, 160 + k % 3, true));
+	const hd_edit_desc *base = nullptr;
+	Pass now;
+	bool cut = false;
+	std::vector<Pass> seen;
+	fake.launch = [&](const std::string &k, void **args) {
+		CHECK(k.find("k_root") == std::string::npos); // (a kernel of the synchronized pipeline)
+		if (k.find("a_top") == std::string::npos)
+			return;
+		if (!base)
+			base = ((const EditParams *)args[0])->edits;
+		now = top_down(k, args, base);
+		seen.push_back(now);
+	};
+	fake.read = [&](void *dst, const void *, size_t n) {
+		if (dst != p.h_pass || n != 4 * kPmHdr)
+			return false;
+		memset(dst, 0, n);
+		if (!cut) // the first pass is cut at its second edit
+			p.h_pass[kPmCut] = ~1u, fake.free_bytes = 64u << 20;
+		cut = true;
+		return true;
+	};
+	u32 r = 0, c = 0;
+	CHECK(edit_plain(p, 1u, kColorNull, e.data(), (u32)e.size(), &r, &c) == HD_OK);
+	u32 next = 0; // the edits once each, in order, the cut pass aside
+	for (size_t k = 1; k < seen.size(); ++k) {
+		CHECK(seen[k].first == next);
+		next += seen[k].count;
+	}
+	printf("first pass %u edits, %llu MB held\n", seen[0].count, (unsigned long long)(p.scratch.held() >> 20));
+	CHECK(seen[0].count == 64 && next == 64);
+}
+
+int main(int argc, char **argv) {
+	const std::map<std::string, void (*)()> tests{{"piece", test_piece}};
+	if (argc != 2 || !tests.count(argv[1]))
+		return printf("unknown test\n"), 2;
+	setvbuf(stdout, nullptr, _IONBF, 0);
+	tests.at(argv[1])();
+	return printf("%s: passed\n", argv[1]), 0;
+}

@@ -5528,7 +5528,8 @@ static int column_count(Pool &p, const hd_edit_desc &d, std::vector<u64> &S) {
 	return HD_OK;
 }
 
-static void plan_pass(Pool &p, const hd_edit_desc *edits, PassPlan &pp) {
+// held: a part of a planned pass, whose buffers are there (the device's free memory does not matter).
+static void plan_pass(Pool &p, const hd_edit_desc *edits, PassPlan &pp, bool held = false) {
 	const u32 L = p.dc.L, leafL = p.dc.color_leaf, vl = p.dc.voxel_level;
 	pp.stateful = false;
 	bool column = false;
@@ -5606,7 +5607,7 @@ static void plan_pass(Pool &p, const hd_edit_desc *edits, PassPlan &pp) {
 		                           pp.cap[leafL] * (60 + 4 * (u64)kEncTmp)) +
 		     pp.cap[L - 1] * (lds_jobs(p.dc) ? 64 * sizeof(unsigned short) : 64 * sizeof(Color) + 8);
 	pp.bytes = b;
-	if (b > kAsyncBudget || (b > (1ull << 30) && b > async_budget(p)) || (pp.stateful && vl - leafL > 7))
+	if ((!held && (b > kAsyncBudget || (b > (1ull << 30) && b > async_budget(p)))) || (pp.stateful && vl - leafL > 7))
 		pp.async = false;
 }
 
@@ -6115,7 +6116,7 @@ static int edit_sequence(Pool &p, u32 root, u32 croot, const std::vector<hd_edit
 			chain_split(open.first + head, open.count - head, part);
 		}
 		for (auto it = part.rbegin(); it != part.rend(); ++it) {
-			plan_pass(p, flat.data(), *it);
+			plan_pass(p, flat.data(), *it, true);
 			todo.push_back(*it);
 		}
 		open = PassPlan{};
@@ -6154,6 +6155,8 @@ static int edit_sequence(Pool &p, u32 root, u32 croot, const std::vector<hd_edit
 				open = pp;
 			}
 		} else {
+			if (pp.chained) // (edit_pass would take its edits as one group)
+				return set_error("hd_edit: a chained pass without its buffers (internal error)"), HD_ERR_CAPACITY;
 			if (on_device) {
 				u32 rr[2];
 				HD_RET(read_u32s(p, B.roots, rr, 2));
