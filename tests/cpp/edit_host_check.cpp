@@ -182,8 +182,33 @@ static void test_piece() {
 	CHECK(seen[0].count == 64 && next == 64);
 }
 
+// ---- a dedup table that grows is cleared, also where the new one lies at the old one's address
+static void test_table() {
+	Pool p;
+	make_pool(p, 12, 8);
+	fake.same_address = true;
+	std::map<u64, u64> cleared; // address, words
+	fake.launch = [&](const std::string &k, void **args) {
+		if (k.find("a_fill_u32") != std::string::npos && *(u32 *)args[2] == 0u)
+			cleared[*(u64 *)args[0]] = *(u64 *)args[1];
+	};
+	u32 r = 0, c = 0;
+	u64 before = 0;
+	for (u32 n : {1u, 8u, 64u}) {
+		std::vector<hd_edit_desc> e;
+		for (u32 k = 0; k < n; ++k)
+			e.push_back(ball(256 + 512 * (k % 8), 256 + 512 * (k / 8), 2048, 100, true));
+		cleared.clear();
+		CHECK(edit_plain(p, 1u, kColorNull, e.data(), n, &r, &c) == HD_OK);
+		const DevBuf &tab = p.scratch.bufs["a_tab"];
+		CHECK(tab.bytes > before); // (the calls are larger each time)
+		before = tab.bytes;
+		CHECK(cleared.count((u64)tab.p) && cleared[(u64)tab.p] >= tab.bytes / 8 * 2);
+	}
+}
+
 int main(int argc, char **argv) {
-	const std::map<std::string, void (*)()> tests{{"piece", test_piece}};
+	const std::map<std::string, void (*)()> tests{{"piece", test_piece}, {"table", test_table}};
 	if (argc != 2 || !tests.count(argv[1]))
 		return printf("unknown test\n"), 2;
 	setvbuf(stdout, nullptr, _IONBF, 0);

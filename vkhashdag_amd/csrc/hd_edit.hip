@@ -5762,15 +5762,15 @@ static int async_setup(Pool &p, const std::vector<PassPlan> &plans, const std::v
 		T <<= 1;
 	{
 		DevBuf &tb = p.scratch.bufs[pre + "tab"];
-		void *before = tb.p;
-		HD_RET(tb.ensure(T * 8));
+		bool grew = false;
+		HD_RET(p.scratch.get<u32>(pre + "gen", 1, &B.gen_ctr));
+		HD_RET(tb.ensure(T * 8, &grew));
 		B.G.tab = tb.as<u64>();
 		u64 slots = tb.bytes / 8; // ensure() may round up: use every slot it gave
 		while (T * 2 <= slots)
 			T <<= 1;
 		B.tab_slots = slots;
-		HD_RET(p.scratch.get<u32>(pre + "gen", 1, &B.gen_ctr));
-		if (tb.p != before) { // a new table: empty, generations restart
+		if (grew) { // a new table (also one at the old one's address): empty, generations restart
 			a_fill_u32<<<std::min<u64>(div_up(2 * slots, 256), 4096), 256, 0, p.stream>>>((u32 *)tb.p, 2 * slots, 0u);
 			a_fill_u32<<<1, 64, 0, p.stream>>>(B.gen_ctr, 1, 0u);
 			HD_TRY(hipGetLastError());

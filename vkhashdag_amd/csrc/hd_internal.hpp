@@ -37,9 +37,12 @@ inline bool edit_color_ok(const hd_edit_desc &d) { return !d.color.has_value || 
 struct DevBuf {
 	void *p = nullptr;
 	size_t bytes = 0;
-	int ensure(size_t n) {
+	// grew: set where the buffer is a new one (whatever its address) and its content undefined.
+	int ensure(size_t n, bool *grew = nullptr) {
 		if (n <= bytes && p)
 			return HD_OK;
+		if (grew)
+			*grew = true;
 		if (p)
 			HD_TRY(hipFree(p));
 		p = nullptr;
