@@ -19,13 +19,14 @@ struct Fake {
 	u64 freed = 0;
 	std::map<u64, u64> held; // address, bytes
 	std::map<const void *, std::string> names;
+	std::function<bool(size_t)> refuse; // an allocation that fails
 	std::function<void(const std::string &, void **)> launch;
 	std::function<bool(void *, const void *, size_t)> read; // device to host: true if it filled the destination
 } fake;
 
 extern "C" {
 hipError_t hipMalloc(void **p, size_t n) {
-	if (n > fake.free_bytes)
+	if (n > fake.free_bytes || (fake.refuse && fake.refuse(n)))
 		return hipErrorOutOfMemory;
 	const u64 at = fake.same_address && fake.freed ? fake.freed : fake.next;
 	fake.freed = 0;
@@ -207,8 +208,27 @@ static void test_table() {
 	}
 }
 
+// ---- the per-bucket lists start empty also when an allocation after theirs failed
+static void test_lists() {
+	Pool p;
+	make_pool(p, 12, 8);
+	std::set<u64> filled;
+	fake.launch = [&](const std::string &k, void **args) {
+		if (k.find("a_fill_u32") != std::string::npos)
+			filled.insert(*(u64 *)args[0]);
+	};
+	const hd_edit_desc e = ball(256, 256, 2048, 100, true);
+	u32 r = 0, c = 0;
+	fake.refuse = [&](size_t n) { return n >= p.total_buckets * kWalkList * 4; };
+	CHECK(edit_plain(p, 1u, kColorNull, &e, 1, &r, &c) == HD_ERR_DEVICE);
+	CHECK(p.scratch.bufs["a_head"].p && !p.scratch.bufs["a_blist"].p); // (that one was refused)
+	fake.refuse = nullptr;
+	CHECK(edit_plain(p, 1u, kColorNull, &e, 1, &r, &c) == HD_OK);
+	CHECK(filled.count((u64)p.scratch.bufs["a_bcnt"].p) && filled.count((u64)p.scratch.bufs["a_head"].p));
+}
+
 int main(int argc, char **argv) {
-	const std::map<std::string, void (*)()> tests{{"piece", test_piece}, {"table", test_table}};
+	const std::map<std::string, void (*)()> tests{{"piece", test_piece}, {"table", test_table}, {"lists", test_lists}};
 	if (argc != 2 || !tests.count(argv[1]))
 		return printf("unknown test\n"), 2;
 	setvbuf(stdout, nullptr, _IONBF, 0);

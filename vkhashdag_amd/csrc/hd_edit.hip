@@ -5782,17 +5782,18 @@ static int async_setup(Pool &p, const std::vector<PassPlan> &plans, const std::v
 	HD_RET(p.scratch.get<u32>(pre + "gfail", T, &B.G.gfail));
 	HD_RET(p.scratch.get<u32>(pre + "gnext", T, &B.G.gnext));
 	// per-bucket group lists: empty between levels (every walker resets its bucket)
-	const char *kb = "a_bcnt", *kh = "a_head";
-	bool fresh = p.scratch.bufs.find(kb) == p.scratch.bufs.end();
-	HD_RET(p.scratch.get<u32>(kb, p.total_buckets, &B.bcnt));
-	HD_RET(p.scratch.get<u32>(kh, p.total_buckets, &B.head));
+	const u32 bucket_grid = std::min<u64>(div_up(p.total_buckets, 256), 4096);
+	auto bucket_list = [&](const char *name, u32 empty, u32 **out) -> int {
+		bool grew = false;
+		HD_RET(p.scratch.get<u32>(name, p.total_buckets, out, &grew));
+		if (grew)
+			a_fill_u32<<<bucket_grid, 256, 0, p.stream>>>(*out, p.total_buckets, empty);
+		return HD_OK;
+	};
+	HD_RET(bucket_list("a_bcnt", 0u, &B.bcnt));
+	HD_RET(bucket_list("a_head", kNull, &B.head));
 	HD_RET(p.scratch.get<u32>("a_blist", (u64)p.total_buckets * kWalkList, &B.blist));
-	if (fresh) {
-		u32 g = std::min<u64>(div_up(p.total_buckets, 256), 4096);
-		a_fill_u32<<<g, 256, 0, p.stream>>>(B.bcnt, p.total_buckets, 0u);
-		a_fill_u32<<<g, 256, 0, p.stream>>>(B.head, p.total_buckets, kNull);
-		HD_TRY(hipGetLastError());
-	}
+	HD_TRY(hipGetLastError());
 	if (!few)
 		HD_TRY(hipStreamSynchronize(p.stream)); // the host staging array may go out of scope
 	return HD_OK;

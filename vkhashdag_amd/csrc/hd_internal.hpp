@@ -74,9 +74,9 @@ struct LevelBufs {
 struct Scratch {
 	std::map<std::string, DevBuf> bufs;
 	std::map<std::string, LevelBufs> levels;
-	template <typename T> int get(const std::string &name, size_t count, T **out) {
+	template <typename T> int get(const std::string &name, size_t count, T **out, bool *grew = nullptr) {
 		DevBuf &b = bufs[name];
-		HD_RET(b.ensure(count * sizeof(T)));
+		HD_RET(b.ensure(count * sizeof(T), grew));
 		*out = b.as<T>();
 		return HD_OK;
 	}
