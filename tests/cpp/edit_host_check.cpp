@@ -219,7 +219,8 @@ static void test_lists() {
 	};
 	const hd_edit_desc e = ball(256, 256, 2048, 100, true);
 	u32 r = 0, c = 0;
-	fake.refuse = [&](size_t n) { return n >= p.total_buckets * kWalkList * 4; };
+	const size_t list = p.total_buckets * kWalkList * 4;
+	fake.refuse = [&](size_t n) { return n == list + list / 4; };
 	CHECK(edit_plain(p, 1u, kColorNull, &e, 1, &r, &c) == HD_ERR_DEVICE);
 	CHECK(p.scratch.bufs["a_head"].p && !p.scratch.bufs["a_blist"].p); // (that one was refused)
 	fake.refuse = nullptr;
