@@ -228,8 +228,83 @@ static void test_lists() {
 	CHECK(filled.count((u64)p.scratch.bufs["a_bcnt"].p) && filled.count((u64)p.scratch.bufs["a_head"].p));
 }
 
+// ---- calls that fit the device's memory one edit at a time are not refused
+static std::vector<hd_edit_desc> apart(u32 n, u32 r) {
+	std::vector<hd_edit_desc> e;
+	for (u32 k = 0; k < n; ++k)
+		e.push_back(ball(256 + 512 * (k % 8), 256 + 512 * (k / 8), 2048, r, true));
+	return e;
+}
+// The passes of a plain call: in order, each edit once.
+static std::vector<Pass> passes(Pool &p, const std::vector<hd_edit_desc> &e) {
+	std::vector<Pass> seen;
+	const hd_edit_desc *base = nullptr;
+	fake.launch = [&](const std::string &k, void **args) {
+		CHECK(k.find("k_root") == std::string::npos); // (a kernel of the synchronized pipeline)
+		if (k.find("a_top") == std::string::npos)
+			return;
+		if (!base)
+			base = ((const EditParams *)args[0])->edits;
+		seen.push_back(top_down(k, args, base));
+	};
+	u32 r = 0, c = 0, next = 0;
+	CHECK(edit_plain(p, 1u, kColorNull, e.data(), (u32)e.size(), &r, &c) == HD_OK);
+	for (const Pass &q : seen) {
+		CHECK(q.first == next && q.chained == (q.count > 1));
+		next += q.count;
+	}
+	CHECK(next == e.size());
+	return seen;
+}
+static void test_memory() { // little is free: shorter passes, the rest of the memory left to others
+	for (u64 mb : {16384u, 2048u, 768u, 256u, 96u}) {
+		Pool p;
+		make_pool(p, 12, 8);
+		fake.held.clear();
+		fake.free_bytes = mb << 20;
+		const std::vector<Pass> seen = passes(p, apart(64, 160));
+		printf("%llu MB free: %zu passes, %llu MB held\n", (unsigned long long)mb, seen.size(),
+		       (unsigned long long)(p.scratch.held() >> 20));
+		CHECK(mb < 16384u || seen.size() == 1);
+		CHECK(p.scratch.held() < std::max<u64>(mb << 19, 80u << 20)); // (one such edit alone takes 70 MB)
+	}
+}
+static void test_refused() { // the device says no all the same (its memory is in pieces, or somebody was faster)
+	Pool p;
+	make_pool(p, 12, 8);
+	fake.refuse = [&](size_t n) { return n > (30u << 20); };
+	CHECK(passes(p, apart(64, 160)).size() == 64);
+	fake.refuse = nullptr;
+	CHECK(passes(p, apart(64, 160)).size() == 1);
+}
+static void test_column() { // a column fill that cannot have its buffers: the synchronized pipeline
+	Pool p;
+	make_pool(p, 12, 8);
+	p.hm_mn = (u32 *)8;
+	fake.read = [&](void *dst, const void *, size_t n) {
+		if (n != 8 * HD_MAX_LEVELS) // the nodes per level that column_count reads
+			return false;
+		for (u32 l = 0; l < HD_MAX_LEVELS; ++l)
+			((u64 *)dst)[l] = 3ull << 2 * l;
+		return true;
+	};
+	fake.launch = [&](const std::string &k, void **) {
+		if (k.find("k_root") != std::string::npos)
+			printf("column: the synchronized pipeline\n"), exit(0);
+	};
+	hd_edit_desc e{};
+	e.kind = HD_EDIT_COLUMN_FILL, e.p1[0] = e.p1[1] = 4096;
+	u32 r = 0, c = 0;
+	CHECK(edit_plain(p, 1u, kColorNull, &e, 1, &r, &c) == HD_OK); // (all there: sync-free)
+	p.scratch.release();
+	fake.refuse = [&](size_t n) { return n > (100u << 20); };
+	edit_plain(p, 1u, kColorNull, &e, 1, &r, &c);
+	CHECK(!"the fill reached the synchronized pipeline");
+}
+
 int main(int argc, char **argv) {
-	const std::map<std::string, void (*)()> tests{{"piece", test_piece}, {"table", test_table}, {"lists", test_lists}};
+	const std::map<std::string, void (*)()> tests{{"piece", test_piece}, {"table", test_table}, {"lists", test_lists}, {"memory", test_memory},
+	                                                 {"refused", test_refused}, {"column", test_column}};
 	if (argc != 2 || !tests.count(argv[1]))
 		return printf("unknown test\n"), 2;
 	setvbuf(stdout, nullptr, _IONBF, 0);

@@ -5607,7 +5607,14 @@ static void plan_pass(Pool &p, const hd_edit_desc *edits, PassPlan &pp, bool hel
 		                           pp.cap[leafL] * (60 + 4 * (u64)kEncTmp)) +
 		     pp.cap[L - 1] * (lds_jobs(p.dc) ? 64 * sizeof(unsigned short) : 64 * sizeof(Color) + 8);
 	pp.bytes = b;
-	if ((!held && (b > kAsyncBudget || (b > (1ull << 30) && b > async_budget(p)))) || (pp.stateful && vl - leafL > 7))
+	// A chained pass and a column fill have another way to run, in less memory: unless the pool holds that
+	// much already they ask what the device has free, and a chained pass, whose buffers are kept and only save
+	// time, takes a quarter of what one that needs them may.
+	const bool spare = pp.chained || column;
+	if (!held && (b > kAsyncBudget || ((b > (1ull << 30) || (spare && b > p.scratch.held())) &&
+	                                   b > async_budget(p) / (pp.chained ? 4u : 1u))))
+		pp.async = false;
+	if (pp.stateful && vl - leafL > 7)
 		pp.async = false;
 }
 
@@ -6054,9 +6061,39 @@ static bool force_sync_path() {
 	return e && strcmp(e, "sync") == 0;
 }
 
+// async_setup; where the device has not the memory, the buffers given back and the passes the way that needs
+// the least: chained edits one by one, column fills by the synchronized pipeline (async is cleared).
+static int setup_passes(Pool &p, std::vector<PassPlan> &plans, const std::vector<hd_edit_desc> &flat, AsyncBufs &B) {
+	auto spare = [](const PassPlan &pp) { return pp.async && (pp.chained || !pp.column.empty()); };
+	int rc = async_setup(p, plans, flat, B);
+	if (rc != HD_ERR_DEVICE || std::none_of(plans.begin(), plans.end(), spare))
+		return rc;
+	(void)hipGetLastError();
+	HD_TRY(hipStreamSynchronize(p.stream)); // what async_setup queued on them
+	p.scratch.release_passes("a_");
+	B = AsyncBufs{};
+	std::vector<PassPlan> part;
+	for (PassPlan &pp : plans) {
+		if (!spare(pp)) {
+			part.push_back(pp);
+			continue;
+		}
+		for (u32 k = 0; k < pp.count; ++k) {
+			PassPlan one;
+			one.first = pp.first + k, one.count = 1;
+			if (pp.chained)
+				plan_pass(p, flat.data(), one);
+			part.push_back(one);
+		}
+	}
+	plans.swap(part);
+	const bool any = std::any_of(plans.begin(), plans.end(), [](const PassPlan &pp) { return pp.async; });
+	return any ? async_setup(p, plans, flat, B) : HD_OK;
+}
+
 // Applies the passes in order: sync-free passes queue back to back with the roots in device
-// memory; a pass the bounds rule out (column fills, scratch over budget) runs the synchronized
-// pipeline in between.
+// memory; a pass the bounds rule out (scratch over budget) runs the synchronized pipeline in
+// between.
 static int edit_sequence(Pool &p, u32 root, u32 croot, const std::vector<hd_edit_desc> &flat,
                          std::vector<PassPlan> &plans, u32 *root_out, u32 *croot_out) {
 	HD_RET(make_filled(p));
@@ -6081,6 +6118,11 @@ static int edit_sequence(Pool &p, u32 root, u32 croot, const std::vector<hd_edit
 		}
 	}
 	plans.swap(planned);
+	AsyncBufs B;
+	if (any_async) {
+		HD_RET(setup_passes(p, plans, flat, B));
+		any_async = std::any_of(plans.begin(), plans.end(), [](const PassPlan &pp) { return pp.async; });
+	}
 	if (!any_async) {
 		for (auto &pp : plans)
 			HD_RET(edit_pass(p, root, croot, flat.data() + pp.first, pp.count, &root, &croot));
@@ -6088,8 +6130,6 @@ static int edit_sequence(Pool &p, u32 root, u32 croot, const std::vector<hd_edit
 		*croot_out = croot;
 		return HD_OK;
 	}
-	AsyncBufs B;
-	HD_RET(async_setup(p, plans, flat, B));
 	a_set_roots<<<1, 64, 0, p.stream>>>(B.roots, root, croot, B.acc);
 	bool on_device = true;
 	std::vector<PassPlan> todo(plans.rbegin(), plans.rend()); // a stack, first pass on top
@@ -6405,7 +6445,7 @@ static int edit_reserve(Pool &p, const hd_edit_desc *edits, u32 n, u32 mode) {
 	if (!any_async || force_sync_path())
 		return HD_OK;
 	AsyncBufs B;
-	HD_RET(async_setup(p, plans, flat, B));
+	HD_RET(setup_passes(p, plans, flat, B));
 	HD_TRY(hipStreamSynchronize(p.stream));
 	return HD_OK;
 }
@@ -6467,18 +6507,8 @@ struct FrameState {
 		}
 		if (h_roots)
 			(void)hipHostFree(h_roots);
-		if (p) { // the frame's own buffers (its graph holds their addresses)
-			for (auto it = p->scratch.bufs.begin(); it != p->scratch.bufs.end();)
-				if (it->first.compare(0, pre.size(), pre) == 0) {
-					it->second.release();
-					it = p->scratch.bufs.erase(it);
-				} else
-					++it;
-			if (auto it = p->scratch.levels.find(pre); it != p->scratch.levels.end()) {
-				it->second.release();
-				p->scratch.levels.erase(it);
-			}
-		}
+		if (p) // the frame's own buffers (its graph holds their addresses)
+			p->scratch.release_passes(pre);
 	}
 };
 

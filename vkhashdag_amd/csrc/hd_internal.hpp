@@ -90,6 +90,22 @@ struct Scratch {
 					n += x.bytes;
 		return n;
 	}
+	// What a user of sync-free passes holds under its prefix; the per-bucket lists, which all users of the pool
+	// share (a captured graph names them), stay.
+	void release_passes(const std::string &pre) {
+		for (auto it = bufs.lower_bound(pre); it != bufs.end() && it->first.compare(0, pre.size(), pre) == 0;) {
+			if (it->first == "a_bcnt" || it->first == "a_head" || it->first == "a_blist") {
+				++it;
+				continue;
+			}
+			it->second.release();
+			it = bufs.erase(it);
+		}
+		if (auto it = levels.find(pre); it != levels.end()) {
+			it->second.release();
+			levels.erase(it);
+		}
+	}
 	void release() {
 		for (auto &kv : bufs)
 			kv.second.release();
