@@ -180,6 +180,13 @@ int hd_edit(hd_pool *pool, uint32_t root, uint32_t color_root, const hd_edit_des
  * for serving loops that must not stall on device allocation. Blocking. */
 int hd_edit_reserve(hd_pool *pool, const hd_edit_desc *edits, uint32_t n, uint32_t mode);
 
+/* The passes of the last hd_edit: those that edits were applied by; those left after their first part because
+ * edits met in empty space, and those that did not hold at their end (the edits of both went to other passes). */
+typedef struct hd_edit_pass_counts {
+	uint64_t applied, left, cut;
+} hd_edit_pass_counts;
+int hd_edit_passes(hd_pool *pool, hd_edit_pass_counts *out);
+
 /* The passes that a plain hd_edit of these edits is planned as on a pool of this configuration that holds no
  * buffers yet: counts[k] (room for n) consecutive edits each, *n_passes of them; more than one edit: a pass of
  * versions. What the world holds may split such a pass further. Works without a device. */

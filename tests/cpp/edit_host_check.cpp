@@ -302,9 +302,143 @@ static void test_column() { // a column fill that cannot have its buffers: the s
 	CHECK(!"the fill reached the synchronized pipeline");
 }
 
+// ---- passes that do not hold: what a call loses by them
+// The device, as far as the host sees it: fills over a world whose nodes above level `full` are all there and
+// below it none. A chained pass is cut at the first edit that enters a node which was null before the
+// pass and which an earlier edit of it fills (early: its top-down knows), or, with late = k > 0, at its k-th edit
+// whatever it does, or it reports a full bucket.
+struct Device {
+	Pool &p;
+	const std::vector<hd_edit_desc> &e;
+	u32 full, late = 0;
+	bool early = true, full_bucket = false;
+	std::set<u64> nodes;
+	const hd_edit_desc *base = nullptr;
+	Pass now;
+	u32 cut = ~0u; // the pass's first edit that must not share it
+	u32 singles = 0, chained = 0, left = 0, again = 0, next = 0, widest = 0;
+	bool open = false;
+
+	template <typename F> void entered(const hd_edit_desc &d, F f) const { // nodes of level full .. the color leaves
+		const i64 r = (i64)std::sqrt((double)d.r2) + 1;
+		for (u32 l = full; l <= p.dc.color_leaf; ++l) {
+			const i64 S = (i64)1 << (p.dc.voxel_level - l);
+			for (i64 z = (d.p0[2] - r) / S; z <= (d.p0[2] + r) / S; ++z)
+				for (i64 y = (d.p0[1] - r) / S; y <= (d.p0[1] + r) / S; ++y)
+					for (i64 x = (d.p0[0] - r) / S; x <= (d.p0[0] + r) / S; ++x)
+						if (reaches(d, {x * S, y * S, z * S}, S))
+							f((u64)l << 48 | (u64)z << 32 | (u64)y << 16 | (u64)x);
+		}
+	}
+	void settle() { // the pass before went through
+		if (!open)
+			return;
+		open = false;
+		CHECK(now.first == next);
+		for (u32 k = now.first; k < now.first + now.count; ++k)
+			entered(e[k], [&](u64 n) { nodes.insert(n); });
+		next += now.count;
+		(now.count > 1 ? chained : singles) += 1;
+		widest = std::max(widest, now.count);
+	}
+	void run() {
+		fake.launch = [this](const std::string &k, void **args) {
+			CHECK(k.find("k_root") == std::string::npos);
+			if (k.find("a_chain_restore") != std::string::npos) {
+				CHECK(cut != ~0u || full_bucket);
+				++again;
+				open = false;
+			}
+			if (k.find("a_top") == std::string::npos)
+				return;
+			if (!base)
+				base = ((const EditParams *)args[0])->edits;
+			const Pass q = top_down(k, args, base);
+			if (open && (cut == ~0u || now.count == 1) && !(full_bucket && now.count > 1))
+				settle(); // (else the host has still to learn that the pass before did not hold)
+			else if (open)
+				return;
+			now = q;
+			open = true;
+			cut = ~0u;
+			std::set<u64> mine;
+			for (u32 j = 0; j < q.count && cut == ~0u; ++j) {
+				const hd_edit_desc &d = e[q.first + j];
+				bool meets = false;
+				entered(d, [&](u64 n) { meets |= !nodes.count(n) && mine.count(n); });
+				if (q.chained && (meets || (late && j == late)))
+					cut = j;
+				entered(d, [&](u64 n) { mine.insert(n); });
+			}
+		};
+		fake.read = [this](void *dst, const void *, size_t n) {
+			memset(dst, 0, n);
+			if (dst == p.h_pass + kHostMeet && n == 4) {
+				if (cut != ~0u && early)
+					*(u32 *)dst = ~cut, ++left, open = false;
+			} else if (dst == p.h_pass && n == 4 * kPmHdr) {
+				p.h_pass[kPmCut] = full_bucket ? ~0u : cut == ~0u ? 0u : ~cut;
+				p.h_pass[kPmFull] = full_bucket;
+			}
+			return true;
+		};
+		u32 r = 0, c = 0;
+		CHECK(edit_plain(p, 1u, kColorNull, e.data(), (u32)e.size(), &r, &c) == HD_OK);
+		settle();
+		CHECK(next == e.size());
+		CHECK(p.passes - p.passes_cut == singles + chained && p.passes_left == left && p.passes_cut == again);
+	}
+	// in passes of one edit: a chained pass takes up to three, its top-down one and a quarter
+	double time() const { return singles + 3.0 * chained + 1.25 * left + 3.0 * again; }
+};
+static double air(const char *name, const std::vector<hd_edit_desc> &e, u32 full, bool wary, u32 late = 0,
+                  bool early = true, bool full_bucket = false) {
+	Pool p;
+	make_pool(p, 12, 8);
+	p.edit_wary = wary;
+	fake.free_bytes = 256ull << 30;
+	fake.held.clear();
+	Device d{p, e, full};
+	d.late = late, d.early = early, d.full_bucket = full_bucket;
+	d.run();
+	printf("%s%s: %zu edits, %u single, %u chained (up to %u), %u left, %u cut: %.2f of one by one\n", name,
+	       wary ? ", wary" : "", e.size(), d.singles, d.chained, d.widest, d.left, d.again, d.time() / (double)e.size());
+	return d.time();
+}
+static std::vector<hd_edit_desc> lattice(u32 nx, u32 ny, u32 nz, u32 step, u32 r) {
+	std::vector<hd_edit_desc> e;
+	for (u32 k = 0; k < nx * ny * nz; ++k)
+		e.push_back(ball(100 + step * (k % nx), 100 + step * (k / nx % ny), 3200 + step * (k / nx / ny), r, true));
+	return e;
+}
+// At most a sixteenth slower than one by one, and a pass and a half that did not hold (of a wary pool: its
+// top-down).
+static double bound(u32 n, bool wary) { return n * (1.0 + 1.0 / 16.0) + (wary ? 1.25 : 4.5); }
+static void test_air() {
+	for (bool wary : {false, true}) {
+		for (u32 n : {2u, 3u, 4u, 8u, 16u, 120u})
+			CHECK(air("row", lattice(n, 1, 1, 32, 6), 2, wary) <= bound(n, wary));
+		CHECK(air("sheet", lattice(16, 16, 1, 48, 10), 2, wary) <= bound(256, wary));
+		CHECK(air("lattice", lattice(8, 8, 8, 48, 10), 2, wary) <= bound(512, wary));
+	}
+}
+static void test_ground() { // nothing is null above the color leaves: nearly everything shares passes
+	for (bool wary : {false, true}) {
+		CHECK(air("ground", lattice(16, 16, 1, 48, 10), 9, wary) <= 6.0);
+		CHECK(air("ground", lattice(3, 1, 1, 48, 10), 9, wary) <= 3.0);
+	}
+}
+static void test_cut() { // passes that are found out at their end only
+	for (u32 late : {1u, 2u, 5u, 40u})
+		CHECK(air("cut", lattice(16, 16, 2, 48, 10), 9, false, late) <= bound(512, false));
+	CHECK(air("meets seen at the end", lattice(16, 16, 1, 48, 10), 2, false, 0, false) <= bound(256, false));
+	CHECK(air("full buckets", lattice(16, 16, 2, 48, 10), 9, false, 0, true, true) <= bound(512, false));
+}
+
 int main(int argc, char **argv) {
 	const std::map<std::string, void (*)()> tests{{"piece", test_piece}, {"table", test_table}, {"lists", test_lists}, {"memory", test_memory},
-	                                                 {"refused", test_refused}, {"column", test_column}};
+	                                                 {"refused", test_refused}, {"column", test_column},
+	                                                 {"air", test_air}, {"ground", test_ground}, {"cut", test_cut}};
 	if (argc != 2 || !tests.count(argv[1]))
 		return printf("unknown test\n"), 2;
 	setvbuf(stdout, nullptr, _IONBF, 0);

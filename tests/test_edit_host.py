@@ -24,7 +24,7 @@ def check(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("name", ["piece", "table", "lists", "memory", "refused", "column"])
+@pytest.mark.parametrize("name", ["piece", "table", "lists", "memory", "refused", "column", "air", "ground", "cut"])
 def test_edit_host(check, name):
     r = subprocess.run([check, name], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stdout + r.stderr

@@ -116,6 +116,7 @@ def lib():
             "hd_pool_clear_overflow": (C.c_int, [VP]),
             "hd_edit": (C.c_int, [VP, U32, U32, VP, U32, U32, P32, P32]),
             "hd_edit_reserve": (C.c_int, [VP, VP, U32, U32]),
+            "hd_edit_passes": (C.c_int, [VP, VP]),
             "hd_edit_plan": (C.c_int, [VP, VP, U32, VP, C.POINTER(U32)]),
             "hd_gc": (C.c_int, [VP, VP, U32]),
             "hd_edit_host": (C.c_int, [VP, U32, C.POINTER(hd_host_editor), P32]),
@@ -304,6 +305,12 @@ class DevicePool:
 
     Edit = edit
     ThreadedEdit = edit
+
+    def edit_passes(self):
+        """hd_edit_passes: (applied, left, cut) passes of the last edit call."""
+        out = (U64 * 3)()
+        check(lib().hd_edit_passes(self.h, out))
+        return tuple(out)
 
     def reserve(self, edits, mode=MODE_PLAIN):
         """hd_edit_reserve: allocate what edit(edits, mode) would, without editing."""

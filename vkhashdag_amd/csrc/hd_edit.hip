@@ -852,7 +852,7 @@ template <u32 kT = kAT> __device__ inline Pair block_excl_scan2(Pair x, Pair *sh
 // per-pass device counters: pm[kPmHdr + l] entries of level l, pm[kPmHdr + L + l] list words
 // (chained passes: kPmCut the first edit that must not share the pass, as ~index, 0 if none; kPmFull
 // whether a bucket or the color pool was full; kPmRoot, kPmCroot, kPmNodes the roots and the color node count
-// that the pass leaves)
+// that the pass leaves; kPmMeet the first edit that meets an earlier one in empty space, as ~index, 0 if none)
 enum PassMeta : u32 {
 	kPmOverflow = 0,
 	kPmEvents = 1,
@@ -864,7 +864,8 @@ enum PassMeta : u32 {
 	kPmRoot = 7,
 	kPmCroot = 8,
 	kPmNodes = 9,
-	kPmHdr = 10
+	kPmMeet = 10,
+	kPmHdr = 11
 };
 // counters accumulated over the passes of one hd_edit call
 enum AccMeta : u32 { kAccEntries = 0, kAccUpserts = 1, kAccJobs = 2, kAccOverflow = 3, kAccCount = 4 };
@@ -1531,12 +1532,25 @@ __device__ inline void chain_versions(const ALevel *__restrict__ lv, u32 l, cons
 	}
 }
 __device__ inline void chain_cut(u32 *__restrict__ pm, u32 edit) { atomicMax(&pm[kPmCut], ~edit); }
-// prev of entry e.
-__device__ inline void chain_link(const ALevel *__restrict__ lv, u32 l, const Entry &E, u32 e) {
+// prev of entry e. A colored edit that enters a node which was null before the pass and which an earlier edit
+// of the pass may fill will be cut there by the joins: kPmMeet tells the host so after the top-down.
+__device__ inline bool chain_fills(const EditParams &P, u32 k) {
+	const DevEditor ed = P.editor(k);
+	return !ed.is_dig() && !ed.is_paint();
+}
+__device__ inline void chain_link(const EditParams &P, const ALevel *__restrict__ lv, u32 l, const Entry &E, u32 e,
+                                  u32 *__restrict__ pm) {
 	u32 p = kNull;
-	chain_versions(lv, l, E, [&](u32, u32 q) {
-		p = q < lv[l].cap ? q : kNull; // (past it only when a level outgrew its bound, which is reported)
-		return false;
+	bool latest = true;
+	const bool empty = E.ptr == kNull && (E.sf & kSfActive);
+	chain_versions(lv, l, E, [&](u32 k, u32 q) {
+		if (latest)
+			p = q < lv[l].cap ? q : kNull; // (past it only when a level outgrew its bound, which is reported)
+		latest = false;
+		const bool meet = empty && chain_fills(P, k);
+		if (meet)
+			atomicMax(&pm[kPmMeet], ~E.loff);
+		return empty && !meet;
 	});
 	stg(lv[l].prev, e, p);
 }
@@ -1550,6 +1564,12 @@ __device__ inline void chain_roots(const EditParams &P, const ALevel &A0, const 
 		const Entry E{0, 0, 0, root, kNull, c.sf & ~kSfNewJob, c.octree, kNull, k, 1u};
 		if (c.t != kProceed)
 			chain_cut(pm, k);
+		if (root == kNull && (c.sf & kSfActive))
+			for (u32 j = 0; j < k; ++j)
+				if (chain_fills(P, j)) {
+					atomicMax(&pm[kPmMeet], ~k);
+					break;
+				}
 		stg(A0.ent, k, E);
 		stg(A0.prev, k, k ? k - 1u : kNull);
 	}
@@ -1725,7 +1745,7 @@ __global__ void __launch_bounds__(kTopThreads<kMode>) a_top(EditParams P0, const
 				o = expand_pair_e(P, l, A, t, E, ev, pm, ev_cap, bits, by_wave ? &hits : nullptr,
 				                  by_wave ? &hits2 : nullptr);
 				if (kChain && (t & 7u) == 0 && l)
-					chain_link(lv, l, E, (u32)(t >> 3));
+					chain_link(P, lv, l, E, (u32)(t >> 3), pm);
 			}
 			sflag[threadIdx.x] = o.flag;
 			Pair tile;
@@ -1799,7 +1819,7 @@ __global__ void __launch_bounds__(kAT) a_count(EditParams P, u32 l, const ALevel
 		PairOut o = expand_pair_e(P, l, A, t, A.ent[(u32)(t >> 3)], ev, pm, ev_cap, nullptr, by_wave ? &hits : nullptr,
 		                          by_wave ? &hits2 : nullptr);
 		if (kChain && (t & 7u) == 0)
-			chain_link(lv, l, A.ent[(u32)(t >> 3)], (u32)(t >> 3));
+			chain_link(P, lv, l, A.ent[(u32)(t >> 3)], (u32)(t >> 3), pm);
 		flag[t] = o.flag;
 		lcnt[t] = o.lcnt;
 		cstate[t] = o.cs;
@@ -5432,6 +5452,8 @@ struct PassPlan {
 	bool stateful = false, async = false;
 	bool folded = false; // the edits may overlap (folded lists)
 	bool chained = false; // the edits one after another in one pass (versions of shared nodes)
+	bool apart = false;   // of a chained pass: no two of its edits meet in empty space (a top-down has shown it)
+	bool part = false;    // of a planned pass: planned when its turn comes, in the buffers of the whole
 	std::vector<u64> cap, list_cap;
 	std::vector<u64> column; // a column fill's proceeding nodes per level, once counted
 	u64 ev_cap = 0, bytes = 0;
@@ -6043,10 +6065,20 @@ static int queue_pass(Pool &p, const PassPlan &pp, AsyncBufs &B, bool reserve = 
 // takes about as long as two single ones).
 constexpr u32 kChainMin = 3;
 constexpr u64 kChainBudget = 4ull << 30; // pass buffers a chained pass may take
-static void chain_split(u32 first, u32 count, std::vector<PassPlan> &plans) {
+// What a call's chained passes have gained over passes of one edit, less what those lost that did not hold, in
+// sixteenths of a pass of one edit (75 us in air, 108 us on a 4096^3 terrain's surface; chained passes take
+// 150 to 250 us, one left after its top-down about 90). Below zero the next edits run one by one, a
+// sixteenth each: whatever the edits do to one another, a call takes about a sixteenth and one or two lost
+// passes longer than one by one; the longer nothing holds, the rarer the tries (leave). From a pass that did not hold until one does (Pool::edit_wary, from call to
+// call) colored passes are asked after their top-down whether edits meet in empty space, the common reason;
+// else nobody waits for the answer (the wait takes about 45 us of a call).
+// (256 fills in a 16 x 16 sheet in the air took 69 ms with every run tried at full length.)
+constexpr int kCreditEdit = 16, kCreditPass = 3 * kCreditEdit, kCreditLeft = kCreditEdit * 5 / 4, kCreditMost = 8 * kCreditEdit;
+constexpr u32 kChainHead = 5; // edits of a pass's first part that are worth a pass again
+static void chain_split(u32 first, u32 count, std::vector<PassPlan> &plans, bool part = false, u32 least = kChainMin) {
 	PassPlan pp;
-	pp.first = first, pp.count = count;
-	if (count >= kChainMin) {
+	pp.first = first, pp.count = count, pp.part = part;
+	if (count >= least) {
 		pp.chained = true;
 		plans.push_back(pp);
 		return;
@@ -6124,6 +6156,7 @@ static int edit_sequence(Pool &p, u32 root, u32 croot, const std::vector<hd_edit
 		any_async = std::any_of(plans.begin(), plans.end(), [](const PassPlan &pp) { return pp.async; });
 	}
 	if (!any_async) {
+		p.passes = plans.size();
 		for (auto &pp : plans)
 			HD_RET(edit_pass(p, root, croot, flat.data() + pp.first, pp.count, &root, &croot));
 		*root_out = root;
@@ -6136,6 +6169,7 @@ static int edit_sequence(Pool &p, u32 root, u32 croot, const std::vector<hd_edit
 	// A chained pass whose counters are on their way: whether it held is asked when the next pass's
 	// top-down is queued, so the host's work on the rest of that pass overlaps it.
 	PassPlan open;
+	int credit = 0, gain = 0, leave = kCreditLeft; // gain: the open pass's, taken for good already
 	hipError_t err = hipSuccess;
 	auto held = [&]() {
 		if (!open.count)
@@ -6143,23 +6177,27 @@ static int edit_sequence(Pool &p, u32 root, u32 croot, const std::vector<hd_edit
 		err = hipEventSynchronize(p.ev_pass);
 		return err == hipSuccess && !p.h_pass[kPmCut];
 	};
-	// It did not: the edits before the cut run again in one pass, then the others; or all one by one.
+	// The edits of pp up to head and the others, or all one by one (head 0), instead of it.
+	auto split = [&](const PassPlan &pp, u32 head) {
+		std::vector<PassPlan> part;
+		chain_split(pp.first, head, part, true, kChainHead);
+		if (!part.empty())
+			part[0].apart = true;
+		if (head)
+			chain_split(pp.first + head, pp.count - head, part, true);
+		else
+			for (u32 k = 0; k < pp.count; ++k)
+				chain_split(pp.first + k, 1, part, true);
+		todo.insert(todo.end(), part.rbegin(), part.rend());
+	};
+	// A pass that did not hold: the edits before the cut run again in one pass, then the others; or all one by one.
 	auto redo = [&]() {
 		a_chain_restore<<<grid_for(p.total_buckets, kAT, 1024), kAT, 0, p.stream>>>(p.bucket_words, B.saved,
 		                                                                           p.total_buckets);
-		std::vector<PassPlan> part;
-		if (p.h_pass[kPmFull])
-			for (u32 k = 0; k < open.count; ++k)
-				chain_split(open.first + k, 1, part);
-		else {
-			const u32 head = std::max(~p.h_pass[kPmCut], 1u);
-			chain_split(open.first, head, part);
-			chain_split(open.first + head, open.count - head, part);
-		}
-		for (auto it = part.rbegin(); it != part.rend(); ++it) {
-			plan_pass(p, flat.data(), *it, true);
-			todo.push_back(*it);
-		}
+		split(open, p.h_pass[kPmFull] ? 0u : std::max(~p.h_pass[kPmCut], 1u));
+		credit -= gain + kCreditPass;
+		p.edit_wary = true;
+		++p.passes_cut;
 		open = PassPlan{};
 	};
 	while (!todo.empty() || open.count) {
@@ -6175,14 +6213,41 @@ static int edit_sequence(Pool &p, u32 root, u32 croot, const std::vector<hd_edit
 			if (todo.empty())
 				break;
 		}
-		const PassPlan pp = todo.back();
+		PassPlan pp = todo.back();
 		todo.pop_back();
+		if (pp.chained && !pp.apart && credit < 0) {
+			const u32 alone = std::min(pp.count, (u32)-credit);
+			PassPlan rest = pp;
+			rest.count = alone;
+			if (alone < pp.count) {
+				std::vector<PassPlan> part;
+				chain_split(pp.first + alone, pp.count - alone, part, true);
+				todo.insert(todo.end(), part.rbegin(), part.rend());
+			}
+			split(rest, 0);
+			credit += (int)alone;
+			continue;
+		}
+		if (pp.part)
+			plan_pass(p, flat.data(), pp, true);
+		pp.part = false;
 		if (pp.async) {
 			if (!on_device)
 				a_set_roots_keep<<<1, 64, 0, p.stream>>>(B.roots, root, croot);
 			on_device = true;
+			const bool ask = pp.chained && pp.stateful && !pp.apart && p.edit_wary;
 			bool ok = true;
-			HD_RET(queue_pass(p, pp, B, true, [&]() { return ok = held(); }));
+			u32 meet = 0;
+			HD_RET(queue_pass(p, pp, B, true, [&]() {
+				ok = held();
+				if (!ok || !ask)
+					return ok;
+				err = hipMemcpyAsync(p.h_pass + kHostMeet, B.pm + kPmMeet, 4, hipMemcpyDeviceToHost, p.stream);
+				if (err == hipSuccess)
+					err = hipStreamSynchronize(p.stream);
+				meet = p.h_pass[kHostMeet];
+				return err == hipSuccess && !meet;
+			}));
 			HD_TRY(err);
 			if (!ok) { // only this pass's top-down has been queued
 				todo.push_back(pp);
@@ -6190,7 +6255,21 @@ static int edit_sequence(Pool &p, u32 root, u32 croot, const std::vector<hd_edit
 				continue;
 			}
 			open = PassPlan{};
+			if (ask)
+				p.edit_wary = meet != 0u;
+			if (meet) { // likewise
+				split(pp, ~meet);
+				credit -= leave;
+				leave = ~meet < kChainHead ? std::min(2 * leave, kCreditMost) : kCreditLeft;
+				++p.passes_left;
+				continue;
+			}
+			++p.passes;
 			if (pp.chained) {
+				leave = kCreditLeft;
+				const int most = std::max(credit, kCreditMost);
+				gain = std::min(credit + kCreditEdit * (int)pp.count - kCreditPass, most) - credit;
+				credit += gain;
 				HD_TRY(hipMemcpyAsync(p.h_pass, B.pm, 4 * kPmHdr, hipMemcpyDeviceToHost, p.stream));
 				HD_TRY(hipEventRecord(p.ev_pass, p.stream));
 				open = pp;
@@ -6204,6 +6283,7 @@ static int edit_sequence(Pool &p, u32 root, u32 croot, const std::vector<hd_edit
 				root = rr[0], croot = rr[1];
 			}
 			on_device = false;
+			++p.passes;
 			HD_RET(edit_pass(p, root, croot, flat.data() + pp.first, pp.count, &root, &croot));
 		}
 	}
@@ -6704,6 +6784,7 @@ extern "C" int hd_edit(hd_pool *h, uint32_t root, uint32_t color_root, const hd_
 	Pool &p = h->p;
 	auto t0 = std::chrono::steady_clock::now();
 	p.last_entries = p.last_upserts = p.last_jobs = 0;
+	p.passes = p.passes_left = p.passes_cut = 0;
 	u32 r = root, c = color_root;
 	for (u32 i = 0; i < n; ++i) {
 		if (edits[i].kind > HD_EDIT_COLUMN_FILL)
@@ -6737,6 +6818,13 @@ extern "C" int hd_edit_reserve(hd_pool *h, const hd_edit_desc *edits, uint32_t n
 			return set_error("edit %u: bits_per_weight %u > 3", i, edits[i].color.bits_per_weight), HD_ERR_ARG;
 	}
 	return edit_reserve(h->p, edits, n, mode);
+}
+
+extern "C" int hd_edit_passes(hd_pool *h, hd_edit_pass_counts *out) {
+	if (!h || !out)
+		return set_error("hd_edit_passes: null argument"), HD_ERR_ARG;
+	*out = hd_edit_pass_counts{h->p.passes - h->p.passes_cut, h->p.passes_left, h->p.passes_cut};
+	return HD_OK;
 }
 
 extern "C" int hd_edit_plan(const hd_config *cfg, const hd_edit_desc *edits, uint32_t n, uint32_t *counts,

@@ -128,6 +128,7 @@ enum Meta : u32 {
 // bounds test, wherever in the pool it starts.
 constexpr u64 kWordsPad = 16;
 
+constexpr u32 kHostMeet = 15; // the word of h_pass for kPmMeet
 constexpr u64 kHostRays = HD_TRAVERSAL_HOST_RAYS;
 
 struct Pool;
@@ -172,6 +173,10 @@ struct Pool {
 	u64 last_entries = 0, last_upserts = 0, last_jobs = 0;
 	u32 last_groups = 0;
 	double last_ms = 0;
+	// the last chained pass that was waited for did not hold: a hint for the next calls' passes, whose results
+	// do not depend on it
+	bool edit_wary = false;
+	u64 passes = 0, passes_left = 0, passes_cut = 0; // hd_edit_pass_counts; passes: the cut ones too
 	u32 edit_gen = 0; // generation of the sync-free pass's group table (hd_edit.hip)
 	u32 *h_pass = nullptr; // pinned: a chained pass's counters, read back after its top-down
 	// pinned: hd_traversal_host's rays and hits (kHostRays of them), which the kernel reads and writes in
