@@ -175,3 +175,38 @@ def test_gc_of_overfull_buckets_keeps_what_fits_in_pointer_order(bits, wbpp, pbp
     assert np.array_equal(dev.bucket_words(), want[0])
     assert np.array_equal(dev.live_words()[1], live_words(want[1], want[0], cfg))
     assert dev.stats().overflow & 4
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("seed", range(6))
+def test_gc_of_a_filled_chain_without_its_root(seed):
+    """A pool that came in with a full root bucket has no filled node of level 0, so nothing holds the chain below
+    it: the collection drops those nodes and finds the chain again, as at the start of editing."""
+    from vkhashdag_amd import capi
+    print(f"seed {seed}", flush=True)
+    cfg = W.PoolConfig(5, 0, [0, 1, 3], 0)
+    rng = np.random.default_rng(seed)
+    words, bw = np.zeros(cfg.total_words, np.uint32), np.zeros(cfg.total_buckets, np.uint32)
+    leaves = [(3 + b) * 32 for b in range(8)]
+    for p in leaves:
+        words[p: p + 2] = rng.integers(1, 1 << 32, 2)
+        bw[p // 32] = 2
+    for i in range(16):  # 8 nodes in each bucket of level 1, a root above each
+        p = 32 + 32 * (i // 8) + 2 * (i % 8)
+        words[p: p + 2] = 1 << (i % 8), leaves[int(rng.integers(8))]
+        words[2 * i: 2 * i + 2] = 1 << (i % 8), p
+    bw[0], bw[1: 3] = 32, 16
+    roots = [2 * i for i in rng.permutation(16)]
+    dev, ora = capi.DevicePool(cfg), O.OraclePool(cfg)
+    dev.write_live_words(bw, live_words(words, bw, cfg))
+    dev.edit(W.edit(W.SPHERE_DIG, (1, 1, 1), r2=1))
+    assert dev.filled()[0] == O.HD_NULL and O.HD_NULL not in dev.filled()[1:]
+    ora.load_state(dev.state())
+    for k in range(2):
+        roots_d, roots_o = dev.gc(extra_roots=roots), ora.gc(extra_roots=roots)
+        assert list(roots_d) == list(roots_o)
+        assert np.array_equal(dev.filled(), ora.filled())
+        bd, wd = dev.live_words()
+        bo, wo = ora.live_words()
+        assert np.array_equal(bd, bo) and np.array_equal(wd, wo)
+        roots = [int(r) for r in roots_o[1:]]

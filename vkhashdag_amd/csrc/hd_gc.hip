@@ -114,14 +114,17 @@ __device__ inline void for_live(const u32 *__restrict__ bits, const u32 *__restr
 
 // ---- forward
 // the roots mark level 0, and the filled chain every level (its nodes have the most parents of all: with
-// their bits set first no parent's atomic queues on them)
+// their bits set first no parent's atomic queues on them), as far down as it hangs together: what is below a
+// missing node nobody holds
 __global__ void k_gc_mark_roots(const u32 *__restrict__ roots, u32 n, const u32 *__restrict__ filled, DevConfig c,
                                 GcLevels G) {
 	const u32 i = blockIdx.x * blockDim.x + threadIdx.x;
 	const u32 l = i < n ? 0u : i - n;
 	if (l >= c.L || (i >= n && !filled))
 		return;
-	const u32 r = i < n ? roots[i] : filled[l];
+	u32 r = i < n ? roots[i] : filled[l];
+	for (u32 k = 0; i >= n && k < l; ++k)
+		r = filled[k] == kNull ? kNull : r;
 	const u64 base = (u64)c.level_base[l] << c.wbpb(), words = 1ull << (c.bucket_bits[l] + c.wbpb());
 	if (r == kNull || (u64)r < base || (u64)r - base >= words)
 		return;
@@ -209,8 +212,9 @@ __global__ void __launch_bounds__(kGcThreads) k_gc_key(const u32 *__restrict__ w
                                                        u64 base, u64 cbase, u64 cwords, const u32 *__restrict__ cnewp,
                                                        u32 *__restrict__ stage, GcLists B, u32 *__restrict__ filled) {
 	if ((threadIdx.x | blockIdx.x) == 0 && filled) {
-		const u64 o = (u64)filled[level + 1u] - cbase;
-		if (o < cwords)
+		const u32 f = filled[level + 1u];
+		const u64 o = (u64)f - cbase; // (of a node that was dropped: launch_refill finds the chain again)
+		if (f != kNull && o < cwords)
 			filled[level + 1u] = cnewp[o >> 1];
 	}
 	for_live(bits, bucket_words, c, level, [&](u32 o) {
@@ -485,8 +489,8 @@ int GcPlan::prepare(Pool &p, const char *prefix) {
 	HD_RET(p.scratch.get<u32>(pre + "gc_newp0", max_words / 2 + 1, &newp[0]));
 	HD_RET(p.scratch.get<u32>(pre + "gc_newp1", max_words / 2 + 1, &newp[1]));
 	HD_RET(p.scratch.get<u32>(pre + "gc_stage", max_words + 16, &stage));
-	HD_RET(p.scratch.get<u32>(pre + "gc_list", max_buckets * cap, &list));
-	HD_RET(p.scratch.get<u32>(pre + "gc_next", max_words / 2 + 1, &next));
+	HD_RET(p.scratch.get<u32>(pre + "gc_list", max_buckets * cap + max_words / 2 + 1, &list));
+	next = list + max_buckets * cap;
 	HD_RET(p.scratch.get<u32>(pre + "gc_cnt", 2 * max_buckets, &cnt)); // and the chains' heads
 	return HD_OK;
 }
