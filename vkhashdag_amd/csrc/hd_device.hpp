@@ -323,8 +323,8 @@ struct DevEditor {
 		return m & ((z < hm->h(x, y) ? 1u : 0u) | (z < hm->h(x + 1u, y) ? 2u : 0u) | (z < hm->h(x, y + 1u) ? 4u : 0u) |
 		            (z < hm->h(x + 1u, y + 1u) ? 8u : 0u));
 	}
-	// edit_voxel / edit_voxel_vbr_asg of those four, v their occupancy: the new one; asg |= the voxels
-	// the edit assigns its color.
+	// edit_voxel / edit_voxel_vbr of those four, v their occupancy: the new one; asg: the voxels that a
+	// colored edit assigns its color (the others keep theirs).
 	__device__ u32 edit_voxel4(u32 x, u32 y, u32 z, u32 v, u32 &asg) const {
 		if (!stateful()) {
 			if (is_paint())
@@ -379,23 +379,6 @@ struct DevEditor {
 		if (is_paint() && !has_ptr)
 			t = kNotAffected;
 		return t;
-	}
-	// edit_voxel_vbr without the voxel's current color: asg is set when the edit assigns c (the color
-	// stays the current one otherwise).
-	__device__ bool edit_voxel_vbr_asg(u32 x, u32 y, u32 z, bool voxel, Color &c, bool &asg) const {
-		bool in = in_range(x, y, z);
-		if (d.kind == HD_EDIT_COLUMN_FILL) {
-			if (in || !voxel) {
-				c = Color::rgb8(column_rgb8(x, y, z));
-				asg = true;
-			}
-			return voxel || in;
-		}
-		if (in || !voxel) {
-			c = color();
-			asg = true;
-		}
-		return is_paint() ? voxel : (voxel || in);
 	}
 	__device__ bool edit_voxel_vbr(u32 x, u32 y, u32 z, bool voxel, Color &c) const {
 		bool in = in_range(x, y, z);

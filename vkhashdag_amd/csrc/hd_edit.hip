@@ -880,7 +880,7 @@ struct ALevel {
 	u32 *status, *pend, *res, *slot, *lpos, *bucket;
 	u32 *content, *csize;
 	u32 *ores, *ccnt, *cbase, *own; // color results, SetNode passes
-	uint4 *pev; // 8 per entry (levels color leaf .. L - 2, color leaves rebuilt in LDS): a pushed
+	uint4 *pev; // 8 per entry (levels color leaf .. L - 2, small jobs): a pushed
 	            // child's {voxel offset in its job, colors, wb, 0}, valid where pmask bit 16 + slot is set
 	u32 *prev; // chained passes: the entry of the latest earlier edit at the same node, or kNull
 	u32 cap, list_cap;
@@ -2113,7 +2113,7 @@ __device__ inline uint2 child_result_fresh(const ALevel &C, const GroupTable &G,
 // (10M leaves of 4096 mixed edits 5.5 -> 2.3 ms and their colors 3.5 -> 1.8 ms; a 2048^2 terrain 250 -> 81 us.)
 // A leaf inside a color job records what its edits assign: on the dense path the colors (lcol, by
 // voxel) and which voxels they are (lmask), which a_leafcolor moves into the job's dense colors (so
-// this kernel does not wait for them to be decoded); with LDS jobs the assigning edit per voxel.
+// this kernel does not wait for them to be decoded); with small jobs the assigning edit per voxel.
 __device__ inline bool leaf_writes_colors(const EditParams &P, const ALevel *__restrict__ lv, const Entry &E) {
 	return (E.sf & kSfWriter) && !(E.sf & kSfFinal) && (E.sf & kSfActive) && E.job < lv[P.c.color_leaf].cap;
 }
@@ -2124,7 +2124,7 @@ __device__ inline bool leaf_writes_colors(const EditParams &P, const ALevel *__r
 // voxel, which of the pass's edits assigned its color last (lidx, kNoEdit for none: 2 bytes instead
 // of the color and a mask bit); the color job reads the color from that edit.
 enum : u32 { kLeafAll = 0, kLeafNodes = 1, kLeafColors = 2 };
-constexpr u32 kNoEdit = 0xFFFFu; // a pass with LDS color jobs holds fewer edits
+constexpr u32 kNoEdit = 0xFFFFu; // a pass with small color jobs holds fewer edits
 template <u32 kMode>
 __global__ void __launch_bounds__(kAT) a_leaf(EditParams P, const ALevel *__restrict__ lv, const u32 *__restrict__ pm,
                                               Color *__restrict__ lcol, u64 *__restrict__ lmask,
@@ -3588,11 +3588,11 @@ template <class Out, class Or> __device__ inline void job_write(const JobSeg &R,
 		run.bits += bpw;
 	}
 }
-// Staging words per job of a sync-free pass with LDS jobs (on average: each workgroup fills its
+// Staging words per job of a sync-free pass with small jobs (on average: each workgroup fills its
 // share of the area in turn); a chunk that no longer fits goes to a_job_rest like one larger than
 // kJobHdr.
 constexpr u32 kEtmpJobWords = 512;
-// One workgroup per writer job rebuilds the job's colors in LDS (job_rebuild) and encodes them as
+// One workgroup per writer job rebuilds the job's colors in registers (job_rebuild) and encodes them as
 // a_encode_size does (SetLeaf's size decision). A chunk of at most kJobHdr words is staged in the
 // workgroup's share of etmp (etmp_cap words); a larger one, or one that no longer fits, is listed for
 // a_job_rest, which rebuilds and encodes it in place once the append offsets are known.
@@ -3660,7 +3660,7 @@ __global__ void __launch_bounds__(kEncThreads, 6) a_job_encode(EditParams P, con
 		}
 	}
 }
-// The jobs a_job_encode listed (their chunk was not staged): rebuilt in LDS again (the same inputs
+// The jobs a_job_encode listed (their chunk was not staged): rebuilt again (the same inputs
 // give the same colors and size) and encoded straight into the color leaves at the offset the
 // append scan gave, or over the old chunk when it fits in place (the rebuild has read it whole
 // before the first store). One workgroup per job.
@@ -3781,8 +3781,7 @@ __global__ void a_scan_fix(u32 leafL, u32 *__restrict__ pm, u32 *__restrict__ ap
 // the wavefront copies the chunks one after another. (A workgroup per chunk, which holds about 130 words, waited
 // for four dependent loads each time: 868k of them 4.1 -> 0.25 ms in a world after 20 batches of 4096 edits.)
 __global__ void __launch_bounds__(kEncThreads) a_encode_write(EditParams P, const ALevel *__restrict__ lv,
-                                                               const u32 *__restrict__ pm, const Color *__restrict__ dense,
-                                                               u32 V, const u32 *__restrict__ info,
+                                                               const u32 *__restrict__ pm, const u32 *__restrict__ info,
                                                                const u32 *__restrict__ appo, u64 leaf_cap,
                                                                const u32 *__restrict__ etmp) {
 	const u32 leafL = P.c.color_leaf, lane = threadIdx.x & 63u;
@@ -5459,9 +5458,9 @@ struct PassPlan {
 	u64 ev_cap = 0, bytes = 0;
 };
 
-// Color leaves of at most kJobV voxels (and no deeper than the node leaves) are rebuilt in LDS by
-// a_job_encode: pushes go to per-pair records instead of the event list.
-static bool lds_jobs(const DevConfig &c) {
+// Small color jobs: color leaves of at most kJobV voxels (and no deeper than the node leaves) are rebuilt by
+// a_job_encode, without dense colors in memory: pushes go to per-pair records instead of the event list.
+static bool small_jobs(const DevConfig &c) {
 	return c.color_leaf + 1u <= c.L && 3u * (c.voxel_level - c.color_leaf) <= 12u;
 }
 
@@ -5609,7 +5608,7 @@ static void plan_pass(Pool &p, const hd_edit_desc *edits, PassPlan &pp, bool hel
 	u64 pev_bytes = 0;
 	if (pp.stateful)
 		for (u32 l = leafL; l + 1 < L; ++l)
-			(lds_jobs(p.dc) ? pev_bytes : pp.ev_cap) += 8 * pp.cap[l];
+			(small_jobs(p.dc) ? pev_bytes : pp.ev_cap) += 8 * pp.cap[l];
 	pp.ev_cap = std::min<u64>(pp.ev_cap, lim);
 	pev_bytes *= sizeof(uint4);
 	// bytes: entries + per-level arrays, expand temporaries, lists, events, dense colors
@@ -5623,11 +5622,11 @@ static void plan_pass(Pool &p, const hd_edit_desc *edits, PassPlan &pp, bool hel
 		}
 	}
 	b += maxpairs * 24 + pp.ev_cap * sizeof(PushEvent) + pev_bytes;
-	if (pp.stateful) // per job: dense colors and a staging slot, or (LDS jobs) bump-allocated staging
-		b += (lds_jobs(p.dc) ? pp.cap[leafL] * (60 + 4 * (u64)kEtmpJobWords)
+	if (pp.stateful) // per job: dense colors and a staging slot, or (small jobs) bump-allocated staging
+		b += (small_jobs(p.dc) ? pp.cap[leafL] * (60 + 4 * (u64)kEtmpJobWords)
 		                     : pp.cap[leafL] * ((u64)sizeof(Color) << (3 * (vl - leafL))) +
 		                           pp.cap[leafL] * (60 + 4 * (u64)kEncTmp)) +
-		     pp.cap[L - 1] * (lds_jobs(p.dc) ? 64 * sizeof(unsigned short) : 64 * sizeof(Color) + 8);
+		     pp.cap[L - 1] * (small_jobs(p.dc) ? 64 * sizeof(unsigned short) : 64 * sizeof(Color) + 8);
 	pp.bytes = b;
 	// A chained pass and a column fill have another way to run, in less memory: unless the pool holds that
 	// much already they ask what the device has free, and a chained pass, whose buffers are kept and only save
@@ -5655,13 +5654,13 @@ struct AsyncBufs {
 	u32 *tsum = nullptr;  // per-tile totals of the jobs' append scan
 	u32 *saved = nullptr; // chained passes: the bucket counters before the pass, its flag and append count
 	uint4 *cstate = nullptr, *jrange = nullptr;
-	u32 etmp_cap = 0; // staging words of LDS jobs (bump-allocated)
+	u32 etmp_cap = 0; // staging words of small jobs (bump-allocated)
 	Pair *bsum = nullptr;
 	PushEvent *ev = nullptr;
 	Color *dense = nullptr, *lcol = nullptr;
 	u64 *lmask = nullptr;
-	unsigned short *lidx = nullptr; // LDS jobs: per leaf voxel, the pass edit that assigned its color
-	uint2 *ecol = nullptr;          // LDS jobs: per pass edit, the color lidx stands for
+	unsigned short *lidx = nullptr; // small jobs: per leaf voxel, the pass edit that assigned its color
+	uint2 *ecol = nullptr;          // small jobs: per pass edit, the color lidx stands for
 	hd_edit_desc *edits = nullptr;
 	GroupTable G{};
 	u64 tab_slots = 0;
@@ -5727,7 +5726,7 @@ static int async_setup(Pool &p, const std::vector<PassPlan> &plans, const std::v
 		HD_RET(get(l, kLvContent, c * (l + 1 < L ? 9 : 2), &A.content));
 		if (l + 1 < L)
 			HD_RET(get(l, kLvCsize, c, &A.csize));
-		if (stateful && lds_jobs(p.dc) && l >= leafL && l + 1 < L)
+		if (stateful && small_jobs(p.dc) && l >= leafL && l + 1 < L)
 			HD_RET(get(l, kLvPev, 8 * c, &A.pev));
 		if (stateful && l <= leafL) {
 			HD_RET(get(l, kLvOres, c, &A.ores));
@@ -5749,7 +5748,7 @@ static int async_setup(Pool &p, const std::vector<PassPlan> &plans, const std::v
 	HD_RET(p.scratch.get<PushEvent>(pre + "events", std::max<u64>(ev, 1), &B.ev));
 	if (stateful) {
 		const u64 jobs = std::max<u64>(cap[leafL], 1);
-		const bool lj = lds_jobs(p.dc); // LDS jobs rebuild what they do not stage: no dense colors
+		const bool lj = small_jobs(p.dc); // small jobs rebuild what they do not stage: no dense colors
 		HD_RET(p.scratch.get<Color>(pre + "dense", lj ? 1 : jobs << (3 * (p.dc.voxel_level - leafL)), &B.dense));
 		HD_RET(p.scratch.get<u32>(pre + "info", 4 * jobs, &B.info));
 		HD_RET(p.scratch.get<u32>(pre + "app", jobs, &B.app));
@@ -5911,7 +5910,7 @@ static void queue_chain_nodes(const Pool &p, const PassPlan &pp, const EditParam
 static int queue_pass(Pool &p, const PassPlan &pp, AsyncBufs &B, bool reserve = true,
                       const std::function<bool()> &held = nullptr) {
 	const u32 L = p.dc.L, leafL = p.dc.color_leaf;
-	if (pp.stateful && lds_jobs(p.dc) && pp.count >= kNoEdit) // leaves record edits by 16-bit index
+	if (pp.stateful && small_jobs(p.dc) && pp.count >= kNoEdit) // leaves record edits by 16-bit index
 		return set_error("hd_edit: a colored pass holds at most %u edits", kNoEdit - 1u), HD_ERR_ARG;
 	const EditParams P = pass_params(p, B.edits + pp.first, pp.count, pp.stateful, pp.folded);
 	const u32 V = pp.stateful ? 1u << (3u * P.leaf_bits) : 0u;
@@ -5948,7 +5947,7 @@ static int queue_pass(Pool &p, const PassPlan &pp, AsyncBufs &B, bool reserve = 
 	// proceeding node, cleared children): SetNode alone, once the top-down has classified them.
 	if (pp.stateful && !colors && leafL > 0 && !pp.chained)
 		queue_setnode(p, pp, P, B, p.stream);
-	const bool ljobs = lds_jobs(p.dc);
+	const bool ljobs = small_jobs(p.dc);
 	if (colors && !ljobs) { // the jobs' dense colors on the color stream, beside the leaves
 		HD_TRY(hipEventRecord(p.ev_top, p.stream));
 		HD_TRY(hipStreamWaitEvent(p.cstream, p.ev_top, 0));
@@ -5959,7 +5958,7 @@ static int queue_pass(Pool &p, const PassPlan &pp, AsyncBufs &B, bool reserve = 
 			                                                           B.lv[leafL].cap, B.dense);
 	}
 	const u32 leaf_grid = grid_for(pp.cap[L - 1], kAT / kLeafLanes, 16384);
-	// with LDS jobs, the leaves' colors start the color stream right after the top-down (always: such
+	// with small jobs, the leaves' colors start the color stream right after the top-down (always: such
 	// a pass has the edit-index buffer lidx, and no lcol / lmask for kLeafAll)
 	const bool split = colors && ljobs;
 	if (split) {
@@ -5979,7 +5978,7 @@ static int queue_pass(Pool &p, const PassPlan &pp, AsyncBufs &B, bool reserve = 
 		++l_from;
 	auto write_colors = [&](hipStream_t s) { // the encoded chunks to their places
 		const u32 G = grid_for(pp.cap[leafL], 1, 8192);
-		a_encode_write<<<grid_for(pp.cap[leafL], kEncThreads / 64, 2048), kEncThreads, 0, s>>>(P, B.d_lv, B.pm, B.dense, V, B.info, B.appo, p.cleaf_cap, B.etmp);
+		a_encode_write<<<grid_for(pp.cap[leafL], kEncThreads / 64, 2048), kEncThreads, 0, s>>>(P, B.d_lv, B.pm, B.info, B.appo, p.cleaf_cap, B.etmp);
 		if (ljobs) {
 			a_job_rest<<<std::min(G, 1024u), kEncThreads, 0, s>>>(P, B.d_lv, B.pm, B.jrange, B.lidx, B.ecol, V, B.info, B.appo,
 			                                               p.cleaf_cap, B.rest);
@@ -6326,7 +6325,7 @@ static void batched_plans(const Pool &p, const hd_edit_desc *edits, u32 n, std::
 static bool chains(const Pool &p, const hd_edit_desc &d) {
 	if (d.kind == HD_EDIT_COLUMN_FILL || p.dc.L < 2)
 		return false;
-	return !is_stateful(d) || (d.color.has_value && !d.color.bits_per_weight && lds_jobs(p.dc) && p.dc.color_leaf > 0);
+	return !is_stateful(d) || (d.color.has_value && !d.color.bits_per_weight && small_jobs(p.dc) && p.dc.color_leaf > 0);
 }
 // Whether an edit reaches the node of size S at lo: sphere_node / aabb_node do not rule it out.
 static bool reaches(const hd_edit_desc &d, const i64 (&lo)[3], i64 S) {
@@ -6467,10 +6466,10 @@ static void folded_plans(const hd_edit_desc *edits, u32 n, std::vector<hd_edit_d
 
 // The passes of a batched call: folded runs, each split in halves until its buffers fit the
 // sync-free budget; dependency groups when a colored pass would rebuild its color leaves from
-// dense per-voxel colors (nested pushes need the leaves rebuilt in LDS).
+// dense per-voxel colors (nested pushes need small jobs).
 static void batch_plans(Pool &p, const hd_edit_desc *edits, u32 n, std::vector<hd_edit_desc> &flat,
                         std::vector<PassPlan> &plans) {
-	if (!lds_jobs(p.dc) || force_sync_path()) {
+	if (!small_jobs(p.dc) || force_sync_path()) {
 		batched_plans(p, edits, n, flat, plans);
 		return;
 	}
@@ -6652,7 +6651,7 @@ static int frame_create(Pool &p, const hd_frame_config &cfg, u32 root, u32 croot
 			pp.list_cap[l] = cfg.max_edits > 1 ? std::min(2 * S, lim) : 0;
 		}
 		pp.ev_cap = 0;
-		if (colors && !lds_jobs(p.dc))
+		if (colors && !small_jobs(p.dc))
 			for (u32 l = p.dc.color_leaf; l + 1 < L; ++l)
 				pp.ev_cap += 8 * pp.cap[l];
 		pp.ev_cap = std::min<u64>(pp.ev_cap, lim);
