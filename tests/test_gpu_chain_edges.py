@@ -92,3 +92,64 @@ def test_color_leaves_in_place_or_kept(history):
         assert dev.edit_passes()[0] < len(e)
         words.append(dev.stats().color_leaf_words)
     assert not history or words == sorted(set(words))  # nothing in place: it grows with every call
+
+
+def assert_same_devices(a, b, where):
+    from vkhashdag_amd import capi
+    assert (a.root, a.color_root) == (b.root, b.color_root), where
+    assert a.stats().overflow == b.stats().overflow, where
+    assert all(np.array_equal(x, y) for x, y in zip(a.live_words(), b.live_words())), where
+    # (the counts go on past the capacity, and what did not fit leaves its words unwritten: the colors are compared)
+    counts = [(p.stats().color_nodes, p.stats().color_leaf_words) for p in (a, b)]
+    assert counts[0] == counts[1], where
+    nodes, words = min(counts[0][0], a.cfg.color_node_capacity), min(counts[0][1], a.cfg.color_leaf_capacity)
+    vox = np.random.default_rng(1).integers(0, 1 << a.cfg.voxel_level, (20000, 3)).astype(np.uint32)
+    vox[:, 2] = 90 + vox[:, 2] % 32
+    got = []
+    for p in (a, b):
+        cn, cl = np.zeros(max(nodes, 1) * 8, np.uint32), np.zeros(max(words, 1), np.uint32)
+        capi.check(capi.lib().hd_pool_read_color_nodes(p.h, 0, nodes, cn.ctypes.data))
+        capi.check(capi.lib().hd_pool_read_color_leaves(p.h, 0, words, cl.ctypes.data))
+        got.append(O.color_fetch(cn, cl, p.color_root, p.cfg.voxel_level, p.cfg.color_leaf_level, vox))
+    assert np.array_equal(*got), where
+
+
+# the calls below take 184 to 259 color nodes and 9800 color leaf words
+@pytest.mark.parametrize("nodes,words", [(1 << 16, 5000), (220, 1 << 20), (1 << 16, 1 << 20)])
+def test_color_pool_runs_out(nodes, words):
+    """Edits of one call where the color nodes or leaves end: as the same edits one call each."""
+    from vkhashdag_amd import capi
+    res = 256
+    print(f"{nodes} color nodes, {words} color leaf words", flush=True)
+    cfg = small_cfg(res, 9, 9, 2, 4, color_node_capacity=nodes, color_leaf_capacity=words)
+    a, b = capi.DevicePool(cfg), capi.DevicePool(cfg)
+    e = W.edits([W.edit(W.AABB_FILL, (0, 0, 0), (res, res, 100), color=0x305070)])
+    for k in range(5):
+        a.edit(e)
+        for i in range(len(e)):
+            b.edit(e[i:i + 1])
+        assert_same_devices(a, b, f"call {k}")
+        e = spheres([(16 + 48 * i + k, 16 + 48 * j, 100 + 3 * k) for i in range(5) for j in range(5)], 6, True)
+    assert (a.stats().overflow == 0) == (nodes == words >> 4)
+
+
+def test_color_words_of_more_than_rgb8():
+    """Words with bits above the 24 of RGB8, and weights of no bits: as the same edits one call each."""
+    from vkhashdag_amd import capi
+    res = 256
+    print("color words of 32 bits", flush=True)
+    cfg = small_cfg(res, 9, 9, 2, 4)
+    a, b = capi.DevicePool(cfg), capi.DevicePool(cfg)
+    rng = np.random.default_rng(3)
+    palette = np.array([0x305070, 0xFF305070, 0x12345678, 0x00305071], np.uint32)
+    e = W.edits([W.edit(W.AABB_FILL, (0, 0, 0), (res, res, 100), color=0x111111)])
+    for k in range(5):
+        a.edit(e)
+        assert k != 1 or a.edit_passes()[0] < len(e)
+        for i in range(len(e)):
+            b.edit(e[i:i + 1])
+        assert_same_devices(a, b, f"call {k}")
+        e = spheres([(24 + 48 * i, 24 + 48 * j, 100) for i in range(5) for j in range(5)], 7 + k % 2, True)
+        e["colors"] = palette[rng.integers(0, 4, len(e))]
+        e["weight"] = rng.integers(0, 2, len(e))
+        e["kind"] = rng.choice([W.SPHERE_FILL, W.SPHERE_PAINT], len(e))
