@@ -1,6 +1,6 @@
 """Device GC with many nodes in a bucket: more than a wavefront sorts at once (bit-exact against the oracle),
 and more than a bucket holds. There the oracle and the reference stop; the device keeps, in old pointer order,
-what fits, writes null for the others and reports it, as the model below does."""
+what fits, takes the others out of their parents and reports it, as the model below does."""
 import numpy as np
 import pytest
 
@@ -62,8 +62,15 @@ def gc_model(words, bw, cfg, roots, filled):
             if l == L - 1:
                 b, node = p // wpb - base[l], old[p: p + 2]
             else:
-                k = bin(int(old[p]) & 255).count("1")
-                node = np.array([old[p]] + [maps[l + 1].get(int(c), O.HD_NULL) for c in old[p + 1: p + 1 + k]], np.uint32)
+                bits = [i for i in range(8) if int(old[p]) >> i & 1]
+                kids = [maps[l + 1].get(int(c), O.HD_NULL) for c in old[p + 1: p + 1 + len(bits)]]
+                left = [(i, c) for i, c in zip(bits, kids) if c != O.HD_NULL]
+                if not left:
+                    maps[l][p] = O.HD_NULL
+                    dropped += 1
+                    continue
+                k = len(left)
+                node = np.array([(int(old[p]) & ~255) | sum(1 << i for i, _ in left)] + [c for _, c in left], np.uint32)
                 b = O.olib().hdo_hash_span(node, k + 1) & ((1 << cfg.bucket_bits[l]) - 1)
             n, a = len(node), at[b]
             if a % wpp + n > wpp:
@@ -175,6 +182,48 @@ def test_gc_of_overfull_buckets_keeps_what_fits_in_pointer_order(bits, wbpp, pbp
     assert np.array_equal(dev.bucket_words(), want[0])
     assert np.array_equal(dev.live_words()[1], live_words(want[1], want[0], cfg))
     assert dev.stats().overflow & 4
+
+
+def null_children(words, cfg, root):
+    """Null pointers under set mask bits below root."""
+    level, n = {root} - {O.HD_NULL}, 0
+    for l in range(cfg.node_levels - 1):
+        kids = [int(c) for p in level for c in words[p + 1: p + 1 + bin(int(words[p]) & 255).count("1")]]
+        n += kids.count(O.HD_NULL)
+        level = set(kids) - {O.HD_NULL}
+    return n
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("bits,wbpp,seed", [(3, 6, 3), (5, 6, 8), (4, 6, 2)])
+def test_worlds_that_lost_nodes_can_be_traced(bits, wbpp, seed):
+    """A terrain that overfills its pool, collected: rays go through what is left of it as the oracle's do through
+    the same words."""
+    from vkhashdag_amd import capi
+    res = 256
+    print(f"{1 << bits} buckets of {4 << wbpp} words", flush=True)
+    h = W.value_noise_heightmap(res, 3, seed, res // 8, res * 3 // 4)
+    cfg = config(res, bits, wbpp, 2)
+    dev = capi.DevicePool(cfg, heights=h)
+    dev.edit(W.terrain_edit(res, seed=seed, skin=4, colored=False))
+    words, filled = dev.full_words(), dev.filled()
+    want = gc_model(words, dev.bucket_words(), cfg, [dev.root], filled)
+    assert want[4] > 0 and O.HD_NULL not in want[3]
+    assert null_children(words, cfg, dev.root) == 0
+    for k in range(2):
+        dev.gc()
+        words = dev.full_words()
+        if k == 0:
+            assert dev.root == want[2][0]
+            assert np.array_equal(dev.bucket_words(), want[0])
+            assert np.array_equal(dev.live_words()[1], live_words(want[1], want[0], cfg))
+        assert null_children(words, cfg, dev.root) == 0
+        rng = np.random.default_rng(seed)
+        o = rng.random((5000, 3), np.float32) * 3 - 1
+        d = rng.random((5000, 3), np.float32) - o
+        hits = dev.traversal(o, d)
+        rec = O.march_rays(words, cfg.node_levels, dev.root, o, d)
+        assert np.array_equal(hits[:, 3] != 0, rec[:, 3] >> 31 != 0) and hits[:, 3].sum() > 100
 
 
 @pytest.mark.gpu

@@ -210,7 +210,8 @@ struct GcLists {
 __global__ void __launch_bounds__(kGcThreads) k_gc_key(const u32 *__restrict__ words, const u32 *__restrict__ bits,
                                                        const u32 *__restrict__ bucket_words, DevConfig c, u32 level,
                                                        u64 base, u64 cbase, u64 cwords, const u32 *__restrict__ cnewp,
-                                                       u32 *__restrict__ stage, GcLists B, u32 *__restrict__ filled) {
+                                                       u32 *__restrict__ stage, GcLists B, u32 *__restrict__ newp,
+                                                       u32 *__restrict__ filled) {
 	if ((threadIdx.x | blockIdx.x) == 0 && filled) {
 		const u32 f = filled[level + 1u];
 		const u64 o = (u64)f - cbase; // (of a node that was dropped: launch_refill finds the chain again)
@@ -222,12 +223,34 @@ __global__ void __launch_bounds__(kGcThreads) k_gc_key(const u32 *__restrict__ w
 #pragma unroll
 		for (u32 k = 0; k < 9; ++k)
 			buf[k] = words[base + o + k];
-		const u32 k = (u32)__builtin_popcount(buf[0] & 0xFFu);
+		u32 k = (u32)__builtin_popcount(buf[0] & 0xFFu), lost = 0;
 		u32 np[8];
 #pragma unroll
 		for (u32 j = 0; j < 8; ++j) {
 			const u64 co = (u64)buf[j + 1] - cbase;
 			np[j] = j < k && co < cwords ? cnewp[co >> 1] : kNull;
+			lost |= (j < k && np[j] == kNull ? 1u : 0u) << j;
+		}
+		if (lost) { // children that a full bucket dropped leave the node (a trace would follow a null pointer)
+			u32 mask = buf[0] & 0xFFu, r = 0;
+			for (u32 m = mask; m; m &= m - 1u, ++r)
+				if ((lost >> r) & 1u)
+					mask &= ~(m & (0u - m));
+#pragma unroll 1
+			for (u32 p = 0; p < 7; ++p) // the others move up, in order
+#pragma unroll
+				for (u32 j = 0; j < 7; ++j) {
+					const bool up = np[j] == kNull;
+					const u32 x = np[j];
+					np[j] = up ? np[j + 1] : x;
+					np[j + 1] = up ? x : np[j + 1];
+				}
+			buf[0] = (buf[0] & ~0xFFu) | mask;
+			k = (u32)__builtin_popcount(mask);
+			if (k == 0u) {
+				newp[o >> 1] = kNull;
+				return;
+			}
 		}
 #pragma unroll
 		for (u32 j = 0; j < 8; ++j)
@@ -522,7 +545,7 @@ int gc_queue(Pool &p, const GcPlan &G, hipStream_t s, u32 *d_roots, u32 n_roots,
 		const GcPlan::Level &V = G.lv[l], &C = G.lv[l + 1];
 		u32 *newp = G.newp[l & 1];
 		k_gc_key<<<waves((u32)l), kGcThreads, 0, s>>>(p.words, V.bits, p.bucket_words, p.dc, (u32)l, V.base, C.base,
-		                                              C.words, G.newp[(l + 1) & 1], G.stage, lists,
+		                                              C.words, G.newp[(l + 1) & 1], G.stage, lists, newp,
 		                                              has_filled ? p.d_filled : nullptr);
 		k_gc_pack_inner<<<grid((V.buckets + kPackBuckets - 1) / kPackBuckets * 64), kGcThreads, 0, s>>>(
 		    p.words, p.bucket_words, p.dc, (u32)l, G.stage, lists, newp, p.meta);
