@@ -6068,10 +6068,11 @@ constexpr u64 kChainBudget = 4ull << 30; // pass buffers a chained pass may take
 // sixteenths of a pass of one edit (75 us in air, 108 us on a 4096^3 terrain's surface; chained passes take
 // 150 to 250 us, one left after its top-down about 90). Below zero the next edits run one by one, a
 // sixteenth each: whatever the edits do to one another, a call takes about a sixteenth and one or two lost
-// passes longer than one by one; the longer nothing holds, the rarer the tries (leave). From a pass that did not hold until one does (Pool::edit_wary, from call to
-// call) colored passes are asked after their top-down whether edits meet in empty space, the common reason;
-// else nobody waits for the answer (the wait takes about 45 us of a call).
-// (256 fills in a 16 x 16 sheet in the air took 69 ms with every run tried at full length.)
+// passes longer than one by one; the longer nothing holds, the rarer the tries (leave). From a pass that did
+// not hold until one does (Pool::edit_wary, from call to call) colored passes are asked after their top-down
+// whether edits meet in empty space, the common reason; else nobody waits for the answer (the wait takes
+// about 45 us of a call). 256 fills in a 16 x 16 sheet in the air: 21.9 ms, 69 with every run tried at full
+// length, 21.1 one by one.
 constexpr int kCreditEdit = 16, kCreditPass = 3 * kCreditEdit, kCreditLeft = kCreditEdit * 5 / 4, kCreditMost = 8 * kCreditEdit;
 constexpr u32 kChainHead = 5; // edits of a pass's first part that are worth a pass again
 static void chain_split(u32 first, u32 count, std::vector<PassPlan> &plans, bool part = false, u32 least = kChainMin) {
